@@ -281,14 +281,19 @@ struct lai_basis {
   DevBuf<int> dshloc;       // sh_loc on the device
   DevBuf<long long> ddmoff; // mol_dmoff on the device
   DevBuf<int> ddmns;        // shells per molecule on the device
+  DevBuf<int> dmpair, dmshell, dmfunc;  // first pair, shell and function of each molecule
+  DevBuf<int> dfsh;         // per function: its shell within the molecule
   // Schwarz: packed per molecule, mol_pair[m] + j*(j+1)/2 + i (molecule-local shells)
   std::vector<double> Q;
   bool have_Q = false;
-  DevBuf<double> dQ;  // per pair, pair order
+  DevBuf<double> dQ;  // per pair, list order
   // worklist
   ClassList cls[kNumClasses];
   DevBuf<JkSegs> segs;
-  DevBuf<int> kets;
+  DevBuf<int> kets;           // pair at each list position
+  DevBuf<PairRec> lpairs;     // the pair records in list order
+  DevBuf<long long> jloc;     // per pair: its block in the Coulomb accumulators
+  long long jl0[kNumPairClasses] = {};  // block of list position p of class x at jl0[x] + p * functions
   DevBuf<double> sdmax;  // per molecule: ns_m x ns_m shell-pair max|D|
   bool have_worklist = false;
   int wl_dscreen = 0, wl_mixed = 0;
@@ -300,8 +305,10 @@ struct lai_basis {
   double flops64 = 0, flops32 = 0;
   int64_t n_eri = 0, n_fp32 = 0;
   uint64_t checksum = 0;
-  // J/K scratch (unsymmetrised)
-  DevBuf<double> Jt, Kt;
+  // J/K scratch, cleared by every build: the unsymmetrised Kt (mat_size
+  // doubles), then the Coulomb blocks of the pairs in list order (jl_size)
+  DevBuf<double> acc;
+  long long jl_size = 0;
   // per-class launch choice
   ClassTune tune[kNumClasses];
   // queue of the persistent launch (LAI_JK_PERSISTENT), built from the
@@ -602,6 +609,7 @@ extern "C" int lai_dev_upload_batch(lai_ctx* ctx, int n_mol, const int* mol_shel
       r.bsum = 0.0;
       for (int k = r.pp_off; k < r.pp_off + r.npp; ++k) r.bsum += pbound[k];
       b->pairs_h[p] = r;
+      b->jl_size += ncart(L[sa]) * ncart(L[sb]);
       b->pair_cls[p] = pair_class(L[sa], L[sb]);
       b->pi[p] = i;
       b->pj[p] = j;
@@ -617,6 +625,9 @@ extern "C" int lai_dev_upload_batch(lai_ctx* ctx, int n_mol, const int* mol_shel
   std::vector<float> pbf(pbound.begin(), pbound.end());
   std::vector<int> dmns(n_mol);
   for (int m = 0; m < n_mol; ++m) dmns[m] = b->mol_shell[m + 1] - b->mol_shell[m];
+  std::vector<int> mfunc(1, 0), fsh;
+  for (int m = 0; m < n_mol; ++m) mfunc.push_back(mfunc.back() + b->mol_nbf[m]);
+  for (int s = 0; s < ns; ++s) fsh.insert(fsh.end(), size_t(ncart(L[s])), b->sh_loc[s]);
   std::vector<double> pih(pph.size());
   for (size_t k = 0; k < pph.size(); ++k) pih[k] = 0.5 / pph[k].zeta;
   hipError_t e;
@@ -637,8 +648,11 @@ extern "C" int lai_dev_upload_batch(lai_ctx* ctx, int n_mol, const int* mol_shel
       (e = b->dshloc.assign(b->sh_loc.data(), b->sh_loc.size())) != hipSuccess ||
       (e = b->ddmoff.assign(b->mol_dmoff.data(), b->mol_dmoff.size())) != hipSuccess ||
       (e = b->ddmns.assign(dmns.data(), dmns.size())) != hipSuccess ||
-      (e = b->Jt.alloc(size_t(b->mat_size))) != hipSuccess ||
-      (e = b->Kt.alloc(size_t(b->mat_size))) != hipSuccess) {
+      (e = b->dmpair.assign(b->mol_pair.data(), b->mol_pair.size())) != hipSuccess ||
+      (e = b->dmshell.assign(b->mol_shell.data(), b->mol_shell.size())) != hipSuccess ||
+      (e = b->dmfunc.assign(mfunc.data(), mfunc.size())) != hipSuccess ||
+      (e = b->dfsh.assign(fsh.data(), fsh.size())) != hipSuccess ||
+      (e = b->acc.alloc(size_t(b->mat_size + b->jl_size))) != hipSuccess) {
     lai_dev_basis_free(b);
     return fail(LAI_ERR_MEMORY, std::string("lai_dev_upload_basis: ") + hipGetErrorString(e));
   }
@@ -668,14 +682,19 @@ extern "C" int lai_dev_basis_free(lai_basis* b) {
   b->dcenter.release();
   b->dexps.release();
   b->dcoefs.release();
-  b->Jt.release();
-  b->Kt.release();
+  b->acc.release();
   for (auto& c : b->cls) {
     c.chunks.release();
     c.gchunks.release();
   }
   b->segs.release();
   b->kets.release();
+  b->lpairs.release();
+  b->jloc.release();
+  b->dmpair.release();
+  b->dmshell.release();
+  b->dmfunc.release();
+  b->dfsh.release();
   b->sdmax.release();
   b->dQ.release();
   b->dmoff.release();
@@ -1058,33 +1077,43 @@ extern "C" int lai_dev_build_worklist(lai_basis* b, double thr, const double* sh
   const int nm = b->n_mol;
   constexpr int NPC = kNumPairClasses, NB = kMaxSegs;
 
-  // Ket lists: per (molecule, pair class, primitive-count bucket), the pairs in
+  // Ket lists: per (pair class, molecule, primitive-count bucket), the pairs in
   // order of decreasing Schwarz bound.  Bucket k holds npp_sig in [2^k, 2^(k+1))
   // (the last one everything above), so the lanes of a wavefront run similar
-  // primitive-loop trip counts.
+  // primitive-loop trip counts.  A pair's position in the lists one after
+  // another is its name in the worklist (chunks, pair records, Schwarz bounds,
+  // Coulomb blocks); the lists of a class are neighbours, so that the Coulomb
+  // block of a position follows from the position alone.
   auto bucket = [&](int p) {
     const int n = b->pairs_h[p].npp_sig;
     int k = 0;
     while (k < NB - 1 && (2 << k) <= n) ++k;
     return k;
   };
+  auto list_of = [&](int m, int pc, int k) { return (size_t(pc) * nm + m) * NB + k; };
   const size_t nlists = size_t(nm) * NPC * NB;
   std::vector<std::vector<int>> lists(nlists);
-  std::vector<int> pbk(npairs), ppos(npairs);
-  for (int p = 0; p < npairs; ++p) {
-    pbk[p] = bucket(p);
-    const int m = b->sh_mol[b->pi[p]];
-    lists[(size_t(m) * NPC + b->pair_cls[p]) * NB + pbk[p]].push_back(p);
-  }
+  for (int p = 0; p < npairs; ++p)
+    lists[list_of(b->sh_mol[b->pi[p]], b->pair_cls[p], bucket(p))].push_back(p);
   std::vector<int> loff(nlists + 1, 0);
   for (size_t l = 0; l < nlists; ++l) {
     auto& v = lists[l];
     std::stable_sort(v.begin(), v.end(), [&](int x, int y) { return Qp[x] > Qp[y]; });
-    for (int k = 0; k < int(v.size()); ++k) ppos[v[k]] = k;
     loff[l + 1] = loff[l] + int(v.size());
   }
   std::vector<int> kets_h(npairs);
+  std::vector<double> Ql(npairs);  // bounds in list order
   for (size_t l = 0; l < nlists; ++l) std::copy(lists[l].begin(), lists[l].end(), kets_h.begin() + loff[l]);
+  for (int k = 0; k < npairs; ++k) Ql[k] = Qp[kets_h[k]];
+  std::vector<long long> jloc(npairs);
+  long long jtot = 0;
+  for (int pc = 0; pc < NPC; ++pc) {
+    const int k0 = loff[list_of(0, pc, 0)], k1 = loff[list_of(0, pc, 0) + size_t(nm) * NB];
+    const int nf = ncart(pc_La(pc)) * ncart(pc_Lb(pc));
+    b->jl0[pc] = jtot - (long long)k0 * nf;
+    for (int k = k0; k < k1; ++k) jloc[kets_h[k]] = b->jl0[pc] + (long long)k * nf;
+    jtot += (long long)(k1 - k0) * nf;
+  }
 
   // Per quartet class: for every bra pair (heaviest primitive bucket first,
   // then decreasing bound) the segments of kets that pass the Schwarz test.
@@ -1101,28 +1130,28 @@ extern "C" int lai_dev_build_worklist(lai_basis* b, double thr, const double* sh
     int64_t tot = 0;
     for (int m = 0; m < nm; ++m)
       for (int bb = NB - 1; bb >= 0; --bb) {
-        const size_t lb = (size_t(m) * NPC + pb) * NB + bb;
-        for (int p : lists[lb]) {
+        const size_t lb = list_of(m, pb, bb);
+        for (int p = loff[lb]; p < loff[lb + 1]; ++p) {
           Entry e{};
           e.bra = p;
           int acc = 0;
           for (int kb = NB - 1; kb >= 0; --kb) {
-            const size_t lk = (size_t(m) * NPC + pk) * NB + kb;
+            const size_t lk = list_of(m, pk, kb);
             const int len = loff[lk + 1] - loff[lk];
             if (len == 0) continue;
             int lo = 0;
             if (pb == pk) {
               if (kb < bb) continue;
-              if (kb == bb) lo = ppos[p];
+              if (kb == bb) lo = p - loff[lb];
             }
             int hi = len;
             if (screen) {  // first position where Q_p Q_r >= thr fails
-              const int* v = kets_h.data() + loff[lk];
+              const double* v = Ql.data() + loff[lk];
               int a = 0, z = len;
-              const double qp = Qp[p];
+              const double qp = Ql[p];
               while (a < z) {
                 const int mid = (a + z) / 2;
-                if (qp * Qp[v[mid]] >= thr)
+                if (qp * v[mid] >= thr)
                   a = mid + 1;
                 else
                   z = mid;
@@ -1162,9 +1191,16 @@ extern "C" int lai_dev_build_worklist(lai_basis* b, double thr, const double* sh
   hipError_t e;
   if ((e = b->kets.assign(kets_h.data(), kets_h.size())) != hipSuccess ||
       (e = b->segs.assign(segs_h.data(), segs_h.size())) != hipSuccess ||
-      (e = b->dQ.assign(Qp.data(), Qp.size())) != hipSuccess ||
+      (e = b->dQ.assign(Ql.data(), Ql.size())) != hipSuccess ||
+      (e = b->jloc.assign(jloc.data(), jloc.size())) != hipSuccess ||
+      (e = b->lpairs.alloc(size_t(npairs))) != hipSuccess ||
       (e = b->sdmax.assign(sdm.data(), sdm.size())) != hipSuccess)
     return fail(LAI_ERR_MEMORY, std::string("lai_dev_build_worklist: ") + hipGetErrorString(e));
+  if (npairs > 0) {
+    hipLaunchKernelGGL(gather_pairs_kernel, dim3(std::min((npairs + 255) / 256, 4096)), dim3(256), 0, nullptr,
+                       b->pairs.p, b->kets.p, npairs, b->lpairs.p);
+    LAI_HIP(hipGetLastError());
+  }
   for (int c = 0; c < kNumClasses; ++c) {
     const int rc = upload_chunks(b, c);
     if (rc != LAI_OK) return rc;
@@ -1198,8 +1234,7 @@ extern "C" int lai_dev_build_worklist(lai_basis* b, double thr, const double* sh
   LAI_HIP(hipMemset(dsum.p, 0, sizeof(unsigned long long)));
   WlStatsArgs sa{};
   sa.segs = b->segs.p;
-  sa.kets = b->kets.p;
-  sa.pairs = b->pairs.p;
+  sa.pairs = b->lpairs.p;
   sa.sel = make_sel(b);
   sa.L = b->dL.p;
   sa.fp = dfp.p;
@@ -1314,14 +1349,13 @@ static int build_persist_queue(lai_basis* b) {
 // Without: the parts are spread over st and the side streams (each to the
 // stream with the least work so far, by executed flops), forked from and
 // joined back into st, so that the last workgroups of one class overlap the
-// next classes (every class adds into Jt and Kt with atomics only, so the
+// next classes (every class adds into Jl and Kt with atomics only, so the
 // order is free).
 static int launch_jk_classes(lai_basis* b, EriArgs a, int flags, hipStream_t st, hipEvent_t* ev) {
   const auto& Ls = launchers();
   const bool mixed = (flags & LAI_JK_MIXED) != 0 && b->wl_mixed;
   const bool persist = (flags & LAI_JK_PERSISTENT) != 0 && (flags & LAI_JK_MIXED) == 0;
   a.segs = b->segs.p;
-  a.kets = b->kets.p;
   a.sel = make_sel(b);
   const int sel_mixed = a.sel.mixed;
   const bool fan = ev == nullptr && b->fork != nullptr;
@@ -1389,30 +1423,48 @@ static int launch_jk_classes(lai_basis* b, EriArgs a, int flags, hipStream_t st,
   return LAI_OK;
 }
 
-// arguments of a J/K build into the scratch Jt, Kt
+// arguments of a J/K build into the scratch Jl, Kt
 static EriArgs jk_args(lai_basis* b, const double* d_D) {
   EriArgs a{};
-  a.pairs = b->pairs.p;
+  a.pairs = b->lpairs.p;
   a.pp = b->pp.p;
   a.rys = b->ctx->rys.p;
   a.ppb = b->ppb.p;
   a.ppih = b->ppih.p;
   a.pcut32 = b->pcut32;
   a.D = d_D;
-  a.Jt = b->Jt.p;
-  a.Kt = b->Kt.p;
+  a.Kt = b->acc.p;
+  a.Jl = b->acc.p + b->mat_size;
+  std::copy(b->jl0, b->jl0 + kNumPairClasses, a.jl0);
   a.nbf = b->max_nbf;
   a.mode = 0;
   return a;
 }
 
+static int clear_jk_scratch(lai_basis* b, void* stream) {
+  return lai_dev_zero(b->acc.p, size_t(b->mat_size + b->jl_size), stream);
+}
+
 // J += (Jt + Jt^T)/2, K += (Kt + Kt^T)/2; with anti (antisymmetric D) only
 // K += (Kt - Kt^T)/2
-static int symmetrize(lai_basis* b, double* d_J, double* d_K, hipStream_t st, bool anti = false) {
-  const size_t nn = size_t(b->max_nbf) * b->max_nbf;
-  const unsigned blocks = unsigned(std::max<size_t>(1, std::min<size_t>((nn + 255) / 256, 2048)));
-  hipLaunchKernelGGL(symmetrize_add_batch_kernel, dim3(blocks, unsigned(b->n_mol)), dim3(256), 0, st, b->Jt.p,
-                     b->Kt.p, d_J, d_K, b->dmoff.p, b->dmnbf.p, anti ? 1 : 0);
+static int finish_jk(lai_basis* b, double* d_J, double* d_K, hipStream_t st, bool anti = false) {
+  if (b->max_nbf == 0) return LAI_OK;
+  FinishArgs a{};
+  a.Jl = b->acc.p + b->mat_size;
+  a.jloc = b->jloc.p;
+  a.Kt = b->acc.p;
+  a.J = d_J;
+  a.K = d_K;
+  a.moff = b->dmoff.p;
+  a.mnbf = b->dmnbf.p;
+  a.mpair = b->dmpair.p;
+  a.mshell = b->dmshell.p;
+  a.mfunc = b->dmfunc.p;
+  a.fsh = b->dfsh.p;
+  a.L = b->dL.p;
+  a.func_off = b->dfunc_off.p;
+  hipLaunchKernelGGL(finish_jk_kernel, dim3(unsigned(std::min(b->max_nbf, 4096)), unsigned(b->n_mol)), dim3(256), 0, st,
+                     a, anti ? 1 : 0);
   LAI_HIP(hipGetLastError());
   return LAI_OK;
 }
@@ -1423,18 +1475,16 @@ extern "C" int lai_dev_jk(lai_basis* b, const double* d_D, double* d_J, double* 
   if ((flags & ~(LAI_JK_MIXED | LAI_JK_ANTISYMMETRIC | LAI_JK_PERSISTENT)) != 0)
     return fail(LAI_ERR_INVALID_ARGUMENT, "lai_dev_jk: unknown flags");
   hipStream_t st = hipStream_t(stream);
-  const size_t nn = size_t(b->mat_size);
   int rc;
   if (!b->fork) {  // side streams are created outside any stream capture
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     LAI_HIP(hipStreamIsCapturing(st, &cs));
     if (cs == hipStreamCaptureStatusNone && (rc = ensure_side_streams(b)) != LAI_OK) return rc;
   }
-  if ((rc = lai_dev_zero(b->Jt.p, nn, stream)) != LAI_OK) return rc;
-  if ((rc = lai_dev_zero(b->Kt.p, nn, stream)) != LAI_OK) return rc;
+  if ((rc = clear_jk_scratch(b, stream)) != LAI_OK) return rc;
   if ((rc = launch_jk_classes(b, jk_args(b, d_D), flags, st, nullptr)) != LAI_OK) return rc;
   LAI_HIP(hipGetLastError());
-  return symmetrize(b, d_J, d_K, st, (flags & LAI_JK_ANTISYMMETRIC) != 0);
+  return finish_jk(b, d_J, d_K, st, (flags & LAI_JK_ANTISYMMETRIC) != 0);
 }
 
 extern "C" int lai_dev_jk_graph_capture(lai_basis* b, const double* d_D, double* d_J, double* d_K, int flags,
@@ -1583,7 +1633,7 @@ extern "C" int lai_dev_jk_grad(lai_basis* b, const double* d_D, double xscale, d
   hipStream_t st = hipStream_t(stream);
   const auto& G = grad_launchers();
   GradArgs a{};
-  a.pairs = b->pairs.p;
+  a.pairs = b->lpairs.p;
   a.pp = b->pp.p;
   a.ppab = b->ppab.p;
   a.rys = b->ctx->rys.p;
@@ -1595,7 +1645,6 @@ extern "C" int lai_dev_jk_grad(lai_basis* b, const double* d_D, double xscale, d
   a.n_atoms = b->n_atoms;
   a.ppih = b->ppih.p;
   a.segs = b->segs.p;
-  a.kets = b->kets.p;
   a.sel = make_sel(b);
   a.sel.mixed = 0;  // the gradient runs every quartet in FP64
   const int max_blocks = b->ctx->n_cu * 16;
@@ -1738,7 +1787,6 @@ extern "C" int lai_dev_autotune(lai_basis* b, const double* d_D, int flags, int 
   const int n_cu = b->ctx->n_cu;
   EriArgs a = jk_args(b, d_D);
   a.segs = b->segs.p;
-  a.kets = b->kets.p;
   a.sel = make_sel(b);
   const bool mixed = flags == LAI_JK_MIXED && b->wl_mixed;
   const int sel_mixed = a.sel.mixed;
@@ -1902,15 +1950,13 @@ extern "C" int lai_dev_jk_profile(lai_basis* b, const double* d_D, double* d_J, 
   if ((flags & ~(LAI_JK_MIXED | LAI_JK_ANTISYMMETRIC)) != 0)
     return fail(LAI_ERR_INVALID_ARGUMENT, "lai_dev_jk_profile: unknown flags");
   hipStream_t st = hipStream_t(stream);
-  const size_t nn = size_t(b->mat_size);
   int rc;
-  if ((rc = lai_dev_zero(b->Jt.p, nn, stream)) != LAI_OK) return rc;
-  if ((rc = lai_dev_zero(b->Kt.p, nn, stream)) != LAI_OK) return rc;
+  if ((rc = clear_jk_scratch(b, stream)) != LAI_OK) return rc;
   std::vector<hipEvent_t> ev(4 * kNumClasses, nullptr);
   for (auto& e : ev) LAI_HIP(hipEventCreate(&e));
   launch_jk_classes(b, jk_args(b, d_D), flags, st, ev.data());
   LAI_HIP(hipGetLastError());
-  if ((rc = symmetrize(b, d_J, d_K, st, (flags & LAI_JK_ANTISYMMETRIC) != 0)) != LAI_OK) return rc;
+  if ((rc = finish_jk(b, d_J, d_K, st, (flags & LAI_JK_ANTISYMMETRIC) != 0)) != LAI_OK) return rc;
   LAI_HIP(hipStreamSynchronize(st));
   // the FP64 and FP32 launches of each class (the FP32 one is empty unless
   // the build is mixed)

@@ -1,5 +1,5 @@
-// aux_kernels.hip -- fills, J/K symmetrisation, Schwarz reduction, one-electron
-// integrals and the Rys/Boys probes.
+// aux_kernels.hip -- fills, Schwarz reduction, one-electron integrals and the
+// Rys/Boys probes.
 #include "aux_kernels.hpp"
 
 namespace lai {
@@ -7,17 +7,6 @@ namespace lai {
 __global__ void fill_zero_kernel(double* __restrict__ p, size_t n) {
   for (size_t i = size_t(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += size_t(gridDim.x) * blockDim.x)
     p[i] = 0.0;
-}
-
-__global__ void symmetrize_add_kernel(const double* __restrict__ Jt, const double* __restrict__ Kt,
-                                      double* __restrict__ J, double* __restrict__ K, int n) {
-  const size_t nn = size_t(n) * n;
-  for (size_t x = size_t(blockIdx.x) * blockDim.x + threadIdx.x; x < nn; x += size_t(gridDim.x) * blockDim.x) {
-    const size_t i = x / n, j = x - i * n;
-    const size_t t = j * n + i;
-    J[x] += 0.5 * (Jt[x] + Jt[t]);
-    K[x] += 0.5 * (Kt[x] + Kt[t]);
-  }
 }
 
 __global__ void schwarz_reduce_kernel(const double* __restrict__ blocks,

@@ -1,6 +1,5 @@
-// aux_kernels.hpp -- small device kernels of the backend: fills, the J/K
-// symmetrisation, the Schwarz diagonal reduction, one-electron integrals and
-// the math probes.
+// aux_kernels.hpp -- small device kernels of the backend: fills, the
+// Schwarz diagonal reduction, one-electron integrals and the math probes.
 #pragma once
 
 #include "common.hpp"
@@ -8,10 +7,6 @@
 namespace lai {
 
 __global__ void fill_zero_kernel(double* __restrict__ p, size_t n);
-
-// J += (Jt + Jt^T)/2, K += (Kt + Kt^T)/2
-__global__ void symmetrize_add_kernel(const double* __restrict__ Jt, const double* __restrict__ Kt,
-                                      double* __restrict__ J, double* __restrict__ K, int n);
 
 // Q[p] = sqrt(max_ab |(ab|ab)|) for the (i,j,i,j) blocks of every pair
 __global__ void schwarz_reduce_kernel(const double* __restrict__ blocks,

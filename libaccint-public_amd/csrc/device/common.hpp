@@ -102,11 +102,14 @@ struct Quartet {
   int bra, ket;
 };
 
-// Worklist of a quartet class.  For one bra pair, the kets that pass the
-// Schwarz test form up to kMaxSegs contiguous runs ("segments") of the ket
-// array, one per primitive-count bucket of the ket pair class: segment s
-// holds kets[start[s] .. start[s] + cum[s+1] - cum[s]).  A chunk is the part
-// [k0, k1) of that concatenated run handled by one workgroup.
+// Worklist of a quartet class.  The pairs of a handle are listed class by
+// class, then by molecule and primitive-count bucket, in order of decreasing
+// Schwarz bound; worklist records name a pair by its position in that list.
+// For one bra pair, the kets that pass the Schwarz test form up to kMaxSegs
+// contiguous runs ("segments") of the list, one per bucket of the ket pair
+// class: segment s holds the positions start[s] .. start[s] + cum[s+1] -
+// cum[s] - 1.  A chunk is the part [k0, k1) of that concatenated run handled
+// by one workgroup.
 inline constexpr int kMaxSegs = 8;
 struct JkSegs {
   int n;
@@ -382,6 +385,14 @@ __device__ __forceinline__ PairRec load_pair_uniform(const PairRec* base, int i)
   r.ABz = p->ABz;
   r.bsum = p->bsum;
   return r;
+}
+
+// A chunk whose index is uniform over the workgroup, likewise: the chunk and
+// what is computed from it stay in SGPRs (as a plain load of the class kernels
+// it would sit in VGPRs, since they store to memory between the chunks)
+__device__ __forceinline__ JkChunk load_chunk_uniform(const JkChunk* base, int i) {
+  const_ptr<int> p = as_const(reinterpret_cast<const int*>(base + i));
+  return JkChunk{p[0], p[1], p[2], p[3]};
 }
 
 // FP64 add to LDS (ds_add_f64)

@@ -114,7 +114,7 @@ void launch_class(const EriArgs& a0, hipStream_t s, const LaunchTune& t) {
       auto kern = jk_kernel_merged<La, Lb, Lc, Ld, MIXED, P::CHA, false>;
       static const size_t stat = static_lds(kern);
       static const size_t dmax = dyn_limit(kern, stat);
-      const size_t per_rep = size_t(P::NCH) * nc * nd * 64 * sizeof(double);
+      const size_t per_rep = size_t(P::NCH) * nc * nd * kJPad * sizeof(double);
       const size_t rows = size_t(na + nb) * nbf * sizeof(double);
       RowsPick rp = pick_rows(kern, dmax, 64 * P::NCH, per_rep, rows);
       // the Rys tables in LDS as well (one to four roots) when that keeps as
@@ -135,10 +135,11 @@ void launch_class(const EriArgs& a0, hipStream_t s, const LaunchTune& t) {
       hipLaunchKernelGGL(kern, dim3(grid_cap(kBlocksPerCuRegs)), dim3(64 * P::NCH * rp.rep), rp.dyn, s, a);
     } else if constexpr (P::regs) {
       const size_t rows = size_t(P::CHA + nb) * nbf * sizeof(double);
+      const size_t per_rep = size_t(4) * kJTile<Lc, Ld> * sizeof(double);
       auto kern = jk_kernel_regs<La, Lb, Lc, Ld, MIXED, P::CHA, false>;
       static const size_t stat = static_lds(kern);
       static const size_t dmax = dyn_limit(kern, stat);
-      RowsPick rp = pick_rows(kern, dmax, 256, 0, rows);
+      RowsPick rp = pick_rows(kern, dmax, 256, per_rep, rows);
       bool lb = false;
       // one- to four-root classes: the Rys tables (Boys Taylor rows or
       // Chebyshev coefficients) in LDS as well, when that keeps as many
@@ -150,7 +151,7 @@ void launch_class(const EriArgs& a0, hipStream_t s, const LaunchTune& t) {
         static const size_t stat_l = static_lds(kl);
         static const size_t dmax_l = dyn_limit(kl, stat_l);
         const RowsPick rl =
-            pick_rows(kl, dmax_l, 256, 0, rows, size_t(kLdsRysDoubles<La, Lb, Lc, Ld>) * sizeof(double));
+            pick_rows(kl, dmax_l, 256, per_rep, rows, size_t(kLdsRysDoubles<La, Lb, Lc, Ld>) * sizeof(double));
         if (rl.rows >= rp.rows && rl.waves >= rp.waves && rl.waves >= 2 * 4 * rl.rep) {
           rp = rl;
           lb = true;

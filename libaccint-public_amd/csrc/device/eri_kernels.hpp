@@ -27,6 +27,18 @@
 // scatter of FockBuilder::accumulate_symmetric
 // (src/shared/consumers/fock_builder.cpp:123-222):
 //   Jt[ab] += s_ij s_kl g D[cd]          Jt[cd] += s_ij s_kl g D[ab]   (!bk)
+// Jt is stored by shell pair in worklist order (Jl): the block of the pair at
+// list position p of pair class x at Jl + jl0[x] + p * (its functions).  The
+// kets of a chunk are runs of the list, so their Coulomb blocks are contiguous
+// and the kernels add them whole cache lines at a time: the device resolves
+// about 23.7e9 atomic cache-line operations per second whatever they hold
+// (1.05e8 FP64 adds to random elements of an n x n matrix take 4.42 ms for n
+// from 400 to 1400, the same number in runs of 64 neighbours 0.57 ms).  With
+// Jt as an n x n matrix, one such operation per quartet and element bound the
+// classes of few primitives: class kernels of C40H82 def2-SVP 68.4 -> 46.4 ms
+// ((ps|ss) 9.0 -> 5.6, (ps|ps) 10.2 -> 5.0), of C17H36 39.3 -> 22.0 ms, of 16
+// waters cc-pVDZ 24.1 -> 21.8 ms; leaving the additions out altogether gives
+// 48.6, 22.9 and 22.0 ms, so they are no longer what bounds these kernels.
 //   Kt[ac] += s_bk g D[bd]               Kt[ad] += s_bk g D[bc]        (!kl)
 //   Kt[bc] += s_bk g D[ad]   (!ij)       Kt[bd] += s_bk g D[ac]        (!ij && !kl)
 // with s_x = 1 if the flag is set, else 2.
@@ -72,11 +84,11 @@ __device__ __forceinline__ int quartet_select(const QuartetSel& s, int bp, const
   return (s.keep == 0 || s.keep == mode) ? mode : 0;
 }
 
-// Ket pair of position k of a chunk's run; seg walks forward with k.
-__device__ __forceinline__ int chunk_ket(const int* __restrict__ kets, const JkSegs* __restrict__ sg, int k,
-                                         int& seg) {
+// List position of the ket at position k of a chunk's run; seg walks forward
+// with k.
+__device__ __forceinline__ int chunk_ket(const JkSegs* __restrict__ sg, int k, int& seg) {
   while (seg + 1 < sg->n && k >= sg->cum[seg + 1]) ++seg;
-  return kets[sg->start[seg] + (k - sg->cum[seg])];
+  return sg->start[seg] + (k - sg->cum[seg]);
 }
 
 // Lane schedule of the lane-per-quartet kernels.  The quartets of a chunk
@@ -87,19 +99,47 @@ __device__ __forceinline__ int chunk_ket(const int* __restrict__ kets, const JkS
 constexpr int kSortRun = 2048;                 // quartets sorted at a time
 constexpr int kSortBins = 256;                 // key: 128 * FP32 + min(npp_sig, 127)
 constexpr unsigned kSortF32 = 0x80000000u;     // flag bit of a sorted entry
+// WIN: for classes whose ket is a pair of s shells (one Coulomb element per
+// quartet) the entry's slot, read once by its lane, then takes the quartet's
+// Coulomb element, and inv (run position -> sorted entry) lets the workgroup
+// add the run's elements to Jl in list order, whole cache lines at a time.
+template <bool WIN>
 struct SortLds {
-  unsigned kp[kSortRun];  // ket pair, kSortF32 set for the FP32 recursion
+  static constexpr bool win = false;
+  unsigned kp[kSortRun];  // list position of the ket, kSortF32 set for the FP32 recursion
   int cnt[kSortBins];
   int n;
+  __device__ __forceinline__ unsigned get(int i) const { return kp[i]; }
+  __device__ __forceinline__ void put(int i, unsigned e, int) { kp[i] = e; }
+  __device__ __forceinline__ void skip(int) {}
+};
+template <>
+struct SortLds<true> {
+  static constexpr bool win = true;
+  static constexpr unsigned short none = 0xffff;  // a quartet that takes no lane
+  union Slot {
+    unsigned kp;
+    double j;
+  };
+  Slot slot[kSortRun];
+  unsigned short inv[kSortRun];
+  int cnt[kSortBins];
+  int n;
+  __device__ __forceinline__ unsigned get(int i) const { return slot[i].kp; }
+  __device__ __forceinline__ void put(int i, unsigned e, int k) {
+    slot[i].kp = e;
+    inv[k] = (unsigned short)i;
+  }
+  __device__ __forceinline__ void skip(int k) { inv[k] = none; }
 };
 
-// Sorts positions [s0, s1) (at most kSortRun) of a chunk's run into s.kp and
+// Sorts positions [s0, s1) (at most kSortRun) of a chunk's run into s and
 // returns how many were kept.  All nt lanes of the workgroup call it (nt a
 // multiple of 64, at least NTMIN); it ends on a barrier.
-template <int NTMIN>
-__device__ __forceinline__ int sort_run(const int* __restrict__ kets, const JkSegs* __restrict__ sg,
-                                        const PairRec* __restrict__ pairs, const QuartetSel& sel, int bp,
-                                        const PairRec& bra, int s0, int s1, SortLds& s, int nt) {
+template <int NTMIN, typename S>
+__device__ __forceinline__ int sort_run(const JkSegs* __restrict__ sg, const PairRec* __restrict__ pairs,
+                                        const QuartetSel& sel, int bp, const PairRec& bra, int s0, int s1, S& s,
+                                        int nt) {
   constexpr int kSortPer = (kSortRun + NTMIN - 1) / NTMIN;  // positions per lane, at most
   const int tid = threadIdx.x;
   for (int i = tid; i < kSortBins; i += nt) s.cnt[i] = 0;
@@ -113,7 +153,7 @@ __device__ __forceinline__ int sort_run(const int* __restrict__ kets, const JkSe
     kp[j] = 0;
     rk[j] = 0;
     if (k < s1) {
-      kp[j] = chunk_ket(kets, sg, k, seg);
+      kp[j] = chunk_ket(sg, k, seg);
       const PairRec ket = pairs[kp[j]];
       const int mode = quartet_select(sel, bp, bra, kp[j], ket);
       if (mode != 0) {
@@ -146,19 +186,24 @@ __device__ __forceinline__ int sort_run(const int* __restrict__ kets, const JkSe
   }
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < kSortPer; ++j)
-    if (key[j] >= 0) s.kp[s.cnt[key[j]] + rk[j]] = unsigned(kp[j]) | (key[j] >= 128 ? kSortF32 : 0u);
+  for (int j = 0; j < kSortPer; ++j) {
+    const int k = tid + nt * j;
+    if (key[j] >= 0)
+      s.put(s.cnt[key[j]] + rk[j], unsigned(kp[j]) | (key[j] >= 128 ? kSortF32 : 0u), k);
+    else if (s0 + k < s1)
+      s.skip(k);
+  }
   __syncthreads();
   return s.n;
 }
 
-// Sorted position of lane tid in round r of a workgroup of nw wavefronts (a
-// power of two): the wavefronts take the nw 64-entry blocks of a round in an
-// order that rotates with r, so that no wavefront always gets the heaviest
-// block.
-__device__ __forceinline__ int sorted_pos(int tid, int r, int nw) {
+// First sorted entry of the 64-entry block that the wavefront of lane tid
+// takes in round r of a workgroup of nw wavefronts (a power of two): the
+// wavefronts take the nw blocks of a round in an order that rotates with r,
+// so that no wavefront always gets the heaviest block.
+__device__ __forceinline__ int sorted_block(int tid, int r, int nw) {
   const int w = tid >> 6;
-  return 64 * (nw * r + ((w + r) & (nw - 1))) + (tid & 63);
+  return 64 * (nw * r + ((w + r) & (nw - 1)));
 }
 
 struct EriArgs {
@@ -173,9 +218,11 @@ struct EriArgs {
   const float* __restrict__ ppb;
   double pcut32;
   const double* __restrict__ ppih;  // 1 / (2 zeta) of each primitive pair
-  // mode 0: digestion into D, Jt, Kt (molecule blocks at PairRec::moff)
+  // mode 0: digestion of D into Jl (blocks of the pairs in list order) and Kt
+  // (molecule blocks at PairRec::moff)
   const double* __restrict__ D;
-  double* Jt;
+  double* Jl;
+  long long jl0[kNumPairClasses];
   double* Kt;
   int nbf;  // largest molecule (LDS rows)
   int mode;
@@ -183,11 +230,11 @@ struct EriArgs {
   double* out;
   const int* __restrict__ perm;        // per quartet: packed original position of class positions
   const long long* __restrict__ obase;  // per quartet: offset of its block in out
-  // mode 0 worklist: bra-anchored chunks over ket segments
+  // mode 0 worklist: bra-anchored chunks over ket segments; pairs holds the
+  // records in list order, and bra and ket are list positions
   const JkChunk* __restrict__ chunks;
   int nchunks;
   const JkSegs* __restrict__ segs;
-  const int* __restrict__ kets;
   int klds;  // 1: the bra rows of Kt are accumulated in LDS (dynamic shared memory)
   QuartetSel sel;
 };
@@ -833,19 +880,44 @@ __global__ __launch_bounds__(NT) void eri_kernel_lds(EriArgs g) {
 // selects only the FP32 quartets, QuartetSel::keep == 2); otherwise FP64.
 // Lanes take the chunk's quartets in the order of sort_run.
 // --------------------------------------------------------------------------
-template <int La, int Lb, int Lc, int Ld, bool MIXED, int A0, int A1, bool LB = false>
-__device__ __forceinline__ void jk_chunk_regs(const EriArgs& g, const JkChunk& ch, double* krow, SortLds& srt,
-                                              lds_cdptr lrows = nullptr) {
+// Doubles of the ket Coulomb tile of a wavefront (jk_chunk_regs): 64 blocks of
+// nc nd, none for an (ss| ket, whose elements go through the sort's slots.
+template <int Lc, int Ld>
+inline constexpr int kJTile = ncart(Lc) * ncart(Ld) > 1 ? 64 * ncart(Lc) * ncart(Ld) : 0;
+
+// Adds the Coulomb blocks of 64 sorted quartets (entries i0 .. i0 + 63) to
+// Jl: element t of the blocks laid one after another is at(q, e), e of quartet
+// q; lanes l0, l0 + nl, ... take consecutive elements, so that neighbouring
+// lanes add to one ket's contiguous block.  The bra's own pair takes none.
+template <int NCD, typename S, typename F>
+__device__ __forceinline__ void add_ket_blocks(double* __restrict__ Jl, const S& srt, int i0, int nsel, int bra, int l0,
+                                               int nl, F&& at) {
+#pragma unroll
+  for (int t = l0; t < 64 * NCD; t += nl) {
+    const int q = t / NCD, e = t - q * NCD;
+    if (i0 + q >= nsel) break;
+    const int pos = int(srt.get(i0 + q) & ~kSortF32);
+    if (pos != bra) atomic_add(&Jl[(long long)pos * NCD + e], at(q, e));
+  }
+}
+
+template <int La, int Lb, int Lc, int Ld, bool MIXED, int A0, int A1, bool LB = false, typename S>
+__device__ __forceinline__ void jk_chunk_regs(const EriArgs& g, const JkChunk& ch, double* krow, S& srt,
+                                              double* jtile, lds_cdptr lrows = nullptr) {
   constexpr int nb = ncart(Lb), nc = ncart(Lc), nd = ncart(Ld);
   constexpr int NA = A1 - A0;
   constexpr int ROWS = NA + nb;
+  constexpr int NCD = nc * nd;
+  constexpr bool WIN = NCD == 1;
+  static_assert(!WIN || S::win, "an (ss| ket needs the sort with Coulomb slots");
   const int tid = threadIdx.x, nt = blockDim.x;
   const bool lds = g.klds != 0;
-  const PairRec bra = g.pairs[ch.bra];
+  const PairRec bra = load_pair_uniform(g.pairs, ch.bra);
   const int n = bra.mn;
   const double* __restrict__ D = g.D + bra.moff;
-  double* Jt = g.Jt + bra.moff;
+  double* Jk = g.Jl + g.jl0[pair_class(Lc, Ld)];
   double* Kt = g.Kt + bra.moff;
+  jtile += (tid >> 6) * kJTile<Lc, Ld>;  // this wavefront's
   const int fa = bra.fa + A0, fb = bra.fb;
   const bool ij = bra.same;
   const JkSegs* sg = g.segs + ch.seg;
@@ -867,12 +939,13 @@ __device__ __forceinline__ void jk_chunk_regs(const EriArgs& g, const JkChunk& c
     for (int b = 0; b < nb; ++b) jab[a][b] = 0.0;
 
   for (int s0 = ch.k0; s0 < ch.k1; s0 += kSortRun) {
-  const int nsel = sort_run<256>(g.kets, sg, g.pairs, g.sel, ch.bra, bra, s0, min(ch.k1, s0 + kSortRun), srt, nt);
+  const int s1 = min(ch.k1, s0 + kSortRun);
+  const int nsel = sort_run<256>(sg, g.pairs, g.sel, ch.bra, bra, s0, s1, srt, nt);
   for (int r = 0; nt * r < nsel; ++r) {
-    const int i = sorted_pos(tid, r, nt >> 6);
-    if (i >= nsel) continue;
-    const unsigned e = srt.kp[i];
-    const int kp = int(e & ~kSortF32);
+    const int i0 = sorted_block(tid, r, nt >> 6);  // uniform over the wavefront
+    const int i = i0 + (tid & 63);
+    if (i < nsel) {
+    const int kp = int(srt.get(i) & ~kSortF32);
     const PairRec ket = g.pairs[kp];
     double gv[NA][nb][nc][nd];
     if constexpr (MIXED)
@@ -895,19 +968,21 @@ __device__ __forceinline__ void jk_chunk_regs(const EriArgs& g, const JkChunk& c
           for (int d = 0; d < nd; ++d) s += gv[a][b][c][d] * D[size_t(fc + c) * n + fd + d];
         jab[a][b] += fJ * s;
       }
-    if (!bk) {  // Jt[cd] += fJ sum_ab g D[ab]
+    // Jt[cd] += fJ sum_ab g D[ab] (!bk), through LDS
 #pragma unroll
-      for (int c = 0; c < nc; ++c)
+    for (int c = 0; c < nc; ++c)
 #pragma unroll
-        for (int d = 0; d < nd; ++d) {
-          double s = 0.0;
+      for (int d = 0; d < nd; ++d) {
+        double s = 0.0;
 #pragma unroll
-          for (int a = 0; a < NA; ++a)
+        for (int a = 0; a < NA; ++a)
 #pragma unroll
-            for (int b = 0; b < nb; ++b) s += gv[a][b][c][d] * D[size_t(fa + a) * n + fb + b];
-          atomic_add(&Jt[size_t(fc + c) * n + fd + d], fJ * s);
-        }
-    }
+          for (int b = 0; b < nb; ++b) s += gv[a][b][c][d] * D[size_t(fa + a) * n + fb + b];
+        if constexpr (WIN)
+          srt.slot[i].j = bk ? 0.0 : fJ * s;
+        else
+          jtile[(tid & 63) * NCD + c * nd + d] = fJ * s;
+      }
     // Kt[ac] += fK sum_bd g D[bd]
 #pragma unroll
     for (int a = 0; a < NA; ++a)
@@ -959,15 +1034,35 @@ __device__ __forceinline__ void jk_chunk_regs(const EriArgs& g, const JkChunk& c
           kadd(NA + b, fd + d, fK * s);
         }
     }
+    }
+    if constexpr (!WIN) {
+      wave_sync();  // the wavefront's blocks are in its tile
+      add_ket_blocks<NCD>(Jk, srt, i0, nsel, ch.bra, tid & 63, 64, [&](int q, int e) { return jtile[q * NCD + e]; });
+      wave_sync();  // the tile is read before the next round fills it
+    }
+  }
+  if constexpr (WIN) {
+    __syncthreads();  // the run's Coulomb elements are in their slots
+    int seg = 0;
+#pragma unroll 1
+    for (int k = s0 + tid; k < s1; k += nt) {
+      const unsigned short q = srt.inv[k - s0];
+      const int pos = chunk_ket(sg, k, seg);
+      if (q != S::none) {
+        const double v = srt.slot[q].j;
+        if (v != 0.0) atomic_add(&Jk[pos], v);
+      }
+    }
   }
   }
   // Jt[ab]: one atomic per wavefront and element
+  double* Jb = g.Jl + g.jl0[pair_class(La, Lb)] + (long long)ch.bra * (ncart(La) * nb);
 #pragma unroll
   for (int a = 0; a < NA; ++a)
 #pragma unroll
     for (int b = 0; b < nb; ++b) {
       const double v = wave_sum(jab[a][b]);
-      if ((tid & 63) == 0 && v != 0.0) atomic_add(&Jt[size_t(fa + a) * n + fb + b], v);
+      if ((tid & 63) == 0 && v != 0.0) atomic_add(&Jb[(A0 + a) * nb + b], v);
     }
   if (lds) {
     __syncthreads();
@@ -982,16 +1077,16 @@ __device__ __forceinline__ void jk_chunk_regs(const EriArgs& g, const JkChunk& c
   }
 }
 
-template <int La, int Lb, int Lc, int Ld, bool MIXED, int CHA, int C, bool LB>
-__device__ __forceinline__ void dispatch_jk_chunk(const EriArgs& g, const JkChunk& ch, double* krow, SortLds& srt,
-                                                  int chunk, lds_cdptr lrows) {
+template <int La, int Lb, int Lc, int Ld, bool MIXED, int CHA, int C, bool LB, typename S>
+__device__ __forceinline__ void dispatch_jk_chunk(const EriArgs& g, const JkChunk& ch, double* krow, S& srt,
+                                                  double* jtile, int chunk, lds_cdptr lrows) {
   constexpr int na = ncart(La);
   constexpr int A0 = C * CHA;
   constexpr int A1 = (A0 + CHA < na) ? A0 + CHA : na;
   if (chunk == C) {
-    jk_chunk_regs<La, Lb, Lc, Ld, MIXED, A0, A1, LB>(g, ch, krow, srt, lrows);
+    jk_chunk_regs<La, Lb, Lc, Ld, MIXED, A0, A1, LB>(g, ch, krow, srt, jtile, lrows);
   } else if constexpr (A1 < na) {
-    dispatch_jk_chunk<La, Lb, Lc, Ld, MIXED, CHA, C + 1, LB>(g, ch, krow, srt, chunk, lrows);
+    dispatch_jk_chunk<La, Lb, Lc, Ld, MIXED, CHA, C + 1, LB>(g, ch, krow, srt, jtile, chunk, lrows);
   }
 }
 
@@ -1038,14 +1133,18 @@ __device__ __forceinline__ void copy_rys_lds(const double* __restrict__ rys, dou
   __syncthreads();
 }
 
+// (The chunk and its bra record are read through the constant address space,
+// so what depends on them alone sits in SGPRs: (ss|ss) 93 -> 83 VGPRs,
+// (ps|ps) 154 -> 135, scratch of the merged (dd|ps) 316 -> 212 bytes a lane.)
 // Kernel A, anchored: 256 or 512 lanes per chunk (the launch picks the
 // workgroup that keeps the most wavefronts resident with the exchange rows in
 // LDS), bra index chunk C = blockIdx.y.  Dynamic LDS: with LB, the class's
-// Rys tables, copied once per workgroup, then the exchange rows [CHA + nb][mn].
+// Rys tables, copied once per workgroup, then the wavefronts' ket Coulomb
+// tiles, then the exchange rows [CHA + nb][mn].
 template <int La, int Lb, int Lc, int Ld, bool MIXED, int CHA, bool LB>
 __global__ __launch_bounds__(512) void jk_kernel_regs(EriArgs g) {
   extern __shared__ double dyn[];
-  __shared__ SortLds srt;
+  __shared__ SortLds<(Lc + Ld == 0)> srt;
   constexpr int NB = LB ? kLdsRysDoubles<La, Lb, Lc, Ld> : 0;
   static_assert(!LB || NB > 0, "LDS Rys tables are for one- to four-root classes");
   lds_cdptr lrows = nullptr;
@@ -1053,10 +1152,11 @@ __global__ __launch_bounds__(512) void jk_kernel_regs(EriArgs g) {
     copy_rys_lds<(La + Lb + Lc + Ld) / 2 + 1>(g.rys, dyn);
     lrows = (lds_cdptr)(dyn);
   }
-  double* krow = dyn + NB;
+  double* jtile = dyn + NB;
+  double* krow = jtile + (blockDim.x / 64) * kJTile<Lc, Ld>;
   for (int c = blockIdx.x; c < g.nchunks; c += gridDim.x) {
-    const JkChunk ch = g.chunks[c];
-    dispatch_jk_chunk<La, Lb, Lc, Ld, MIXED, CHA, 0, LB>(g, ch, krow, srt, blockIdx.y, lrows);
+    const JkChunk ch = load_chunk_uniform(g.chunks, c);
+    dispatch_jk_chunk<La, Lb, Lc, Ld, MIXED, CHA, 0, LB>(g, ch, krow, srt, jtile, blockIdx.y, lrows);
   }
 }
 
@@ -1068,9 +1168,12 @@ __global__ __launch_bounds__(512) void jk_kernel_regs(EriArgs g) {
 // consecutive 64-quartet blocks of the sorted run.  The exchange rows of A
 // and B, the sort and the chunk's loads are shared by the whole workgroup;
 // the slices' partial ket Coulomb blocks Jt[cd] meet in LDS and go to HBM
-// with one atomic per element instead of one per slice.
-template <int La, int Lb, int Lc, int Ld, bool MIXED, int CHA, int C, bool LB = false>
-__device__ __forceinline__ void jk_chunk_merged(const EriArgs& g, const JkChunk& ch, double* krow, SortLds& srt,
+// with one atomic per element instead of one per slice, block by block.
+// (kJPad doubles per element: 64 quartets and one of padding, so that the
+// elements of one quartet lie in different banks.)
+constexpr int kJPad = 65;
+template <int La, int Lb, int Lc, int Ld, bool MIXED, int CHA, int C, bool LB = false, typename S>
+__device__ __forceinline__ void jk_chunk_merged(const EriArgs& g, const JkChunk& ch, double* krow, S& srt,
                                                 double* jpart, lds_cdptr lrows = nullptr) {
   constexpr int na = ncart(La), nb = ncart(Lb), nc = ncart(Lc), nd = ncart(Ld);
   constexpr int NCH = (na + CHA - 1) / CHA;
@@ -1080,12 +1183,12 @@ __device__ __forceinline__ void jk_chunk_merged(const EriArgs& g, const JkChunk&
   constexpr int ROWS = na + nb;
   const int tid = threadIdx.x, lane = tid & 63, NT = blockDim.x;
   const int rep = NT / (64 * NCH), grp = (tid >> 6) / NCH;
-  jpart += grp * (NCH * NCD * 64);  // this group's slices
+  jpart += grp * (NCH * NCD * kJPad);  // this group's slices
   const bool lds = g.klds != 0;
-  const PairRec bra = g.pairs[ch.bra];
+  const PairRec bra = load_pair_uniform(g.pairs, ch.bra);
   const int n = bra.mn;
   const double* __restrict__ D = g.D + bra.moff;
-  double* Jt = g.Jt + bra.moff;
+  double* Jk = g.Jl + g.jl0[pair_class(Lc, Ld)];
   double* Kt = g.Kt + bra.moff;
   const int fa = bra.fa, fb = bra.fb;
   const bool ij = bra.same;
@@ -1109,25 +1212,19 @@ __device__ __forceinline__ void jk_chunk_merged(const EriArgs& g, const JkChunk&
 
   for (int s0 = ch.k0; s0 < ch.k1; s0 += kSortRun) {
     const int nsel =
-        sort_run<64 * NCH>(g.kets, sg, g.pairs, g.sel, ch.bra, bra, s0, min(ch.k1, s0 + kSortRun), srt, NT);
+        sort_run<64 * NCH>(sg, g.pairs, g.sel, ch.bra, bra, s0, min(ch.k1, s0 + kSortRun), srt, NT);
     for (int r = 0; 64 * rep * r < nsel; ++r) {
-      const int i = 64 * (rep * r + grp) + lane;
-      const bool valid = i < nsel;
-      int fc = 0, fd = 0;
-      bool bk = true;
-      if (valid) {
-        const unsigned e = srt.kp[i];
-        const int kp = int(e & ~kSortF32);
+      const int i0 = 64 * (rep * r + grp), i = i0 + lane;
+      if (i < nsel) {
+        const int kp = int(srt.get(i) & ~kSortF32);
         const PairRec ket = g.pairs[kp];
         double gv[NA][nb][nc][nd];
         if constexpr (MIXED)
           quartet_block_regs<La, Lb, Lc, Ld, float, A0, A1>(g, bra, ket, false, gv);
         else
           quartet_block_regs<La, Lb, Lc, Ld, double, A0, A1, LB>(g, bra, ket, false, gv, lrows);
-        fc = ket.fa;
-        fd = ket.fb;
-        const bool kl = ket.same;
-        bk = (kp == ch.bra);
+        const int fc = ket.fa, fd = ket.fb;
+        const bool kl = ket.same, bk = (kp == ch.bra);
         const double fJ = (ij ? 1.0 : 2.0) * (kl ? 1.0 : 2.0);
         const double fK = bk ? 1.0 : 2.0;
         // Jt[ab] += fJ sum_cd g D[cd]  (this slice's rows, summed over the chunk)
@@ -1152,9 +1249,9 @@ __device__ __forceinline__ void jk_chunk_merged(const EriArgs& g, const JkChunk&
             for (int a = 0; a < NA; ++a)
 #pragma unroll
               for (int b = 0; b < nb; ++b) t += gv[a][b][c][d] * D[size_t(fa + A0 + a) * n + fb + b];
-            jpart[(C * NCD + c * nd + d) * 64 + lane] = fJ * t;
+            jpart[(C * NCD + c * nd + d) * kJPad + lane] = fJ * t;
           }
-        // Kt[ac] += fK sum_bd g D[bd]
+            // Kt[ac] += fK sum_bd g D[bd]
 #pragma unroll
         for (int a = 0; a < NA; ++a)
 #pragma unroll
@@ -1207,25 +1304,24 @@ __device__ __forceinline__ void jk_chunk_merged(const EriArgs& g, const JkChunk&
         }
       }
       __syncthreads();  // every slice's part of Jt[cd] is in LDS
-      if (valid && !bk) {
-        // element e of the ket block: wavefront e mod NCH adds the slices' sum
-        for (int e = C; e < NCD; e += NCH) {
-          double t = 0.0;
+      // the group's lanes add the slices' sums
+      add_ket_blocks<NCD>(Jk, srt, i0, nsel, ch.bra, 64 * C + lane, 64 * NCH, [&](int q, int e) {
+        double t = 0.0;
 #pragma unroll
-          for (int w = 0; w < NCH; ++w) t += jpart[(w * NCD + e) * 64 + lane];
-          atomic_add(&Jt[size_t(fc + e / nd) * n + fd + e % nd], t);
-        }
-      }
+        for (int w = 0; w < NCH; ++w) t += jpart[(w * NCD + e) * kJPad + q];
+        return t;
+      });
       __syncthreads();  // jpart is rewritten by the next round
     }
   }
   // Jt[ab] of this slice: one atomic per wavefront and element
+  double* Jb = g.Jl + g.jl0[pair_class(La, Lb)] + (long long)ch.bra * (na * nb);
 #pragma unroll
   for (int a = 0; a < NA; ++a)
 #pragma unroll
     for (int b = 0; b < nb; ++b) {
       const double v = wave_sum(jab[a][b]);
-      if (lane == 0 && v != 0.0) atomic_add(&Jt[size_t(fa + A0 + a) * n + fb + b], v);
+      if (lane == 0 && v != 0.0) atomic_add(&Jb[(A0 + a) * nb + b], v);
     }
   if (lds) {
     __syncthreads();
@@ -1240,8 +1336,8 @@ __device__ __forceinline__ void jk_chunk_merged(const EriArgs& g, const JkChunk&
   }
 }
 
-template <int La, int Lb, int Lc, int Ld, bool MIXED, int CHA, int C, bool LB = false>
-__device__ __forceinline__ void dispatch_merged(const EriArgs& g, const JkChunk& ch, double* krow, SortLds& srt,
+template <int La, int Lb, int Lc, int Ld, bool MIXED, int CHA, int C, bool LB = false, typename S>
+__device__ __forceinline__ void dispatch_merged(const EriArgs& g, const JkChunk& ch, double* krow, S& srt,
                                                 double* jpart, int w, lds_cdptr lrows = nullptr) {
   constexpr int na = ncart(La);
   if (w == C) {
@@ -1253,7 +1349,7 @@ __device__ __forceinline__ void dispatch_merged(const EriArgs& g, const JkChunk&
 
 // Kernel A, merged slices: rep groups of NCH wavefronts per chunk, wavefront
 // w = slice w mod NCH of group w / NCH.  Dynamic LDS: with LB the class's Rys
-// tables, then the groups' ket Coulomb parts [rep][NCH][nc*nd][64], then the
+// tables, then the groups' ket Coulomb parts [rep][NCH][nc*nd][kJPad], then the
 // exchange rows [na + nb][mn]; static: the sort.
 template <int La, int Lb, int Lc, int Ld, bool MIXED, int CHA, bool LB = false>
 __global__ __launch_bounds__(512) void jk_kernel_merged(EriArgs g) {
@@ -1261,17 +1357,17 @@ __global__ __launch_bounds__(512) void jk_kernel_merged(EriArgs g) {
   constexpr int NB = LB ? kLdsRysDoubles<La, Lb, Lc, Ld> : 0;
   static_assert(!LB || NB > 0, "LDS Rys tables are for one- to four-root classes");
   extern __shared__ double dyn[];
-  __shared__ SortLds srt;
+  __shared__ SortLds<false> srt;
   lds_cdptr lrows = nullptr;
   if constexpr (LB) {
     copy_rys_lds<(La + Lb + Lc + Ld) / 2 + 1>(g.rys, dyn);
     lrows = (lds_cdptr)(dyn);
   }
   double* jpart = dyn + NB;
-  double* krow = jpart + (blockDim.x / 64) * (ncart(Lc) * ncart(Ld) * 64);
+  double* krow = jpart + (blockDim.x / 64) * (ncart(Lc) * ncart(Ld) * kJPad);
   const int w = (threadIdx.x >> 6) % NCH;  // uniform over the wavefront
   for (int c = blockIdx.x; c < g.nchunks; c += gridDim.x) {
-    const JkChunk ch = g.chunks[c];
+    const JkChunk ch = load_chunk_uniform(g.chunks, c);
     dispatch_merged<La, Lb, Lc, Ld, MIXED, CHA, 0, LB>(g, ch, krow, srt, jpart, w, lrows);
   }
 }
@@ -1424,18 +1520,19 @@ __global__ __launch_bounds__(NT, (lds_kernel_wpe<La, Lb, Lc, Ld, NT>())) void jk
   }
 
   for (int ci = blockIdx.x; ci < g.nchunks; ci += gridDim.x) {
-    const JkChunk ch = g.chunks[ci];
+    const JkChunk ch = load_chunk_uniform(g.chunks, ci);
     const PairRec bra = load_pair_uniform(g.pairs, ch.bra);
     const int n = bra.mn;
     const double* __restrict__ D = g.D + bra.moff;
-    double* Jt = g.Jt + bra.moff;
+    double* Jk = g.Jl + g.jl0[pair_class(Lc, Ld)];
+    double* Jb = g.Jl + g.jl0[pair_class(La, Lb)] + (long long)ch.bra * (na * nb);
     double* Kt = g.Kt + bra.moff;
     const int fa = bra.fa, fb = bra.fb;
     const bool ij = bra.same;
     const JkSegs* sg = g.segs + ch.seg;
     int seg = 0;
     for (int k = ch.k0; k < ch.k1; ++k) {
-      const int kp = chunk_ket(g.kets, sg, k, seg);
+      const int kp = chunk_ket(sg, k, seg);
       const PairRec ket = load_pair_uniform(g.pairs, kp);
       const int mode = quartet_select(g.sel, ch.bra, bra, kp, ket);
       if (mode == 0) continue;  // uniform over the workgroup
@@ -1528,13 +1625,15 @@ __global__ __launch_bounds__(NT, (lds_kernel_wpe<La, Lb, Lc, Ld, NT>())) void jk
         if (x == 0.0) continue;
         blk[e] = 0.0;
         size_t r, q;
-        double* M = Kt;
-        if (e < OAC) { r = fc + (e - OCD) / nd; q = fd + (e - OCD) % nd; M = Jt; }
-        else if (e < OAD) { r = fa + (e - OAC) / nc; q = fc + (e - OAC) % nc; }
+        if (e < OAC) {
+          atomic_add(&Jk[(long long)kp * (nc * nd) + (e - OCD)], x);
+          continue;
+        }
+        if (e < OAD) { r = fa + (e - OAC) / nc; q = fc + (e - OAC) % nc; }
         else if (e < OBC) { r = fa + (e - OAD) / nd; q = fd + (e - OAD) % nd; }
         else if (e < OBD) { r = fb + (e - OBC) / nc; q = fc + (e - OBC) % nc; }
         else { r = fb + (e - OBD) / nd; q = fd + (e - OBD) % nd; }
-        atomic_add(&M[r * n + q], x);
+        atomic_add(&Kt[r * n + q], x);
       }
       __syncthreads();
     }
@@ -1543,7 +1642,7 @@ __global__ __launch_bounds__(NT, (lds_kernel_wpe<La, Lb, Lc, Ld, NT>())) void jk
       const double x = blk[e];
       if (x == 0.0) continue;
       blk[e] = 0.0;
-      atomic_add(&Jt[size_t(fa + e / nb) * n + fb + e % nb], x);
+      atomic_add(&Jb[e], x);
     }
     __syncthreads();
   }
@@ -1753,18 +1852,19 @@ __global__ __launch_bounds__(64 * NW, (WaveLds<La, Lb, Lc, Ld, NW>::WPE)) void j
   }
 
   for (int ci = blockIdx.x; ci < g.nchunks; ci += gridDim.x) {
-    const JkChunk ch = g.chunks[ci];
+    const JkChunk ch = load_chunk_uniform(g.chunks, ci);
     const PairRec bra = load_pair_uniform(g.pairs, ch.bra);
     const int n = bra.mn;
     const double* __restrict__ D = g.D + bra.moff;
-    double* Jt = g.Jt + bra.moff;
+    double* Jk = g.Jl + g.jl0[pair_class(Lc, Ld)];
+    double* Jb = g.Jl + g.jl0[pair_class(La, Lb)] + (long long)ch.bra * (na * nb);
     double* Kt = g.Kt + bra.moff;
     const int fa = bra.fa, fb = bra.fb;
     const bool ij = bra.same;
     const JkSegs* sg = g.segs + ch.seg;
     int seg = 0;
     for (int k = ch.k0 + wave; k < ch.k1; k += NW) {  // uniform over the wavefront
-      const int kp = chunk_ket(g.kets, sg, k, seg);
+      const int kp = chunk_ket(sg, k, seg);
       const PairRec ket = load_pair_uniform(g.pairs, kp);
       const int mode = quartet_select(g.sel, ch.bra, bra, kp, ket);
       if (mode == 0) continue;
@@ -1826,13 +1926,15 @@ __global__ __launch_bounds__(64 * NW, (WaveLds<La, Lb, Lc, Ld, NW>::WPE)) void j
         if (x == 0.0) continue;
         bw[o] = 0.0;
         size_t r, q;
-        double* M = Kt;
-        if (o < OAC) { r = fc + (o - OCD) / nd; q = fd + (o - OCD) % nd; M = Jt; }
-        else if (o < OAD) { r = fa + (o - OAC) / nc; q = fc + (o - OAC) % nc; }
+        if (o < OAC) {
+          atomic_add(&Jk[(long long)kp * (nc * nd) + (o - OCD)], x);
+          continue;
+        }
+        if (o < OAD) { r = fa + (o - OAC) / nc; q = fc + (o - OAC) % nc; }
         else if (o < OBC) { r = fa + (o - OAD) / nd; q = fd + (o - OAD) % nd; }
         else if (o < OBD) { r = fb + (o - OBC) / nc; q = fc + (o - OBC) % nc; }
         else { r = fb + (o - OBD) / nd; q = fd + (o - OBD) % nd; }
-        atomic_add(&M[r * n + q], x);
+        atomic_add(&Kt[r * n + q], x);
       }
       wave_sync();  // the blocks are clear for the wave's next quartet
     }
@@ -1841,7 +1943,7 @@ __global__ __launch_bounds__(64 * NW, (WaveLds<La, Lb, Lc, Ld, NW>::WPE)) void j
       const double x = bw[o];
       if (x == 0.0) continue;
       bw[o] = 0.0;
-      atomic_add(&Jt[size_t(fa + o / nb) * n + fb + o % nb], x);
+      atomic_add(&Jb[o], x);
     }
     wave_sync();
   }

@@ -20,7 +20,7 @@
 namespace lai {
 
 struct GradArgs {
-  const PairRec* __restrict__ pairs;
+  const PairRec* __restrict__ pairs;  // in list order
   const PrimPair* __restrict__ pp;
   const double2* __restrict__ ppab;  // exponents (alpha_a, alpha_b) of each primitive pair
   const double* __restrict__ rys;
@@ -35,7 +35,6 @@ struct GradArgs {
   const JkChunk* __restrict__ chunks;
   int nchunks;
   const JkSegs* __restrict__ segs;
-  const int* __restrict__ kets;
   QuartetSel sel;
   const double* __restrict__ ppih;  // 1 / (2 zeta) of each primitive pair
 };
@@ -106,7 +105,7 @@ __global__ __launch_bounds__(NT) void grad_kernel(GradArgs g) {
    const int kb = ch.k0 + int((long long)len * blockIdx.y / gridDim.y);
    const int ke = ch.k0 + int((long long)len * (blockIdx.y + 1) / gridDim.y);
    for (int kq = kb; kq < ke; ++kq) {
-    const int kp = chunk_ket(g.kets, sg, kq, seg);
+    const int kp = chunk_ket(sg, kq, seg);
     const PairRec ket = g.pairs[kp];
     if (quartet_select(g.sel, ch.bra, bra, kp, ket) == 0) continue;  // uniform over the workgroup
     const bool ij = bra.same, kl = ket.same, bk = (kp == ch.bra);
@@ -359,7 +358,7 @@ __device__ __forceinline__ void grad_quartet_regs(const GradArgs& g, const PairR
 template <int La, int Lb, int Lc, int Ld>
 __global__ __launch_bounds__(256) void grad_kernel_regs(GradArgs g) {
   extern __shared__ double gacc[];
-  __shared__ SortLds srt;  // lane schedule of the chunk (sort_run)
+  __shared__ SortLds<false> srt;  // lane schedule of the chunk (sort_run)
   const int tid = threadIdx.x;
   const bool glds = g.glds != 0;
   if (glds) {
@@ -379,11 +378,11 @@ __global__ __launch_bounds__(256) void grad_kernel_regs(GradArgs g) {
     double fab[6] = {0, 0, 0, 0, 0, 0};
     const JkSegs* sg = g.segs + ch.seg;
     for (int s0 = ch.k0; s0 < ch.k1; s0 += kSortRun) {
-    const int nsel = sort_run<256>(g.kets, sg, g.pairs, g.sel, ch.bra, bra, s0, min(ch.k1, s0 + kSortRun), srt, 256);
+    const int nsel = sort_run<256>(sg, g.pairs, g.sel, ch.bra, bra, s0, min(ch.k1, s0 + kSortRun), srt, 256);
     for (int r = 0; 256 * r < nsel; ++r) {
-      const int i = sorted_pos(tid, r, 4);
+      const int i = sorted_block(tid, r, 4) + (tid & 63);
       if (i >= nsel) continue;
-      const int kp = int(srt.kp[i] & ~kSortF32);
+      const int kp = int(srt.get(i) & ~kSortF32);
       const PairRec ket = g.pairs[kp];
       double f[9];
       grad_quartet_regs<La, Lb, Lc, Ld>(g, bra, ket, kp == ch.bra, f);

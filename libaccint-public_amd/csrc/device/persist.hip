@@ -32,22 +32,23 @@ struct PersistClass {
   // (classes whose slices take the larger register budget keep their own
   // launches: their footprint would set the one kernel's)
   static constexpr bool covered = P::regs && P::CHA == P::CHA0 && (P::NCH == 1 || P::NCH == 2 || P::NCH == 4);
-  // dynamic LDS in doubles: the merged slices' ket Coulomb parts, then the
-  // exchange rows (na + nb rows of nbf)
-  static constexpr int jpart = P::NCH > 1 ? (kPersistNT / 64) * ncart(Lc) * ncart(Ld) * 64 : 0;
+  // dynamic LDS in doubles: the merged slices' ket Coulomb parts or the
+  // wavefronts' tiles, then the exchange rows (na + nb rows of nbf)
+  static constexpr int jpart =
+      (kPersistNT / 64) * (P::NCH > 1 ? ncart(Lc) * ncart(Ld) * kJPad : kJTile<Lc, Ld>);
   static constexpr int rows = ncart(La) + ncart(Lb);
 };
 
 // Runs chunk ch of class cls (a covered class).
 template <int ID>
 __device__ __forceinline__ void persist_chunk(const EriArgs& g, int cls, const JkChunk& ch, double* dyn,
-                                              SortLds& srt) {
+                                              SortLds<true>& srt) {
   if constexpr (ID < kNumClasses) {
     using C = PersistClass<ID>;
     if constexpr (C::covered) {
       if (cls == ID) {
         if constexpr (C::P::NCH == 1) {
-          jk_chunk_regs<C::La, C::Lb, C::Lc, C::Ld, false, 0, ncart(C::La)>(g, ch, dyn, srt);
+          jk_chunk_regs<C::La, C::Lb, C::Lc, C::Ld, false, 0, ncart(C::La)>(g, ch, dyn + C::jpart, srt, dyn);
         } else {
           dispatch_merged<C::La, C::Lb, C::Lc, C::Ld, false, C::P::CHA, 0>(g, ch, dyn + C::jpart, srt, dyn,
                                                                          (threadIdx.x >> 6) % C::P::NCH);
@@ -64,7 +65,7 @@ __device__ __forceinline__ void persist_chunk(const EriArgs& g, int cls, const J
 __global__ __launch_bounds__(kPersistNT) void jk_kernel_persistent(EriArgs g, const PersistItem* __restrict__ items,
                                                                    int n_items, int* __restrict__ counter) {
   extern __shared__ double dyn[];
-  __shared__ SortLds srt;
+  __shared__ SortLds<true> srt;
   __shared__ int next;
   for (;;) {
     if (threadIdx.x == 0) next = atomicAdd(counter, 1);

@@ -1,4 +1,4 @@
-// wl_kernels.hip -- worklist statistics and batched symmetrisation.
+// wl_kernels.hip -- worklist order, statistics and the last step of a J/K build.
 #include "wl_kernels.hpp"
 
 namespace lai {
@@ -27,15 +27,21 @@ __global__ __launch_bounds__(256) void worklist_stats_kernel(WlStatsArgs a) {
     const JkSegs* sg = a.segs + ch.seg;
     int seg = 0;
     for (int k = ch.k0 + tid; k < ch.k1; k += blockDim.x) {
-      const int kp = chunk_ket(a.kets, sg, k, seg);
+      const int kp = chunk_ket(sg, k, seg);
       const PairRec ket = a.pairs[kp];
       const int mode = quartet_select(a.sel, ch.bra, bra, kp, ket);
       if (mode == 0) continue;
-      // reference orientation: the pair with the smaller index first, each
-      // pair's shells in index order
-      const PairRec& p0 = ch.bra <= kp ? bra : ket;
-      const PairRec& p1 = ch.bra <= kp ? ket : bra;
-      const int i = min(p0.sa, p0.sb), j = max(p0.sa, p0.sb), kk = min(p1.sa, p1.sb), l = max(p1.sa, p1.sb);
+      // reference orientation: each pair's shells in index order, and the pair
+      // whose shells come first (in that order) first
+      int i = min(bra.sa, bra.sb), j = max(bra.sa, bra.sb), kk = min(ket.sa, ket.sb), l = max(ket.sa, ket.sb);
+      if (kk < i || (kk == i && l < j)) {
+        int t = i;
+        i = kk;
+        kk = t;
+        t = j;
+        j = l;
+        l = t;
+      }
       const unsigned long long key =
           ((unsigned long long)(unsigned short)a.sel.sh_loc[i] << 48) |
           ((unsigned long long)(unsigned short)a.sel.sh_loc[j] << 32) |
@@ -84,23 +90,47 @@ __global__ __launch_bounds__(256) void worklist_stats_kernel(WlStatsArgs a) {
   }
 }
 
-__global__ void symmetrize_add_batch_kernel(const double* __restrict__ Jt, const double* __restrict__ Kt,
-                                            double* __restrict__ J, double* __restrict__ K,
-                                            const long long* __restrict__ moff, const int* __restrict__ mnbf,
-                                            int anti) {
-  const int m = blockIdx.y;
-  const size_t n = size_t(mnbf[m]), nn = n * n;
-  const size_t o = size_t(moff[m]);
-  for (size_t x = size_t(blockIdx.x) * blockDim.x + threadIdx.x; x < nn; x += size_t(gridDim.x) * blockDim.x) {
-    const size_t i = x / n, j = x - i * n;
-    const size_t t = j * n + i;
-    if (anti) {
-      K[o + x] += 0.5 * (Kt[o + x] - Kt[o + t]);
-    } else {
-      J[o + x] += 0.5 * (Jt[o + x] + Jt[o + t]);
-      K[o + x] += 0.5 * (Kt[o + x] + Kt[o + t]);
-    }
+__global__ void gather_pairs_kernel(const PairRec* __restrict__ pairs, const int* __restrict__ order, int n,
+                                    PairRec* __restrict__ out) {
+  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x) out[p] = pairs[order[p]];
+}
+
+// Element (i, j) of the symmetrised Coulomb matrix from the pair blocks: a
+// pair of two shells holds its block once, a pair of a shell with itself the
+// whole square.
+__device__ __forceinline__ double finish_j(const FinishArgs& a, int m, int i, int j) {
+  const int f0 = a.mfunc[m], s0 = a.mshell[m];
+  const int si = a.fsh[f0 + i], sj = a.fsh[f0 + j];
+  const int ns = a.mshell[m + 1] - s0;
+  const int lo = min(si, sj), hi = max(si, sj);
+  const double* blk = a.Jl + a.jloc[a.mpair[m] + lo * ns - lo * (lo - 1) / 2 + (hi - lo)];
+  const int xi = i - a.func_off[s0 + si], xj = j - a.func_off[s0 + sj];
+  if (si == sj) {
+    const int nf = ncart(a.L[s0 + si]);
+    return 0.5 * (blk[xi * nf + xj] + blk[xj * nf + xi]);
   }
+  // class order: the shell of larger angular momentum first, the earlier one
+  // where they are equal
+  const bool i_first = a.L[s0 + si] != a.L[s0 + sj] ? a.L[s0 + si] > a.L[s0 + sj] : si < sj;
+  return 0.5 * (i_first ? blk[xi * ncart(a.L[s0 + sj]) + xj] : blk[xj * ncart(a.L[s0 + si]) + xi]);
+}
+
+// Bound by the transposed reads of Kt and the gathered pair blocks (1010
+// functions: 8 MB each, a few tens of microseconds of a 50 ms build).
+__global__ void finish_jk_kernel(FinishArgs a, int anti) {
+  const int m = blockIdx.y;
+  const int n = a.mnbf[m];
+  const size_t o = size_t(a.moff[m]);
+  for (int i = blockIdx.x; i < n; i += gridDim.x)
+    for (int j = threadIdx.x; j < n; j += blockDim.x) {
+      const size_t x = o + size_t(i) * n + j, t = o + size_t(j) * n + i;
+      if (anti) {
+        a.K[x] += 0.5 * (a.Kt[x] - a.Kt[t]);
+      } else {
+        a.J[x] += finish_j(a, m, i, j);
+        a.K[x] += 0.5 * (a.Kt[x] + a.Kt[t]);
+      }
+    }
 }
 
 }  // namespace lai

@@ -1,7 +1,8 @@
-// wl_kernels.hpp -- device passes over the implicit worklist: per-class
+// wl_kernels.hpp -- device passes over the implicit worklist: the pair records
+// in list order, per-class
 // statistics (quartet and ERI counts, the order-independent list checksum,
 // the FLOP model of the reference recursion) with the same per-quartet
-// selection the J/K kernels apply, and the batched J/K symmetrisation.
+// selection the J/K kernels apply, and the J/K matrices from the accumulators.
 #pragma once
 
 #include "eri_kernels.hpp"
@@ -12,8 +13,7 @@ struct WlStatsArgs {
   const JkChunk* __restrict__ chunks;
   int nchunks;
   const JkSegs* __restrict__ segs;
-  const int* __restrict__ kets;
-  const PairRec* __restrict__ pairs;
+  const PairRec* __restrict__ pairs;  // in list order
   QuartetSel sel;
   const int* __restrict__ L;      // angular momentum per shell
   const double* __restrict__ fp;  // F_prim[La][Lb][Lc][Ld], 4^4 entries, reference orientation
@@ -32,12 +32,30 @@ struct WlStatsArgs {
 
 __global__ void worklist_stats_kernel(WlStatsArgs a);
 
-// J[m] += (Jt[m] + Jt[m]^T)/2, K[m] likewise, for every molecule block m
-// (blockIdx.y = molecule); with anti != 0 (an antisymmetric density) only
-// K[m] += (Kt[m] - Kt[m]^T)/2
-__global__ void symmetrize_add_batch_kernel(const double* __restrict__ Jt, const double* __restrict__ Kt,
-                                            double* __restrict__ J, double* __restrict__ K,
-                                            const long long* __restrict__ moff, const int* __restrict__ mnbf,
-                                            int anti);
+// out[p] = pairs[order[p]]: the pair records in list order
+__global__ void gather_pairs_kernel(const PairRec* __restrict__ pairs, const int* __restrict__ order, int n,
+                                    PairRec* __restrict__ out);
+
+// Where the functions of a handle lie, for finish_jk_kernel.
+struct FinishArgs {
+  const double* __restrict__ Jl;       // Coulomb blocks of the pairs in list order
+  const long long* __restrict__ jloc;  // per pair (reference order): its block in Jl
+  const double* __restrict__ Kt;
+  double* __restrict__ J;
+  double* __restrict__ K;
+  const long long* __restrict__ moff;  // per molecule: its matrices
+  const int* __restrict__ mnbf;
+  const int* __restrict__ mpair;       // per molecule: first pair, first shell, first function
+  const int* __restrict__ mshell;
+  const int* __restrict__ mfunc;
+  const int* __restrict__ fsh;         // per function: its shell within the molecule
+  const int* __restrict__ L;           // per shell
+  const int* __restrict__ func_off;    // per shell: first function within the molecule
+};
+
+// J[m] += (Jt[m] + Jt[m]^T)/2 from the pair blocks, K[m] += (Kt[m] +
+// Kt[m]^T)/2, for every molecule block m (blockIdx.y = molecule); with anti !=
+// 0 (an antisymmetric density) only K[m] += (Kt[m] - Kt[m]^T)/2
+__global__ void finish_jk_kernel(FinishArgs a, int anti);
 
 }  // namespace lai

@@ -1,0 +1,65 @@
+"""The Coulomb accumulators in list order (blocks of the shell pairs in the
+order of the worklist, added whole cache lines at a time) against the oracle,
+at the sizes where the list arithmetic can go wrong: one pair; ket runs just
+below, at and above the 2048 quartets that are sorted at a time; (ss| kets,
+which go through the sort's slots, beside kets of 3 to 10 Coulomb elements,
+which go through the wavefront tiles; runs shortened by the density screen;
+molecules of different sizes in one list.  Bar: 1e-10 relative, the J/K bar of
+test_gpu_parity.py (FP64 sums in another order)."""
+import numpy as np
+import pytest
+
+import oracle
+from libaccint import systems
+import libaccint as lai
+
+pytestmark = pytest.mark.gpu
+TOL = 1e-10
+
+
+def rel(a, b):
+    return float(np.max(np.abs(a - b)) / max(np.max(np.abs(b)), 1e-300))
+
+
+def hydrogens(n):
+    """n H atoms on a jittered cubic grid of 2.2 bohr: n s shells, n (n + 1) / 2
+    (ss| pairs, few of them negligible."""
+    m = int(np.ceil(n ** (1.0 / 3.0) - 1e-9))
+    jit = np.random.default_rng(n).uniform(-0.2, 0.2, (n, 3))
+    grid = [(x, y, z) for x in range(m) for y in range(m) for z in range(m)][:n]
+    return [(1, tuple(2.2 * np.array(g) + j)) for g, j in zip(grid, jit)]
+
+
+def case(name):
+    if name.startswith("h"):
+        return "sto-3g", hydrogens(int(name[1:]))
+    if name == "water_tz":
+        return "cc-pvtz", systems.h2o_sto3g_geometry()
+    return name, systems.water_cluster(2, 8.0, seed=3)
+
+
+@pytest.mark.parametrize("name", ["h1", "h2", "h63", "h64", "h91", "sto-3g", "def2-svp", "water_tz"])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_jk_matches_oracle(name, weighted):
+    print("coulomb lists", name, weighted, flush=True)
+    basis_name, atoms = case(name)
+    basis = lai.basis_set(basis_name, atoms)
+    n = basis.n_basis_functions()
+    D = systems.density(n, max(1, n // 4), 7, 1.0 / np.sqrt(n))
+    J, K = lai.Engine(basis).build_jk(D, lai.JKOptions(schwarz_threshold=1e-12, density_weighted=weighted))
+    Jo, Ko = oracle.Oracle(oracle.RawBasis(basis_name, atoms)).jk_canonical(D)
+    assert rel(J, Jo) < TOL and rel(K, Ko) < TOL
+
+
+def test_batch_of_unequal_molecules():
+    mols = [("sto-3g", hydrogens(64)), ("cc-pvdz", systems.h2o_sto3g_geometry()), ("sto-3g", hydrogens(1)),
+            ("def2-svp", systems.random_molecule(np.random.default_rng(3), 5, 5))]
+    bases = [lai.basis_set(b, a) for b, a in mols]
+    be = lai.BatchEngine(bases)
+    off = be.matrix_offsets()
+    Ds = [systems.density(b.n_basis_functions(), 1, 3 + k, 0.3) for k, b in enumerate(bases)]
+    J, K = be.build_jk(np.concatenate([d.ravel() for d in Ds]), lai.JKOptions(schwarz_threshold=1e-12))
+    for k, (b, a) in enumerate(mols):
+        Jo, Ko = oracle.Oracle(oracle.RawBasis(b, a)).jk_canonical(Ds[k])
+        sl = slice(off[k], off[k + 1])
+        assert rel(J[sl].reshape(Jo.shape), Jo) < TOL and rel(K[sl].reshape(Ko.shape), Ko) < TOL
