@@ -227,6 +227,11 @@ struct ClassList {
   // one entry per (bra, segment list): k0 = 0, k1 = its length; chunks are
   // cut from these
   std::vector<JkChunk> runs;
+  // primitive quartets of the class, the most primitive pairs of a ket, and the
+  // longest chain of primitive quartets a lane should run (0: any), for
+  // ket_split
+  double prims = 0.0;
+  int kmax = 0, chain = 0;
   // chunks of the default rule when the tuned ones differ (the gradient
   // kernels are sized for those)
   DevBuf<JkChunk> gchunks;
@@ -290,6 +295,8 @@ struct lai_basis {
   // worklist
   ClassList cls[kNumClasses];
   DevBuf<JkSegs> segs;
+  std::vector<JkSegs> segs_h;
+  std::vector<long long> lcum;  // significant primitive pairs before each list position
   DevBuf<int> kets;           // pair at each list position
   DevBuf<PairRec> lpairs;     // the pair records in list order
   DevBuf<long long> jloc;     // per pair: its block in the Coulomb accumulators
@@ -1006,14 +1013,57 @@ int default_chunk(int shape, size_t n, int n_cu, int nt = 256) {
   return int(std::clamp<size_t>(q, 1, 32));
 }
 
-// Cuts each run into near-equal chunks of at most cmax quartets.
-std::vector<JkChunk> cut_runs(const std::vector<JkChunk>& runs, int cmax) {
+// Longest chain of primitive quartets a lane of a lane-per-quartet class with
+// n quartets and t primitive quartets should run, 0 where no ket has to be
+// divided for it.  The chip holds 2 waves per SIMD of most of these classes,
+// 512 lanes per CU; a lane should not run longer than half of what an even
+// spread over those lanes gives.  kMinChain: a shorter part's digestion costs
+// more than its primitives.
+constexpr int kMinChain = 16;
+int class_chain(double t, int kmax, int nbmax, int n_cu) {
+  const double even = t / (512.0 * n_cu);
+  const double chain = std::max(double(kMinChain), 0.5 * even);
+  return double(kmax) * nbmax <= chain ? 0 : int(std::min(chain, 1e9));
+}
+
+// Cuts each run into near-equal chunks of at most cmax entries.  An entry is a
+// quartet, or with chain > 0 a part of one (ket_split): a ket of k primitive
+// pairs then counts as 1 + k / per.
+std::vector<JkChunk> cut_runs(const lai_basis* b, const ClassList& cl, int cmax, int chain) {
   std::vector<JkChunk> C;
-  for (const auto& r : runs) {
+  for (const auto& r : cl.runs) {
     const int len = r.k1;
-    const int pieces = (len + cmax - 1) / cmax;
-    const int per = (len + pieces - 1) / pieces;
-    for (int k0 = 0; k0 < len; k0 += per) C.push_back(JkChunk{r.bra, r.seg, k0, std::min(len, k0 + per)});
+    const KetSplit sp = ket_split(chain, cl.kmax, int(b->lcum[r.bra + 1] - b->lcum[r.bra]));
+    if (sp.per >= cl.kmax) {
+      const int pieces = (len + cmax - 1) / cmax;
+      const int per = (len + pieces - 1) / pieces;
+      for (int k0 = 0; k0 < len; k0 += per) C.push_back(JkChunk{r.bra, r.seg, k0, std::min(len, k0 + per)});
+      continue;
+    }
+    // entries before position k of the run
+    const JkSegs& sg = b->segs_h[r.seg];
+    auto before = [&](int k) {
+      double x = 0.0;
+      for (int s = 0; s < sg.n && sg.cum[s] < k; ++s) {
+        const int m = std::min(k, sg.cum[s + 1]) - sg.cum[s];
+        x += m + double(b->lcum[sg.start[s] + m] - b->lcum[sg.start[s]]) / sp.per;
+      }
+      return x;
+    };
+    const double tot = before(len);
+    const int pieces = std::min(len, int(tot / cmax) + 1);
+    int k0 = 0;
+    for (int q = 1; q <= pieces && k0 < len; ++q) {
+      int lo = k0 + 1, hi = len;  // first k with before(k) >= q/pieces of all
+      while (lo < hi) {
+        const int mid = (lo + hi) / 2;
+        if (before(mid) >= tot * q / pieces) hi = mid;
+        else lo = mid + 1;
+      }
+      if (q == pieces) lo = len;
+      C.push_back(JkChunk{r.bra, r.seg, k0, lo});
+      k0 = lo;
+    }
   }
   return C;
 }
@@ -1032,17 +1082,24 @@ bool class_split(const lai_basis* b, int c, bool mixed) {
   return mixed && class_shape(launchers().info[c], b->tune[c]) != kShapeRegs;
 }
 
+// The default chunk cap of class c for `shape`, in entries.
+int default_cap(const lai_basis* b, int c, int shape, int nt) {
+  const ClassList& C = b->cls[c];
+  size_t n = 0;
+  for (const auto& r : C.runs) n += size_t(r.k1);
+  if (shape == kShapeRegs && C.chain > 0) n += size_t(C.prims / C.chain);
+  return default_chunk(shape, n, b->ctx->n_cu, nt);
+}
+
 // Chunks of class c under its launch choice (and, when that is not the
 // default, the default chunks for the gradient kernels) on the device.
 int upload_chunks(lai_basis* b, int c) {
   const auto& Ls = launchers();
   ClassList& C = b->cls[c];
-  size_t n = 0;
-  for (const auto& r : C.runs) n += size_t(r.k1);
   const ClassTune& t = b->tune[c];
-  const int shape = class_shape(Ls.info[c], t);
-  const int cmax = t.chunk > 0 ? t.chunk : default_chunk(shape, n, b->ctx->n_cu, Ls.info[c].nt);
-  const std::vector<JkChunk> ch = cut_runs(C.runs, cmax);
+  const int shape = class_shape(Ls.info[c], t), nt = Ls.info[c].nt;
+  const int cmax = t.chunk > 0 ? t.chunk : default_cap(b, c, shape, nt);
+  const std::vector<JkChunk> ch = cut_runs(b, C, cmax, shape == kShapeRegs ? C.chain : 0);
   hipError_t e;
   if ((e = C.chunks.assign(ch.data(), ch.size())) != hipSuccess)
     return fail(LAI_ERR_MEMORY, std::string("chunk upload: ") + hipGetErrorString(e));
@@ -1050,7 +1107,9 @@ int upload_chunks(lai_basis* b, int c) {
   C.gchunks.release();
   C.ngchunks = 0;
   if (!t.is_default()) {
-    const std::vector<JkChunk> g = cut_runs(C.runs, default_chunk(Ls.info[c].shape, n, b->ctx->n_cu, Ls.info[c].nt));
+    const int dshape = Ls.info[c].shape;
+    const std::vector<JkChunk> g =
+        cut_runs(b, C, default_cap(b, c, dshape, nt), dshape == kShapeRegs ? C.chain : 0);
     if ((e = C.gchunks.assign(g.data(), g.size())) != hipSuccess)
       return fail(LAI_ERR_MEMORY, std::string("chunk upload: ") + hipGetErrorString(e));
     C.ngchunks = int64_t(g.size());
@@ -1104,7 +1163,11 @@ extern "C" int lai_dev_build_worklist(lai_basis* b, double thr, const double* sh
   std::vector<int> kets_h(npairs);
   std::vector<double> Ql(npairs);  // bounds in list order
   for (size_t l = 0; l < nlists; ++l) std::copy(lists[l].begin(), lists[l].end(), kets_h.begin() + loff[l]);
-  for (int k = 0; k < npairs; ++k) Ql[k] = Qp[kets_h[k]];
+  b->lcum.assign(size_t(npairs) + 1, 0);
+  for (int k = 0; k < npairs; ++k) {
+    Ql[k] = Qp[kets_h[k]];
+    b->lcum[k + 1] = b->lcum[k] + b->pairs_h[kets_h[k]].npp_sig;
+  }
   std::vector<long long> jloc(npairs);
   long long jtot = 0;
   for (int pc = 0; pc < NPC; ++pc) {
@@ -1174,14 +1237,28 @@ extern "C" int lai_dev_build_worklist(lai_basis* b, double thr, const double* sh
   }, 1);
 
   // Chunks: one run per (bra, segment list), cut by the class's chunk rule
-  std::vector<JkSegs> segs_h;
+  std::vector<JkSegs>& segs_h = b->segs_h;
+  segs_h.clear();
   for (int c = 0; c < kNumClasses; ++c) {
-    auto& R = b->cls[c].runs;
-    R.clear();
+    ClassList& C = b->cls[c];
+    C.runs.clear();
+    C.prims = 0.0;
+    int nbmax = 0;
     for (const auto& e : E[c]) {
-      R.push_back(JkChunk{e.bra, int(segs_h.size()), 0, e.sg.cum[e.sg.n]});
+      C.runs.push_back(JkChunk{e.bra, int(segs_h.size()), 0, e.sg.cum[e.sg.n]});
       segs_h.push_back(e.sg);
+      const int nb = int(b->lcum[e.bra + 1] - b->lcum[e.bra]);
+      nbmax = std::max(nbmax, nb);
+      for (int s = 0; s < e.sg.n; ++s) {
+        const int m = e.sg.cum[s + 1] - e.sg.cum[s];
+        C.prims += double(nb) * double(b->lcum[e.sg.start[s] + m] - b->lcum[e.sg.start[s]]);
+      }
     }
+    C.kmax = 0;
+    const int pk = cls_ket(c);
+    for (int k = loff[list_of(0, pk, 0)]; k < loff[list_of(0, pk, 0) + size_t(nm) * NB]; ++k)
+      C.kmax = std::max(C.kmax, int(b->lcum[k + 1] - b->lcum[k]));
+    C.chain = class_chain(C.prims, C.kmax, nbmax, b->ctx->n_cu);
     std::vector<Entry>().swap(E[c]);
   }
   // shell-pair max|D| per molecule (density screen, FP32 split)
@@ -1327,7 +1404,8 @@ static int build_persist_queue(lai_basis* b) {
     if (!persist_covers(c) || C.runs.empty()) continue;
     size_t n = 0;
     for (const auto& r : C.runs) n += size_t(r.k1);
-    for (const JkChunk& ch : cut_runs(C.runs, default_chunk(kShapeRegs, n, b->ctx->n_cu, Ls.info[c].nt)))
+    // (undivided kets: one kernel runs every covered class)
+    for (const JkChunk& ch : cut_runs(b, C, default_chunk(kShapeRegs, n, b->ctx->n_cu, Ls.info[c].nt), 0))
       items.push_back(PersistItem{c, ch});
   }
   hipError_t e;
@@ -1398,6 +1476,8 @@ static int launch_jk_classes(lai_basis* b, EriArgs a, int flags, hipStream_t st,
         }
         a.chunks = C.chunks.p;
         a.nchunks = int(C.nchunks);
+        a.chain = C.chain;
+        a.kmax = C.kmax;
         a.sel.keep = split ? part + 1 : 0;
         LaunchTune t;
         t.alt = b->tune[c].alt;
@@ -1672,6 +1752,8 @@ extern "C" int lai_dev_jk_grad(lai_basis* b, const double* d_D, double xscale, d
     const ClassList& C = b->cls[c];
     if (C.nchunks <= 0) continue;
     const bool own = C.ngchunks > 0;  // the J/K chunks are tuned: default ones
+    a.chain = C.chain;
+    a.kmax = C.kmax;
     a.chunks = own ? C.gchunks.p : C.chunks.p;
     a.nchunks = int(own ? C.ngchunks : C.nchunks);
     int k = 0;
@@ -1805,6 +1887,8 @@ extern "C" int lai_dev_autotune(lai_basis* b, const double* d_D, int flags, int 
     const ClassList& C = b->cls[c];
     a.chunks = C.chunks.p;
     a.nchunks = int(C.nchunks);
+    a.chain = C.chain;
+    a.kmax = C.kmax;
     LaunchTune t;
     t.alt = b->tune[c].alt;
     t.blocks_per_cu = b->tune[c].bpc;
@@ -1856,7 +1940,7 @@ extern "C" int lai_dev_autotune(lai_basis* b, const double* d_D, int flags, int 
     failed_saved = saved;
     if ((rc = eval(best, dflt_ms)) != LAI_OK) break;
     best_ms = dflt_ms;
-    tried.emplace_back(info.shape, default_chunk(info.shape, nq, n_cu, info.nt));
+    tried.emplace_back(info.shape, default_cap(b, c, info.shape, info.nt));
     for (int alt = 0; alt <= (info.alt != kShapeNone ? 1 : 0) && rc == LAI_OK; ++alt) {
       const int shape = alt ? info.alt : info.shape;
       std::vector<int> caps;
@@ -1867,7 +1951,7 @@ extern "C" int lai_dev_autotune(lai_basis* b, const double* d_D, int flags, int 
       else caps = {4, 8, 16, 32};
       if (alt) caps.insert(caps.begin(), 0);
       for (int cap_q : caps) {
-        const int eff = cap_q > 0 ? cap_q : default_chunk(shape, nq, n_cu, shape == info.shape ? info.nt : 256);
+        const int eff = cap_q > 0 ? cap_q : default_cap(b, c, shape, shape == info.shape ? info.nt : 256);
         if (std::find(tried.begin(), tried.end(), std::make_pair(shape, eff)) != tried.end()) continue;
         tried.emplace_back(shape, eff);
         ClassTune t{};

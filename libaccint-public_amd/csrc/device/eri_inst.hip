@@ -114,7 +114,7 @@ void launch_class(const EriArgs& a0, hipStream_t s, const LaunchTune& t) {
       auto kern = jk_kernel_merged<La, Lb, Lc, Ld, MIXED, P::CHA, false>;
       static const size_t stat = static_lds(kern);
       static const size_t dmax = dyn_limit(kern, stat);
-      const size_t per_rep = size_t(P::NCH) * nc * nd * kJPad * sizeof(double);
+      const size_t per_rep = size_t(kJPart<P::NCH, nc * nd>) * sizeof(double);
       const size_t rows = size_t(na + nb) * nbf * sizeof(double);
       RowsPick rp = pick_rows(kern, dmax, 64 * P::NCH, per_rep, rows);
       // the Rys tables in LDS as well (one to four roots) when that keeps as

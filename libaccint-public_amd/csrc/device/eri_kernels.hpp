@@ -84,11 +84,17 @@ __device__ __forceinline__ int quartet_select(const QuartetSel& s, int bp, const
   return (s.keep == 0 || s.keep == mode) ? mode : 0;
 }
 
-// List position of the ket at position k of a chunk's run; seg walks forward
-// with k.
-__device__ __forceinline__ int chunk_ket(const JkSegs* __restrict__ sg, int k, int& seg) {
-  while (seg + 1 < sg->n && k >= sg->cum[seg + 1]) ++seg;
-  return sg->start[seg] + (k - sg->cum[seg]);
+// List position of the ket at position k of a chunk's run (the segments are
+// read with scalar loads: the chunk is uniform over the workgroup).
+__device__ __forceinline__ int chunk_ket(const JkSegs* sg0, int k) {
+  const __attribute__((address_space(4))) JkSegs* sg = (const __attribute__((address_space(4))) JkSegs*)sg0;
+  const int n = sg->n;
+  int d = sg->start[0];
+  for (int s = 1; s < n; ++s) {
+    const int c = sg->cum[s];
+    d = k >= c ? sg->start[s] - c : d;
+  }
+  return k + d;
 }
 
 // Lane schedule of the lane-per-quartet kernels.  The quartets of a chunk
@@ -96,69 +102,85 @@ __device__ __forceinline__ int chunk_ket(const JkSegs* __restrict__ sg, int k, i
 // flag, primitive pairs of the ket), heaviest first, so that the 64 lanes of a
 // wavefront run primitive loops of nearly equal length and one precision;
 // quartets removed by the density screen take no lane.
-constexpr int kSortRun = 2048;                 // quartets sorted at a time
-constexpr int kSortBins = 256;                 // key: 128 * FP32 + min(npp_sig, 127)
-constexpr unsigned kSortF32 = 0x80000000u;     // flag bit of a sorted entry
+//
+// Where a class has few quartets, a quartet's ket primitive pairs are divided
+// over several lanes (KetSplit): each lane digests the part of the integrals
+// that its primitives give, J and K being linear in them.  Without that, one
+// lane runs the whole primitive loop of the most contracted quartet while the
+// chip idles: (ss|ss) of three waters in cc-pVDZ took 1.66 ms for 26 539
+// quartets, the time of one chain of 64 x 64 primitive quartets (now 0.04 ms).
+// Class kernels one after another, before and after: three waters 8.1 -> 1.6
+// ms, a nine-atom molecule in cc-pVTZ 32.6 -> 20.4, seven molecules of 3-13
+// atoms 81 -> 63; classes with quartets enough are not divided (class_chain).
+constexpr int kSortRun = 2048;  // entries sorted at a time
+constexpr int kSortBins = 256;  // key: 128 * FP32 + min(primitive pairs of the entry, 127)
+constexpr int kMaxParts = 127;  // lanes a quartet may be divided over
+
+// A sorted entry: position in the run (11 bits) and part of the ket.
+__device__ __forceinline__ int entry_pos(unsigned e) { return int(e & (kSortRun - 1)); }
+__device__ __forceinline__ int entry_part(unsigned e) { return int(e / kSortRun); }
+
+// Ket primitive pairs per lane for one bra, and how many quartets are sorted
+// at a time so that their entries fit: a lane's chain of primitive quartets is
+// at most about `chain` long (0: no division).  kmax: the most primitive pairs
+// of any ket.
+struct KetSplit {
+  int per, run;
+};
+__host__ __device__ __forceinline__ KetSplit ket_split(int chain, int kmax, int npp_bra) {
+  if (chain == 0) return KetSplit{1 << 24, kSortRun};
+  const int nb = max(npp_bra, 1);
+  const int per = max((chain + nb - 1) / nb, (kmax + kMaxParts - 1) / kMaxParts);
+  const int parts = (kmax + per - 1) / per;
+  return KetSplit{per, parts > 1 ? kSortRun / parts : kSortRun};
+}
+
+// The same in SGPRs (the bra is uniform over the workgroup).
+__device__ __forceinline__ KetSplit ket_split_uniform(int chain, int kmax, int npp_bra) {
+  const KetSplit s = ket_split(chain, kmax, npp_bra);
+  return KetSplit{__builtin_amdgcn_readfirstlane(s.per), __builtin_amdgcn_readfirstlane(s.run)};
+}
+
 // WIN: for classes whose ket is a pair of s shells (one Coulomb element per
-// quartet) the entry's slot, read once by its lane, then takes the quartet's
-// Coulomb element, and inv (run position -> sorted entry) lets the workgroup
-// add the run's elements to Jl in list order, whole cache lines at a time.
+// quartet) the elements of a run are summed in LDS by run position, and the
+// workgroup adds them to Jl in list order, whole cache lines at a time.
 template <bool WIN>
 struct SortLds {
-  static constexpr bool win = false;
-  unsigned kp[kSortRun];  // list position of the ket, kSortF32 set for the FP32 recursion
+  static constexpr bool win = WIN;
+  unsigned e[kSortRun];
+  double j[WIN ? kSortRun : 1];
   int cnt[kSortBins];
   int n;
-  __device__ __forceinline__ unsigned get(int i) const { return kp[i]; }
-  __device__ __forceinline__ void put(int i, unsigned e, int) { kp[i] = e; }
-  __device__ __forceinline__ void skip(int) {}
-};
-template <>
-struct SortLds<true> {
-  static constexpr bool win = true;
-  static constexpr unsigned short none = 0xffff;  // a quartet that takes no lane
-  union Slot {
-    unsigned kp;
-    double j;
-  };
-  Slot slot[kSortRun];
-  unsigned short inv[kSortRun];
-  int cnt[kSortBins];
-  int n;
-  __device__ __forceinline__ unsigned get(int i) const { return slot[i].kp; }
-  __device__ __forceinline__ void put(int i, unsigned e, int k) {
-    slot[i].kp = e;
-    inv[k] = (unsigned short)i;
-  }
-  __device__ __forceinline__ void skip(int k) { inv[k] = none; }
 };
 
-// Sorts positions [s0, s1) (at most kSortRun) of a chunk's run into s and
-// returns how many were kept.  All nt lanes of the workgroup call it (nt a
-// multiple of 64, at least NTMIN); it ends on a barrier.
+// Sorts positions [s0, s1) (at most sp.run) of a chunk's run into s and
+// returns how many entries there are.  All nt lanes of the workgroup call it
+// (nt a multiple of 64, at least NTMIN); it ends on a barrier.
 template <int NTMIN, typename S>
-__device__ __forceinline__ int sort_run(const JkSegs* __restrict__ sg, const PairRec* __restrict__ pairs,
-                                        const QuartetSel& sel, int bp, const PairRec& bra, int s0, int s1, S& s,
-                                        int nt) {
+__device__ __forceinline__ int sort_run(const JkSegs* sg, const PairRec* __restrict__ pairs, const QuartetSel& sel,
+                                        int bp, const PairRec& bra, const KetSplit& sp, int s0, int s1, S& s, int nt) {
   constexpr int kSortPer = (kSortRun + NTMIN - 1) / NTMIN;  // positions per lane, at most
   const int tid = threadIdx.x;
   for (int i = tid; i < kSortBins; i += nt) s.cnt[i] = 0;
+  if constexpr (S::win)
+    for (int k = tid; k < s1 - s0; k += nt) s.j[k] = 0.0;
   __syncthreads();
-  int kp[kSortPer], key[kSortPer], rk[kSortPer];
-  int seg = 0;
+  int key[kSortPer], rk[kSortPer];  // key: 256 * (parts - 1) + bin, -1 for a quartet that takes no lane
 #pragma unroll
   for (int j = 0; j < kSortPer; ++j) {
     const int k = s0 + tid + nt * j;
     key[j] = -1;
-    kp[j] = 0;
     rk[j] = 0;
     if (k < s1) {
-      kp[j] = chunk_ket(sg, k, seg);
-      const PairRec ket = pairs[kp[j]];
-      const int mode = quartet_select(sel, bp, bra, kp[j], ket);
+      const int kp = chunk_ket(sg, k);
+      const PairRec ket = pairs[kp];
+      const int mode = quartet_select(sel, bp, bra, kp, ket);
       if (mode != 0) {
-        key[j] = (mode == 2 ? 128 : 0) + min(ket.npp_sig, 127);
-        rk[j] = atomicAdd(&s.cnt[key[j]], 1);
+        const int np = ket.npp_sig;
+        const int parts = np > sp.per ? (np + sp.per - 1) / sp.per : 1;
+        const int bin = (mode == 2 ? 128 : 0) + min(min(np, sp.per), 127);
+        key[j] = 256 * (parts - 1) + bin;
+        rk[j] = atomicAdd(&s.cnt[bin], parts);
       }
     }
   }
@@ -186,15 +208,13 @@ __device__ __forceinline__ int sort_run(const JkSegs* __restrict__ sg, const Pai
   }
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < kSortPer; ++j) {
-    const int k = tid + nt * j;
-    if (key[j] >= 0)
-      s.put(s.cnt[key[j]] + rk[j], unsigned(kp[j]) | (key[j] >= 128 ? kSortF32 : 0u), k);
-    else if (s0 + k < s1)
-      s.skip(k);
-  }
+  for (int j = 0; j < kSortPer; ++j)
+    if (key[j] >= 0) {
+      const int at = s.cnt[key[j] & 255] + rk[j], parts = (key[j] >> 8) + 1;
+      for (int p = 0; p < parts; ++p) s.e[at + p] = unsigned(tid + nt * j) + unsigned(p) * kSortRun;
+    }
   __syncthreads();
-  return s.n;
+  return __builtin_amdgcn_readfirstlane(s.n);
 }
 
 // First sorted entry of the 64-entry block that the wavefront of lane tid
@@ -202,7 +222,7 @@ __device__ __forceinline__ int sort_run(const JkSegs* __restrict__ sg, const Pai
 // wavefronts take the nw blocks of a round in an order that rotates with r,
 // so that no wavefront always gets the heaviest block.
 __device__ __forceinline__ int sorted_block(int tid, int r, int nw) {
-  const int w = tid >> 6;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   return 64 * (nw * r + ((w + r) & (nw - 1)));
 }
 
@@ -236,6 +256,7 @@ struct EriArgs {
   int nchunks;
   const JkSegs* __restrict__ segs;
   int klds;  // 1: the bra rows of Kt are accumulated in LDS (dynamic shared memory)
+  int chain, kmax;  // division of the kets' primitives over lanes (ket_split)
   QuartetSel sel;
 };
 
@@ -314,14 +335,14 @@ __device__ __forceinline__ int orig_offset(int perm, const int (&idx)[4], const 
 // --------------------------------------------------------------------------
 // Contracted, normalised block gv[a - A0][b][c][d] of the quartet (bra|ket);
 // all_prims selects every primitive pair (raw ERIs) or only those above the
-// primitive screening bound (J/K).
+// primitive screening bound (J/K), there only the ket's ik0 .. ik0 + per - 1.
 // LB: the Boys Taylor rows (one and two roots) or the Chebyshev coefficients
 // of the rule (three and four roots) from the workgroup's copy in LDS
 // (lrows), else from the device table
 template <int La, int Lb, int Lc, int Ld, typename R, int A0, int A1, bool LB = false>
 __device__ __forceinline__ void quartet_block_regs(
     const EriArgs& g, const PairRec& bra, const PairRec& ket, bool all_prims,
-    double (&gv)[A1 - A0][ncart(Lb)][ncart(Lc)][ncart(Ld)], lds_cdptr lrows = nullptr) {
+    double (&gv)[A1 - A0][ncart(Lb)][ncart(Lc)][ncart(Ld)], lds_cdptr lrows = nullptr, int ik0 = 0, int per = 0) {
   constexpr int nb = ncart(Lb), nc = ncart(Lc), nd = ncart(Ld);
   constexpr int NA = A1 - A0;
   constexpr int NR = (La + Lb + Lc + Ld) / 2 + 1;
@@ -339,7 +360,7 @@ __device__ __forceinline__ void quartet_block_regs(
   const R ABx = R(bra.ABx), ABy = R(bra.ABy), ABz = R(bra.ABz);
   const R CDx = R(ket.ABx), CDy = R(ket.ABy), CDz = R(ket.ABz);
   const int nb_pp = all_prims ? bra.npp : bra.npp_sig;
-  const int nk_pp = all_prims ? ket.npp : ket.npp_sig;
+  const int nk_pp = all_prims ? ket.npp : min(ket.npp_sig, ik0 + per);
   // FP32 part: primitive pairs are sorted by bound, so both loops stop at the
   // first primitive quartet below the relative cut
   constexpr bool fp32 = sizeof(R) == 4;
@@ -348,7 +369,7 @@ __device__ __forceinline__ void quartet_block_regs(
   // ket primitive pairs outside (one load per lane and pair), bra primitive
   // pairs inside: the bra is the same for the whole workgroup in the J/K
   // kernels, so its records are uniform (scalar) loads
-  for (int ik = 0; ik < nk_pp; ++ik) {
+  for (int ik = ik0; ik < nk_pp; ++ik) {
     const float bk = fp32 ? g.ppb[ket.pp_off + ik] : 0.0f;
     if (fp32 && bk * bb0 < qcut) break;
     const PrimPair Q = g.pp[ket.pp_off + ik];
@@ -881,23 +902,24 @@ __global__ __launch_bounds__(NT) void eri_kernel_lds(EriArgs g) {
 // Lanes take the chunk's quartets in the order of sort_run.
 // --------------------------------------------------------------------------
 // Doubles of the ket Coulomb tile of a wavefront (jk_chunk_regs): 64 blocks of
-// nc nd, none for an (ss| ket, whose elements go through the sort's slots.
+// nc nd and the 64 list positions they belong to, none for an (ss| ket, whose
+// elements are summed in SortLds::j.
 template <int Lc, int Ld>
-inline constexpr int kJTile = ncart(Lc) * ncart(Ld) > 1 ? 64 * ncart(Lc) * ncart(Ld) : 0;
+inline constexpr int kJTile = ncart(Lc) * ncart(Ld) > 1 ? 64 * ncart(Lc) * ncart(Ld) + 32 : 0;
 
-// Adds the Coulomb blocks of 64 sorted quartets (entries i0 .. i0 + 63) to
-// Jl: element t of the blocks laid one after another is at(q, e), e of quartet
-// q; lanes l0, l0 + nl, ... take consecutive elements, so that neighbouring
-// lanes add to one ket's contiguous block.  The bra's own pair takes none.
-template <int NCD, typename S, typename F>
-__device__ __forceinline__ void add_ket_blocks(double* __restrict__ Jl, const S& srt, int i0, int nsel, int bra, int l0,
-                                               int nl, F&& at) {
+// Adds the Coulomb blocks of n <= 64 kets at list positions pos[0 .. n) to Jl:
+// element t of the blocks laid one after another is at(q, e), e of ket q; lanes
+// l0, l0 + nl, ... take consecutive elements, so that neighbouring lanes add to
+// one ket's contiguous block.  The bra's own pair takes none.
+template <int NCD, typename F>
+__device__ __forceinline__ void add_ket_blocks(double* __restrict__ Jl, const int* pos, int n, int bra, int l0, int nl,
+                                               F&& at) {
 #pragma unroll
   for (int t = l0; t < 64 * NCD; t += nl) {
     const int q = t / NCD, e = t - q * NCD;
-    if (i0 + q >= nsel) break;
-    const int pos = int(srt.get(i0 + q) & ~kSortF32);
-    if (pos != bra) atomic_add(&Jl[(long long)pos * NCD + e], at(q, e));
+    if (q >= n) break;
+    const int p = pos[q];
+    if (p != bra) atomic_add(&Jl[(long long)p * NCD + e], at(q, e));
   }
 }
 
@@ -918,6 +940,7 @@ __device__ __forceinline__ void jk_chunk_regs(const EriArgs& g, const JkChunk& c
   double* Jk = g.Jl + g.jl0[pair_class(Lc, Ld)];
   double* Kt = g.Kt + bra.moff;
   jtile += (tid >> 6) * kJTile<Lc, Ld>;  // this wavefront's
+  int* jpos = reinterpret_cast<int*>(jtile + 64 * NCD);
   const int fa = bra.fa + A0, fb = bra.fb;
   const bool ij = bra.same;
   const JkSegs* sg = g.segs + ch.seg;
@@ -938,20 +961,22 @@ __device__ __forceinline__ void jk_chunk_regs(const EriArgs& g, const JkChunk& c
 #pragma unroll
     for (int b = 0; b < nb; ++b) jab[a][b] = 0.0;
 
-  for (int s0 = ch.k0; s0 < ch.k1; s0 += kSortRun) {
-  const int s1 = min(ch.k1, s0 + kSortRun);
-  const int nsel = sort_run<256>(sg, g.pairs, g.sel, ch.bra, bra, s0, s1, srt, nt);
+  const KetSplit sp = ket_split_uniform(g.chain, g.kmax, bra.npp_sig);
+  for (int s0 = ch.k0; s0 < ch.k1; s0 += sp.run) {
+  const int s1 = min(ch.k1, s0 + sp.run);
+  const int nsel = sort_run<256>(sg, g.pairs, g.sel, ch.bra, bra, sp, s0, s1, srt, nt);
   for (int r = 0; nt * r < nsel; ++r) {
     const int i0 = sorted_block(tid, r, nt >> 6);  // uniform over the wavefront
     const int i = i0 + (tid & 63);
     if (i < nsel) {
-    const int kp = int(srt.get(i) & ~kSortF32);
+    const unsigned ent = srt.e[i];
+    const int kp = chunk_ket(sg, s0 + entry_pos(ent)), ik0 = entry_part(ent) * sp.per;
     const PairRec ket = g.pairs[kp];
     double gv[NA][nb][nc][nd];
     if constexpr (MIXED)
-      quartet_block_regs<La, Lb, Lc, Ld, float, A0, A1>(g, bra, ket, false, gv);
+      quartet_block_regs<La, Lb, Lc, Ld, float, A0, A1>(g, bra, ket, false, gv, nullptr, ik0, sp.per);
     else
-      quartet_block_regs<La, Lb, Lc, Ld, double, A0, A1, LB>(g, bra, ket, false, gv, lrows);
+      quartet_block_regs<La, Lb, Lc, Ld, double, A0, A1, LB>(g, bra, ket, false, gv, lrows, ik0, sp.per);
     const int fc = ket.fa, fd = ket.fb;
     const bool kl = ket.same, bk = (kp == ch.bra);
     const double fJ = (ij ? 1.0 : 2.0) * (kl ? 1.0 : 2.0);
@@ -978,11 +1003,12 @@ __device__ __forceinline__ void jk_chunk_regs(const EriArgs& g, const JkChunk& c
         for (int a = 0; a < NA; ++a)
 #pragma unroll
           for (int b = 0; b < nb; ++b) s += gv[a][b][c][d] * D[size_t(fa + a) * n + fb + b];
-        if constexpr (WIN)
-          srt.slot[i].j = bk ? 0.0 : fJ * s;
-        else
+        if constexpr (WIN) {
+          if (!bk) lds_add(&srt.j[entry_pos(srt.e[i])], fJ * s);
+        } else
           jtile[(tid & 63) * NCD + c * nd + d] = fJ * s;
       }
+    if constexpr (!WIN) jpos[tid & 63] = kp;
     // Kt[ac] += fK sum_bd g D[bd]
 #pragma unroll
     for (int a = 0; a < NA; ++a)
@@ -1037,22 +1063,19 @@ __device__ __forceinline__ void jk_chunk_regs(const EriArgs& g, const JkChunk& c
     }
     if constexpr (!WIN) {
       wave_sync();  // the wavefront's blocks are in its tile
-      add_ket_blocks<NCD>(Jk, srt, i0, nsel, ch.bra, tid & 63, 64, [&](int q, int e) { return jtile[q * NCD + e]; });
+      add_ket_blocks<NCD>(Jk, jpos, min(nsel - i0, 64), ch.bra, tid & 63, 64,
+                          [&](int q, int e) { return jtile[q * NCD + e]; });
       wave_sync();  // the tile is read before the next round fills it
     }
   }
   if constexpr (WIN) {
-    __syncthreads();  // the run's Coulomb elements are in their slots
-    int seg = 0;
+    __syncthreads();  // the run's Coulomb elements are complete
 #pragma unroll 1
-    for (int k = s0 + tid; k < s1; k += nt) {
-      const unsigned short q = srt.inv[k - s0];
-      const int pos = chunk_ket(sg, k, seg);
-      if (q != S::none) {
-        const double v = srt.slot[q].j;
-        if (v != 0.0) atomic_add(&Jk[pos], v);
-      }
+    for (int k = tid; k < s1 - s0; k += nt) {
+      const double v = srt.j[k];
+      if (v != 0.0) atomic_add(&Jk[chunk_ket(sg, s0 + k)], v);
     }
+    __syncthreads();  // and read before the next run clears them
   }
   }
   // Jt[ab]: one atomic per wavefront and element
@@ -1133,6 +1156,14 @@ __device__ __forceinline__ void copy_rys_lds(const double* __restrict__ rys, dou
   __syncthreads();
 }
 
+// Wavefronts per SIMD that bound the registers of the unsplit kernel, by its
+// outputs per lane: the next step of resident waves where the compiler gets
+// there without scratch ((ps|ps) 144 -> 128 VGPRs with 12 bytes, (pp|ss),
+// (fs|ss) 134-139 -> 127, (ds|ps), (dp|ss) 171 -> 167).
+// Three for 27 and 30 outputs (100-170 bytes of scratch) was no gain: (pp|ps)
+// 1.43 -> 1.34 ms on 16 waters, but 3.56 -> 4.26 ms on C40H82.
+constexpr int regs_wpe(int nout) { return nout <= 10 ? 4 : nout <= 18 ? 3 : 2; }
+
 // (The chunk and its bra record are read through the constant address space,
 // so what depends on them alone sits in SGPRs: (ss|ss) 93 -> 83 VGPRs,
 // (ps|ps) 154 -> 135, scratch of the merged (dd|ps) 316 -> 212 bytes a lane.)
@@ -1142,7 +1173,7 @@ __device__ __forceinline__ void copy_rys_lds(const double* __restrict__ rys, dou
 // Rys tables, copied once per workgroup, then the wavefronts' ket Coulomb
 // tiles, then the exchange rows [CHA + nb][mn].
 template <int La, int Lb, int Lc, int Ld, bool MIXED, int CHA, bool LB>
-__global__ __launch_bounds__(512) void jk_kernel_regs(EriArgs g) {
+__global__ __launch_bounds__(512, (regs_wpe(CHA * ncart(Lb) * ncart(Lc) * ncart(Ld)))) void jk_kernel_regs(EriArgs g) {
   extern __shared__ double dyn[];
   __shared__ SortLds<(Lc + Ld == 0)> srt;
   constexpr int NB = LB ? kLdsRysDoubles<La, Lb, Lc, Ld> : 0;
@@ -1172,6 +1203,9 @@ __global__ __launch_bounds__(512) void jk_kernel_regs(EriArgs g) {
 // (kJPad doubles per element: 64 quartets and one of padding, so that the
 // elements of one quartet lie in different banks.)
 constexpr int kJPad = 65;
+// doubles of a group's parts, with the list positions of its 64 kets
+template <int NCH, int NCD>
+inline constexpr int kJPart = NCH * NCD * kJPad + 32;
 template <int La, int Lb, int Lc, int Ld, bool MIXED, int CHA, int C, bool LB = false, typename S>
 __device__ __forceinline__ void jk_chunk_merged(const EriArgs& g, const JkChunk& ch, double* krow, S& srt,
                                                 double* jpart, lds_cdptr lrows = nullptr) {
@@ -1182,8 +1216,9 @@ __device__ __forceinline__ void jk_chunk_merged(const EriArgs& g, const JkChunk&
   constexpr int NCD = nc * nd;
   constexpr int ROWS = na + nb;
   const int tid = threadIdx.x, lane = tid & 63, NT = blockDim.x;
-  const int rep = NT / (64 * NCH), grp = (tid >> 6) / NCH;
-  jpart += grp * (NCH * NCD * kJPad);  // this group's slices
+  const int rep = NT / (64 * NCH), grp = __builtin_amdgcn_readfirstlane(tid >> 6) / NCH;
+  jpart += grp * kJPart<NCH, NCD>;  // this group's slices
+  int* jpos = reinterpret_cast<int*>(jpart + NCH * NCD * kJPad);
   const bool lds = g.klds != 0;
   const PairRec bra = load_pair_uniform(g.pairs, ch.bra);
   const int n = bra.mn;
@@ -1210,19 +1245,21 @@ __device__ __forceinline__ void jk_chunk_merged(const EriArgs& g, const JkChunk&
 #pragma unroll
     for (int b = 0; b < nb; ++b) jab[a][b] = 0.0;
 
-  for (int s0 = ch.k0; s0 < ch.k1; s0 += kSortRun) {
+  const KetSplit sp = ket_split_uniform(g.chain, g.kmax, bra.npp_sig);
+  for (int s0 = ch.k0; s0 < ch.k1; s0 += sp.run) {
     const int nsel =
-        sort_run<64 * NCH>(sg, g.pairs, g.sel, ch.bra, bra, s0, min(ch.k1, s0 + kSortRun), srt, NT);
+        sort_run<64 * NCH>(sg, g.pairs, g.sel, ch.bra, bra, sp, s0, min(ch.k1, s0 + sp.run), srt, NT);
     for (int r = 0; 64 * rep * r < nsel; ++r) {
       const int i0 = 64 * (rep * r + grp), i = i0 + lane;
       if (i < nsel) {
-        const int kp = int(srt.get(i) & ~kSortF32);
+        const unsigned ent = srt.e[i];
+        const int kp = chunk_ket(sg, s0 + entry_pos(ent)), ik0 = entry_part(ent) * sp.per;
         const PairRec ket = g.pairs[kp];
         double gv[NA][nb][nc][nd];
         if constexpr (MIXED)
-          quartet_block_regs<La, Lb, Lc, Ld, float, A0, A1>(g, bra, ket, false, gv);
+          quartet_block_regs<La, Lb, Lc, Ld, float, A0, A1>(g, bra, ket, false, gv, nullptr, ik0, sp.per);
         else
-          quartet_block_regs<La, Lb, Lc, Ld, double, A0, A1, LB>(g, bra, ket, false, gv, lrows);
+          quartet_block_regs<La, Lb, Lc, Ld, double, A0, A1, LB>(g, bra, ket, false, gv, lrows, ik0, sp.per);
         const int fc = ket.fa, fd = ket.fb;
         const bool kl = ket.same, bk = (kp == ch.bra);
         const double fJ = (ij ? 1.0 : 2.0) * (kl ? 1.0 : 2.0);
@@ -1251,6 +1288,7 @@ __device__ __forceinline__ void jk_chunk_merged(const EriArgs& g, const JkChunk&
               for (int b = 0; b < nb; ++b) t += gv[a][b][c][d] * D[size_t(fa + A0 + a) * n + fb + b];
             jpart[(C * NCD + c * nd + d) * kJPad + lane] = fJ * t;
           }
+        if constexpr (C == 0) jpos[lane] = kp;
             // Kt[ac] += fK sum_bd g D[bd]
 #pragma unroll
         for (int a = 0; a < NA; ++a)
@@ -1305,7 +1343,7 @@ __device__ __forceinline__ void jk_chunk_merged(const EriArgs& g, const JkChunk&
       }
       __syncthreads();  // every slice's part of Jt[cd] is in LDS
       // the group's lanes add the slices' sums
-      add_ket_blocks<NCD>(Jk, srt, i0, nsel, ch.bra, 64 * C + lane, 64 * NCH, [&](int q, int e) {
+      add_ket_blocks<NCD>(Jk, jpos, min(nsel - i0, 64), ch.bra, 64 * C + lane, 64 * NCH, [&](int q, int e) {
         double t = 0.0;
 #pragma unroll
         for (int w = 0; w < NCH; ++w) t += jpart[(w * NCD + e) * kJPad + q];
@@ -1349,8 +1387,8 @@ __device__ __forceinline__ void dispatch_merged(const EriArgs& g, const JkChunk&
 
 // Kernel A, merged slices: rep groups of NCH wavefronts per chunk, wavefront
 // w = slice w mod NCH of group w / NCH.  Dynamic LDS: with LB the class's Rys
-// tables, then the groups' ket Coulomb parts [rep][NCH][nc*nd][kJPad], then the
-// exchange rows [na + nb][mn]; static: the sort.
+// tables, then the groups' ket Coulomb parts [rep][kJPart], then the exchange
+// rows [na + nb][mn]; static: the sort.
 template <int La, int Lb, int Lc, int Ld, bool MIXED, int CHA, bool LB = false>
 __global__ __launch_bounds__(512) void jk_kernel_merged(EriArgs g) {
   constexpr int NCH = (ncart(La) + CHA - 1) / CHA;
@@ -1364,7 +1402,7 @@ __global__ __launch_bounds__(512) void jk_kernel_merged(EriArgs g) {
     lrows = (lds_cdptr)(dyn);
   }
   double* jpart = dyn + NB;
-  double* krow = jpart + (blockDim.x / 64) * (ncart(Lc) * ncart(Ld) * kJPad);
+  double* krow = jpart + (blockDim.x / (64 * NCH)) * kJPart<NCH, ncart(Lc) * ncart(Ld)>;
   const int w = (threadIdx.x >> 6) % NCH;  // uniform over the wavefront
   for (int c = blockIdx.x; c < g.nchunks; c += gridDim.x) {
     const JkChunk ch = load_chunk_uniform(g.chunks, c);
@@ -1530,9 +1568,8 @@ __global__ __launch_bounds__(NT, (lds_kernel_wpe<La, Lb, Lc, Ld, NT>())) void jk
     const int fa = bra.fa, fb = bra.fb;
     const bool ij = bra.same;
     const JkSegs* sg = g.segs + ch.seg;
-    int seg = 0;
     for (int k = ch.k0; k < ch.k1; ++k) {
-      const int kp = chunk_ket(sg, k, seg);
+      const int kp = chunk_ket(sg, k);
       const PairRec ket = load_pair_uniform(g.pairs, kp);
       const int mode = quartet_select(g.sel, ch.bra, bra, kp, ket);
       if (mode == 0) continue;  // uniform over the workgroup
@@ -1862,9 +1899,8 @@ __global__ __launch_bounds__(64 * NW, (WaveLds<La, Lb, Lc, Ld, NW>::WPE)) void j
     const int fa = bra.fa, fb = bra.fb;
     const bool ij = bra.same;
     const JkSegs* sg = g.segs + ch.seg;
-    int seg = 0;
     for (int k = ch.k0 + wave; k < ch.k1; k += NW) {  // uniform over the wavefront
-      const int kp = chunk_ket(sg, k, seg);
+      const int kp = chunk_ket(sg, k);
       const PairRec ket = load_pair_uniform(g.pairs, kp);
       const int mode = quartet_select(g.sel, ch.bra, bra, kp, ket);
       if (mode == 0) continue;

@@ -37,6 +37,7 @@ struct GradArgs {
   const JkSegs* __restrict__ segs;
   QuartetSel sel;
   const double* __restrict__ ppih;  // 1 / (2 zeta) of each primitive pair
+  int chain, kmax;  // division of the kets' primitives over lanes (ket_split)
 };
 
 // Primitive quartets per step of the LDS-shape gradient kernel: 3 n_r lanes
@@ -95,17 +96,16 @@ __global__ __launch_bounds__(NT) void grad_kernel(GradArgs g) {
   }
 
   for (int ci = blockIdx.x; ci < g.nchunks; ci += gridDim.x) {
-   const JkChunk ch = g.chunks[ci];
-   const PairRec bra = g.pairs[ch.bra];
+   const JkChunk ch = load_chunk_uniform(g.chunks, ci);
+   const PairRec bra = load_pair_uniform(g.pairs, ch.bra);
    const JkSegs* sg = g.segs + ch.seg;
-   int seg = 0;
    // gridDim.y workgroups share a chunk (chunks of the register-shape J/K
    // classes hold up to 2048 quartets)
    const int len = ch.k1 - ch.k0;
    const int kb = ch.k0 + int((long long)len * blockIdx.y / gridDim.y);
    const int ke = ch.k0 + int((long long)len * (blockIdx.y + 1) / gridDim.y);
    for (int kq = kb; kq < ke; ++kq) {
-    const int kp = chunk_ket(sg, kq, seg);
+    const int kp = chunk_ket(sg, kq);
     const PairRec ket = g.pairs[kp];
     if (quartet_select(g.sel, ch.bra, bra, kp, ket) == 0) continue;  // uniform over the workgroup
     const bool ij = bra.same, kl = ket.same, bk = (kp == ch.bra);
@@ -254,7 +254,7 @@ __global__ __launch_bounds__(NT) void grad_kernel(GradArgs g) {
 // --------------------------------------------------------------------------
 template <int La, int Lb, int Lc, int Ld>
 __device__ __forceinline__ void grad_quartet_regs(const GradArgs& g, const PairRec& bra, const PairRec& ket,
-                                                  bool bk, double (&f)[9]) {
+                                                  bool bk, int ik0, int per, double (&f)[9]) {
   constexpr int NR = (La + Lb + Lc + Ld + 1) / 2 + 1;
   constexpr int na = ncart(La), nb = ncart(Lb), nc = ncart(Lc), nd = ncart(Ld);
   const size_t n = size_t(bra.mn);
@@ -279,7 +279,8 @@ __device__ __forceinline__ void grad_quartet_regs(const GradArgs& g, const PairR
   for (int x = 0; x < 9; ++x) f[x] = 0.0;
   const double ABx = bra.ABx, ABy = bra.ABy, ABz = bra.ABz;
   const double CDx = ket.ABx, CDy = ket.ABy, CDz = ket.ABz;
-  for (int ik = 0; ik < ket.npp_sig; ++ik) {
+  const int ik1 = min(ket.npp_sig, ik0 + per);
+  for (int ik = ik0; ik < ik1; ++ik) {
     const PrimPair Q = g.pp[ket.pp_off + ik];
     const double2 ek = g.ppab[ket.pp_off + ik];
     const double eta = Q.zeta, h_e = g.ppih[ket.pp_off + ik];
@@ -372,20 +373,22 @@ __global__ __launch_bounds__(256) void grad_kernel_regs(GradArgs g) {
       atomic_add(&g.grad[i], v);
   };
   for (int ci = blockIdx.x; ci < g.nchunks; ci += gridDim.x) {
-    const JkChunk ch = g.chunks[ci];
-    const PairRec bra = g.pairs[ch.bra];
+    const JkChunk ch = load_chunk_uniform(g.chunks, ci);
+    const PairRec bra = load_pair_uniform(g.pairs, ch.bra);
     const int iA = 3 * g.shell_atom[bra.sa], iB = 3 * g.shell_atom[bra.sb];
     double fab[6] = {0, 0, 0, 0, 0, 0};
     const JkSegs* sg = g.segs + ch.seg;
-    for (int s0 = ch.k0; s0 < ch.k1; s0 += kSortRun) {
-    const int nsel = sort_run<256>(sg, g.pairs, g.sel, ch.bra, bra, s0, min(ch.k1, s0 + kSortRun), srt, 256);
+    const KetSplit sp = ket_split_uniform(g.chain, g.kmax, bra.npp_sig);
+    for (int s0 = ch.k0; s0 < ch.k1; s0 += sp.run) {
+    const int nsel = sort_run<256>(sg, g.pairs, g.sel, ch.bra, bra, sp, s0, min(ch.k1, s0 + sp.run), srt, 256);
     for (int r = 0; 256 * r < nsel; ++r) {
       const int i = sorted_block(tid, r, 4) + (tid & 63);
       if (i >= nsel) continue;
-      const int kp = int(srt.get(i) & ~kSortF32);
+      const unsigned ent = srt.e[i];
+      const int kp = chunk_ket(sg, s0 + entry_pos(ent));
       const PairRec ket = g.pairs[kp];
       double f[9];
-      grad_quartet_regs<La, Lb, Lc, Ld>(g, bra, ket, kp == ch.bra, f);
+      grad_quartet_regs<La, Lb, Lc, Ld>(g, bra, ket, kp == ch.bra, entry_part(ent) * sp.per, sp.per, f);
 #pragma unroll
       for (int x = 0; x < 6; ++x) fab[x] += f[x];
       const int iC = 3 * g.shell_atom[ket.sa], iD = 3 * g.shell_atom[ket.sb];

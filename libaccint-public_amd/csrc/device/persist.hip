@@ -34,8 +34,9 @@ struct PersistClass {
   static constexpr bool covered = P::regs && P::CHA == P::CHA0 && (P::NCH == 1 || P::NCH == 2 || P::NCH == 4);
   // dynamic LDS in doubles: the merged slices' ket Coulomb parts or the
   // wavefronts' tiles, then the exchange rows (na + nb rows of nbf)
-  static constexpr int jpart =
-      (kPersistNT / 64) * (P::NCH > 1 ? ncart(Lc) * ncart(Ld) * kJPad : kJTile<Lc, Ld>);
+  static constexpr int jpart = P::NCH > 1
+                                   ? (kPersistNT / (64 * P::NCH)) * kJPart<P::NCH, ncart(Lc) * ncart(Ld)>
+                                   : (kPersistNT / 64) * kJTile<Lc, Ld>;
   static constexpr int rows = ncart(La) + ncart(Lb);
 };
 

@@ -25,9 +25,8 @@ __global__ __launch_bounds__(256) void worklist_stats_kernel(WlStatsArgs a) {
     const JkChunk ch = a.chunks[ci];
     const PairRec bra = a.pairs[ch.bra];
     const JkSegs* sg = a.segs + ch.seg;
-    int seg = 0;
     for (int k = ch.k0 + tid; k < ch.k1; k += blockDim.x) {
-      const int kp = chunk_ket(sg, k, seg);
+      const int kp = chunk_ket(sg, k);
       const PairRec ket = a.pairs[kp];
       const int mode = quartet_select(a.sel, ch.bra, bra, kp, ket);
       if (mode == 0) continue;

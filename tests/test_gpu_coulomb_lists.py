@@ -63,3 +63,47 @@ def test_batch_of_unequal_molecules():
         Jo, Ko = oracle.Oracle(oracle.RawBasis(b, a)).jk_canonical(Ds[k])
         sl = slice(off[k], off[k + 1])
         assert rel(J[sl].reshape(Jo.shape), Jo) < TOL and rel(K[sl].reshape(Ko.shape), Ko) < TOL
+
+
+def contracted(n, n_prim, seed):
+    """n atoms, each with one s and one p shell of n_prim primitives."""
+    rng = np.random.default_rng(seed)
+    ex = list(0.15 * 2.1 ** np.arange(n_prim))
+    at = rng.uniform(0.0, 3.0 * n ** (1.0 / 3.0), (n, 3))
+    return [(l, tuple(p), ex, list(rng.uniform(0.2, 1.0, n_prim))) for p in at for l in (0, 1)]
+
+
+@pytest.mark.parametrize("n_atoms, n_prim", [(1, 1), (1, 2), (2, 5), (3, 10), (1, 13), (9, 4)])
+def test_divided_kets_match_oracle(n_atoms, n_prim):
+    """Few quartets of long contractions: a quartet's ket primitives are divided
+    over lanes (n_prim^2 pairs a ket: 1 to 169, so one part, several, more than
+    the 127 a quartet may have), in J, K and the gradient."""
+    print("divided kets", n_atoms, n_prim, flush=True)
+    sh = contracted(n_atoms, n_prim, 5)
+    basis = lai.BasisSet([lai.Shell(l, list(p), e, c) for l, p, e, c in sh])
+    n = basis.n_basis_functions()
+    D = systems.density(n, 2, 11, 1.0 / np.sqrt(n))
+    raw = oracle.RawBasis.__new__(oracle.RawBasis)
+    raw.L = np.array([s[0] for s in sh], dtype=np.int32)
+    raw.centers = np.array([s[1] for s in sh])
+    raw.nprim = np.array([n_prim] * len(sh), dtype=np.int32)
+    raw.exps = np.concatenate([s[2] for s in sh])
+    raw.raw_coefs = np.concatenate([s[3] for s in sh])
+    raw.nbf, raw.n_shells = n, len(sh)
+    opts = lai.JKOptions(schwarz_threshold=0.0)
+    e = lai.Engine(basis)
+    J, K = e.build_jk(D, opts)
+    Jo, Ko = oracle.Oracle(raw).jk_canonical(D)
+    assert rel(J, Jo) < TOL and rel(K, Ko) < TOL
+    # dE/dx of the first shell against fourth-order central differences of the
+    # same energy: with h = 1e-4 and exponents up to 0.15 * 2.1^12 = 1100 the
+    # truncation h^4/30 E^(5) ~ h^4/30 |g| (2 * 1100)^2 is below 1e-9 (second
+    # order leaves h^2/6 |g| 2200 ~ 1e-4), rounding 1e-15 |E| / h below 1e-10
+    g = e.compute_jk_gradient(D, 1.0, len(sh))
+
+    def energy(dx):
+        moved = [(l, (p[0] + (dx if k == 0 else 0.0), p[1], p[2]), x, c) for k, (l, p, x, c) in enumerate(sh)]
+        J, K = lai.Engine(lai.BasisSet([lai.Shell(l, list(p), x, c) for l, p, x, c in moved])).build_jk(D, opts)
+        return 0.5 * np.sum(D * J) - 0.25 * np.sum(D * K)
+    fd = (8.0 * (energy(1e-4) - energy(-1e-4)) - (energy(2e-4) - energy(-2e-4))) / 12e-4
+    assert abs(g[0, 0] - fd) < 1e-6 * max(1.0, abs(energy(0.0)))
