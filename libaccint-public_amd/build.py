@@ -32,6 +32,7 @@ HIP_FLAGS = [
     "-I" + INC, "-I" + DEV, "-Wno-unused-command-line-argument",
 ]
 NPARTS = 8
+NGRAD = 4
 
 
 def _run(cmd):
@@ -67,7 +68,14 @@ def build_device(incremental=False, jobs=8):
         if not incremental or _stale(o, [src] + hdr):
             tasks.append([HIPCC] + HIP_FLAGS + ["-DLAI_PART=%d" % k, "-DLAI_NPARTS=%d" % NPARTS,
                                                 "-c", src, "-o", o])
-    for name in ("aux_kernels", "grad_inst", "wl_kernels", "df", "fock_kernels", "persist", "api"):
+    for k in range(NGRAD):
+        o = os.path.join(BUILD, "grad_inst_%d.o" % k)
+        src = os.path.join(DEV, "grad_inst.hip")
+        objs.append(o)
+        if not incremental or _stale(o, [src] + hdr):
+            tasks.append([HIPCC] + HIP_FLAGS + ["-DLAI_PART=%d" % k, "-DLAI_NPARTS=%d" % NGRAD,
+                                                "-c", src, "-o", o])
+    for name in ("aux_kernels", "wl_kernels", "df", "fock_kernels", "persist", "api"):
         src = os.path.join(DEV, name + ".hip")
         o = os.path.join(BUILD, name + ".o")
         objs.append(o)

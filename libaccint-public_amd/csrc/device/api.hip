@@ -64,7 +64,12 @@ const Launchers& launchers() {
 
 struct GradLaunchers {
   GradLauncher f[kNumGradClasses] = {};
-  GradLaunchers() { fill_grad_launchers(f); }
+  GradLaunchers() {
+    fill_grad_launchers_part_0(f);
+    fill_grad_launchers_part_1(f);
+    fill_grad_launchers_part_2(f);
+    fill_grad_launchers_part_3(f);
+  }
 };
 const GradLaunchers& grad_launchers() {
   static GradLaunchers G;

@@ -240,6 +240,34 @@ __device__ __forceinline__ void boys01(double T, const double* __restrict__ tab,
   boys01_at(T, tab + LAI_B8_OFF, F0, F1);
 }
 
+// F_0, F_1 and F_2 from the two-root rows (F_0..F_9 of each grid point, seven
+// Taylor terms each), and from the limit F_m = (2m-1)!!/(2T)^m sqrt(pi/T)/2
+// at or above the two-root cut
+template <typename P>
+__device__ __forceinline__ void boys012_at(double T, P rows, double& F0, double& F1, double& F2) {
+  if (T < double(lai_rys_tcut[2])) {
+    const int k = int(fma(T, double(LAI_BT_PER_UNIT), 0.5));
+    const double d = T - double(k) * (1.0 / LAI_BT_PER_UNIT);
+    double e[7];
+#pragma unroll
+    for (int j = 1; j <= 6; ++j) e[j] = -d * (1.0 / j);
+    double r[9];
+#pragma unroll
+    for (int m = 0; m < 9; ++m) r[m] = rows[k * kRowStride<P, kBoysRowW<2>> + m];
+    F0 = boys_step(r, 0, e);
+    F1 = boys_step(r, 1, e);
+    F2 = boys_step(r, 2, e);
+  } else {
+    double y = __builtin_amdgcn_rsq(T);
+    y = fma(0.5 * y, fma(-T * y, y, 1.0), y);
+    y = fma(0.5 * y, fma(-T * y, y, 1.0), y);
+    const double h = 0.5 * y * y;  // 1 / (2 T)
+    F0 = 0.88622692545275801365 * y;  // sqrt(pi) / 2
+    F1 = F0 * h;
+    F2 = 3.0 * F1 * h;
+  }
+}
+
 // One- and two-root rules: moments F_0..F_{2N-1} from the Boys Taylor rows
 // (T below the cut), then the Gauss rule of the moments in closed form
 template <int N, typename P>

@@ -60,6 +60,9 @@ int launch_persistent(const EriArgs& a, const PersistItem* items, int n_items, i
 // gradient kernels exist for the classes whose shells are at most d
 inline constexpr int kNumGradClasses = 21;
 using GradLauncher = void (*)(const GradArgs&, hipStream_t, int max_blocks);
-void fill_grad_launchers(GradLauncher*);
+void fill_grad_launchers_part_0(GradLauncher*);
+void fill_grad_launchers_part_1(GradLauncher*);
+void fill_grad_launchers_part_2(GradLauncher*);
+void fill_grad_launchers_part_3(GradLauncher*);
 
 }  // namespace lai
