@@ -358,15 +358,20 @@ int lai_dev_df_dims(const lai_df* df, int* n_orb, int* n_aux);
  * compute_k_internal (src/shared/consumers/df_fock_builder.cpp:283-378). */
 #define LAI_DF_J 1
 #define LAI_DF_K 2
-/* with LAI_DF_K: the caller states that D is symmetric, so K is symmetric;
- * the exchange product then skips the workgroup tiles below the diagonal and
- * copies the lower triangle of K from the upper one */
+/* the caller states that D is symmetric (only its upper triangle may be read),
+ * so K is symmetric: the exchange product skips the workgroup tiles below the
+ * diagonal and copies the lower triangle of K from the upper one.  A D that is
+ * also positive semidefinite of rank at most n_orb/2, as the density of
+ * occupied orbitals is, is factored on the device and the exchange runs over
+ * the factor's columns (D is reproduced to 7e-15 of its largest diagonal
+ * element, else the general products run) */
 #define LAI_DF_SYMMETRIC 4
 int lai_dev_df_jk(lai_df* df, const double* d_D, double* d_J, double* d_K, int flags, void* stream);
 /* as lai_dev_df_jk, synchronous, with each kernel timed by HIP events on
- * stream: ms[0] the fitted density gamma (a pass over B for J alone; with J
- * and K together, the diagonal of X: gamma_P = sum_a (B_P D)_aa), ms[1] the
- * J pass, ms[2] the X = B D GEMM,
+ * stream: ms[0] the fitted density gamma (a pass over B for J alone and for a
+ * D that is factored; with J and K together otherwise the diagonal of X:
+ * gamma_P = sum_a (B_P D)_aa), ms[1] the J pass, ms[2] the X = B D GEMM (or the
+ * factorisation of D and X = B L),
  * ms[3] the K = X B^T GEMM (split over the summation index), ms[4] the sum of
  * its slices (entries of kernels not run are 0).  No reference counterpart
  * (measurement). */
