@@ -779,24 +779,75 @@ struct EriBatch {
   std::vector<Quartet> q[kNumClasses];
   std::vector<int> perm[kNumClasses];
   std::vector<long long> obase[kNumClasses];
+  long long work[kNumClasses] = {};     // primitive quartets of the class
+  long long longest[kNumClasses] = {};  // and of its longest quartet
+
+  void add(const lai_basis* b, int c, const Quartet& x, int pm, long long off) {
+    q[c].push_back(x);
+    perm[c].push_back(pm);
+    obase[c].push_back(off);
+    const long long w = (long long)b->pairs_h[x.bra].npp * b->pairs_h[x.ket].npp;
+    work[c] += w;
+    longest[c] = std::max(longest[c], w);
+  }
+  // staging layout: per class with work, its Quartet, perm and obase arrays,
+  // each 256-byte aligned; at most 20 bytes per quartet plus 3 * 256 per class
+  static size_t up(size_t x) { return (x + 255) & ~size_t(255); }
+  size_t staging_bytes() const {
+    size_t need = 0;
+    for (int c = 0; c < kNumClasses; ++c) {
+      const size_t nq = q[c].size();
+      if (nq) need += up(nq * sizeof(Quartet)) + up(nq * sizeof(int)) + up(nq * sizeof(long long));
+    }
+    return need;
+  }
 };
 
-// Runs mode-1 kernels for a classified batch writing into d_out (device).
-int run_eri_batch(lai_basis* b, EriBatch& eb, double* d_out, hipStream_t st) {
-  const auto& Ls = launchers();
+// Lanes per quartet of a class.  While the list leaves the chip idle, so many
+// that a lane keeps four primitive quartets of the longest (one lane per
+// quartet, the 2401 (ss|ss) of a water in cc-pVDZ took 1.76 ms, with 64 lanes
+// 0.05 ms: the longest has 4096; the whole list of 20736 quartets 10.2 -> 1.4
+// ms, of which 0.6 are kernels); beyond 8 wavefronts per CU only while the mean quartet gives each
+// lane four as well, since lanes without work then cost time.
+int eri_lanes(const EriBatch& eb, int c, int n_cu) {
+  const long long nq = (long long)eb.q[c].size(), mean = eb.work[c] / std::max(1ll, nq);
+  int l = 1;
+  while (l < 64 && 8 * l <= eb.longest[c] && (nq * 2 * l <= 512ll * n_cu || 8 * l <= mean)) l *= 2;
+  return l;
+}
+
+// Stages the classified batch at base (staging_bytes() of device memory) and
+// runs the mode-1 kernels, writing into d_out (device); returns when they are
+// done.  One copy and one wait for all classes.
+int run_eri_staged(lai_basis* b, const EriBatch& eb, unsigned char* base, double* d_out, hipStream_t st) {
+  std::vector<unsigned char> stage(eb.staging_bytes());
+  if (stage.empty()) return LAI_OK;
+  size_t off = 0;
+  auto put = [&](const void* p, size_t n) {
+    std::memcpy(stage.data() + off, p, n);
+    off += EriBatch::up(n);
+  };
   for (int c = 0; c < kNumClasses; ++c) {
-    const int nq = int(eb.q[c].size());
+    const size_t nq = eb.q[c].size();
     if (nq == 0) continue;
-    DevBuf<Quartet> dq;
-    DevBuf<int> dp;
-    DevBuf<long long> dob;
-    hipError_t e;
-    if ((e = dq.assign(eb.q[c].data(), nq)) != hipSuccess || (e = dp.assign(eb.perm[c].data(), nq)) != hipSuccess ||
-        (e = dob.assign(eb.obase[c].data(), nq)) != hipSuccess)
-      return fail(LAI_ERR_MEMORY, std::string("eri batch: ") + hipGetErrorString(e));
+    put(eb.q[c].data(), nq * sizeof(Quartet));
+    put(eb.perm[c].data(), nq * sizeof(int));
+    put(eb.obase[c].data(), nq * sizeof(long long));
+  }
+  LAI_HIP(hipMemcpyAsync(base, stage.data(), stage.size(), hipMemcpyHostToDevice, st));
+  const auto& Ls = launchers();
+  hipError_t e = hipSuccess;
+  for (int c = 0; c < kNumClasses && e == hipSuccess; ++c) {
+    const size_t nq = eb.q[c].size();
+    if (nq == 0) continue;
     EriArgs a{};
-    a.q = dq.p;
-    a.nq = nq;
+    a.q = reinterpret_cast<const Quartet*>(base);
+    base += EriBatch::up(nq * sizeof(Quartet));
+    a.perm = reinterpret_cast<const int*>(base);
+    base += EriBatch::up(nq * sizeof(int));
+    a.obase = reinterpret_cast<const long long*>(base);
+    base += EriBatch::up(nq * sizeof(long long));
+    a.nq = int(nq);
     a.pairs = b->pairs.p;
     a.pp = b->pp.p;
     a.rys = b->ctx->rys.p;
@@ -805,16 +856,28 @@ int run_eri_batch(lai_basis* b, EriBatch& eb, double* d_out, hipStream_t st) {
     a.pcut32 = b->pcut32;
     a.mode = 1;
     a.out = d_out;
-    a.perm = dp.p;
-    a.obase = dob.p;
     a.nbf = b->max_nbf;
     LaunchTune t;
     t.n_cu = b->ctx->n_cu;
+    a.lanes = eri_lanes(eb, c, t.n_cu);
     Ls.f64[c](a, st, t);
-    LAI_HIP(hipGetLastError());
-    LAI_HIP(hipStreamSynchronize(st));
+    e = hipGetLastError();
   }
+  // the staged arrays are released on return: copy and kernels must be done,
+  // after a failed launch too
+  const hipError_t w = hipStreamSynchronize(st);
+  LAI_HIP(e);
+  LAI_HIP(w);
   return LAI_OK;
+}
+
+int run_eri_batch(lai_basis* b, const EriBatch& eb, double* d_out, hipStream_t st) {
+  DevBuf<unsigned char> d;
+  const hipError_t e = d.alloc(eb.staging_bytes());
+  if (e != hipSuccess) return fail(LAI_ERR_MEMORY, std::string("eri batch: ") + hipGetErrorString(e));
+  const int rc = run_eri_staged(b, eb, d.p, d_out, st);
+  d.release();
+  return rc;
 }
 }  // namespace
 
@@ -833,9 +896,7 @@ int classify_batch(lai_basis* b, int64_t n, const int* s4, int64_t* offsets, Eri
     if (c < 0)
       return fail(LAI_ERR_INVALID_ARGUMENT, std::string(what) + ": the shells of a pair must belong to one molecule");
     offsets[t] = off;
-    eb.q[c].push_back(q);
-    eb.perm[c].push_back(perm);
-    eb.obase[c].push_back(off);
+    eb.add(b, c, q, perm, off);
     off += int64_t(ncart(b->L[s[0]])) * ncart(b->L[s[1]]) * ncart(b->L[s[2]]) * ncart(b->L[s[3]]);
   }
   offsets[n] = off;
@@ -887,55 +948,10 @@ extern "C" int lai_dev_eri_quartets_device_noalloc(lai_basis* b, int64_t n, cons
   const int dev = b->ctx->device;
   if (dev < 0 || dev >= kMaxDevices || !g_scratch[dev])
     return fail(LAI_ERR_INVALID_STATE, "lai_dev_eri_quartets_device_noalloc: staging array not set up");
-  unsigned char* base = static_cast<unsigned char*>(g_scratch[dev]);
-  // layout: per class with work, its Quartet, perm and obase arrays, each
-  // 256-byte aligned; at most 20 bytes per quartet plus 3 * 256 per class
-  auto up = [](size_t x) { return (x + 255) & ~size_t(255); };
-  size_t need = 0;
-  for (int c = 0; c < kNumClasses; ++c) {
-    const size_t nq = eb.q[c].size();
-    if (nq) need += up(nq * sizeof(Quartet)) + up(nq * sizeof(int)) + up(nq * sizeof(long long));
-  }
-  if (need > kScratchBytes)
+  if (eb.staging_bytes() > kScratchBytes)
     return fail(LAI_ERR_INVALID_ARGUMENT, "lai_dev_eri_quartets_device_noalloc: staging array too small");
-  hipStream_t st = hipStream_t(stream);
   std::lock_guard<std::mutex> lk(g_scratch_mtx);  // one staging call at a time in this process
-  const auto& Ls = launchers();
-  size_t off = 0;
-  for (int c = 0; c < kNumClasses; ++c) {
-    const int nq = int(eb.q[c].size());
-    if (nq == 0) continue;
-    auto* dq = reinterpret_cast<Quartet*>(base + off);
-    off += up(size_t(nq) * sizeof(Quartet));
-    auto* dp = reinterpret_cast<int*>(base + off);
-    off += up(size_t(nq) * sizeof(int));
-    auto* dob = reinterpret_cast<long long*>(base + off);
-    off += up(size_t(nq) * sizeof(long long));
-    LAI_HIP(hipMemcpyAsync(dq, eb.q[c].data(), sizeof(Quartet) * nq, hipMemcpyHostToDevice, st));
-    LAI_HIP(hipMemcpyAsync(dp, eb.perm[c].data(), sizeof(int) * nq, hipMemcpyHostToDevice, st));
-    LAI_HIP(hipMemcpyAsync(dob, eb.obase[c].data(), sizeof(long long) * nq, hipMemcpyHostToDevice, st));
-    EriArgs a{};
-    a.q = dq;
-    a.nq = nq;
-    a.pairs = b->pairs.p;
-    a.pp = b->pp.p;
-    a.rys = b->ctx->rys.p;
-    a.ppb = b->ppb.p;
-    a.ppih = b->ppih.p;
-    a.pcut32 = b->pcut32;
-    a.mode = 1;
-    a.out = d_out;
-    a.perm = dp;
-    a.obase = dob;
-    a.nbf = b->max_nbf;
-    LaunchTune t;
-    t.n_cu = b->ctx->n_cu;
-    Ls.f64[c](a, st, t);
-    LAI_HIP(hipGetLastError());
-  }
-  // the host descriptor arrays are released on return: the copies must be done
-  LAI_HIP(hipStreamSynchronize(st));
-  return LAI_OK;
+  return run_eri_staged(b, eb, static_cast<unsigned char*>(g_scratch[dev]), d_out, hipStream_t(stream));
 }
 
 // ---------------------------------------------------------------------------
@@ -954,9 +970,7 @@ extern "C" int lai_dev_schwarz(lai_basis* b, double* Qout) {
     Quartet q;
     int perm;
     const int c = classify(b, s, q, perm);
-    eb.q[c].push_back(q);
-    eb.perm[c].push_back(perm);
-    eb.obase[c].push_back(off);
+    eb.add(b, c, q, perm, off);
     offs[p] = off;
     ni[p] = ncart(b->L[i]);
     nj[p] = ncart(b->L[j]);

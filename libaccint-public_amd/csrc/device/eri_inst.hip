@@ -87,7 +87,7 @@ void launch_class(const EriArgs& a0, hipStream_t s, const LaunchTune& t) {
     if (MIXED || a.nq <= 0) return;
     const int max_blocks = t.n_cu * 16;  // grid-stride over the quartet list
     if constexpr (P::regs) {
-      int blocks = (a.nq + 127) / 128;
+      int blocks = int(((long long)a.nq * a.lanes + 127) / 128);
       if (blocks > max_blocks) blocks = max_blocks;
       dim3 grid(blocks, P::NCH);
       hipLaunchKernelGGL((eri_kernel_regs<La, Lb, Lc, Ld, double, P::CHA>), grid, dim3(128), 0, s, a);

@@ -255,6 +255,7 @@ struct EriArgs {
   const JkChunk* __restrict__ chunks;
   int nchunks;
   const JkSegs* __restrict__ segs;
+  int lanes;  // raw ERIs: lanes that divide the primitive quartets of one quartet
   int klds;  // 1: the bra rows of Kt are accumulated in LDS (dynamic shared memory)
   int chain, kmax;  // division of the kets' primitives over lanes (ket_split)
   QuartetSel sel;
@@ -331,18 +332,24 @@ __device__ __forceinline__ int orig_offset(int perm, const int (&idx)[4], const 
 }
 
 // --------------------------------------------------------------------------
-// Kernel A: one lane per shell quartet, bra index a in [A0, A1)
+// Kernel A: g.lanes lanes (a power of two, at most 64) per shell quartet, bra
+// index a in [A0, A1).  The lanes divide the primitive quartets and add their
+// blocks by shuffles: a lane alone takes up to 64 x 64 of them in turn (0.4 us
+// each), and a list of some thousand quartets does not fill the chip.
 // --------------------------------------------------------------------------
 // Contracted, normalised block gv[a - A0][b][c][d] of the quartet (bra|ket);
 // all_prims selects every primitive pair (raw ERIs) or only those above the
 // primitive screening bound (J/K), there only the ket's ik0 .. ik0 + per - 1.
+// Raw ERIs take every kstep-th ket pair from ik0 and every bstep-th bra pair
+// from ib0.
 // LB: the Boys Taylor rows (one and two roots) or the Chebyshev coefficients
 // of the rule (three and four roots) from the workgroup's copy in LDS
 // (lrows), else from the device table
 template <int La, int Lb, int Lc, int Ld, typename R, int A0, int A1, bool LB = false>
 __device__ __forceinline__ void quartet_block_regs(
     const EriArgs& g, const PairRec& bra, const PairRec& ket, bool all_prims,
-    double (&gv)[A1 - A0][ncart(Lb)][ncart(Lc)][ncart(Ld)], lds_cdptr lrows = nullptr, int ik0 = 0, int per = 0) {
+    double (&gv)[A1 - A0][ncart(Lb)][ncart(Lc)][ncart(Ld)], lds_cdptr lrows = nullptr, int ik0 = 0, int per = 0,
+    int kstep = 1, int ib0 = 0, int bstep = 1) {
   constexpr int nb = ncart(Lb), nc = ncart(Lc), nd = ncart(Ld);
   constexpr int NA = A1 - A0;
   constexpr int NR = (La + Lb + Lc + Ld) / 2 + 1;
@@ -369,13 +376,13 @@ __device__ __forceinline__ void quartet_block_regs(
   // ket primitive pairs outside (one load per lane and pair), bra primitive
   // pairs inside: the bra is the same for the whole workgroup in the J/K
   // kernels, so its records are uniform (scalar) loads
-  for (int ik = ik0; ik < nk_pp; ++ik) {
+  for (int ik = ik0; ik < nk_pp; ik += kstep) {
     const float bk = fp32 ? g.ppb[ket.pp_off + ik] : 0.0f;
     if (fp32 && bk * bb0 < qcut) break;
     const PrimPair Q = g.pp[ket.pp_off + ik];
     const double eta = Q.zeta;
     const double h_e = g.ppih[ket.pp_off + ik];  // 1 / (2 eta)
-    for (int ib = 0; ib < nb_pp; ++ib) {
+    for (int ib = ib0; ib < nb_pp; ib += bstep) {
       if (fp32 && as_const(g.ppb)[bra.pp_off + ib] * bk < qcut) break;
       // the bra is uniform in the J/K kernels: scalar loads
       const PrimPair P = load_prim(g.pp, bra.pp_off + ib);
@@ -473,14 +480,27 @@ __device__ __forceinline__ void quartet_block_regs(
 }
 
 template <int La, int Lb, int Lc, int Ld, typename R, int A0, int A1>
-__device__ __forceinline__ void quartet_regs(const EriArgs& g, int qi) {
+__device__ __forceinline__ void quartet_regs(const EriArgs& g, int qi, int part) {
   constexpr int nb = ncart(Lb), nc = ncart(Lc), nd = ncart(Ld);
   constexpr int NA = A1 - A0;
   const Quartet q = g.q[qi];
   const PairRec bra = g.pairs[q.bra];
   const PairRec ket = g.pairs[q.ket];
   double gv[NA][nb][nc][nd];
-  quartet_block_regs<La, Lb, Lc, Ld, R, A0, A1>(g, bra, ket, true, gv);
+  // ket pairs over as many of the lanes as there are, bra pairs over the rest
+  int kl = 1;
+  while (kl < g.lanes && kl < ket.npp) kl *= 2;
+  quartet_block_regs<La, Lb, Lc, Ld, R, A0, A1>(g, bra, ket, true, gv, nullptr, part & (kl - 1), 0, kl, part / kl,
+                                                g.lanes / kl);
+  for (int o = g.lanes / 2; o >= 1; o /= 2)
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
+      for (int b = 0; b < nb; ++b)
+#pragma unroll
+        for (int c = 0; c < nc; ++c)
+#pragma unroll
+          for (int d = 0; d < nd; ++d) gv[a][b][c][d] += __shfl_xor(gv[a][b][c][d], o, 64);
 
   constexpr int na = ncart(La);
   const int perm = g.perm[qi];
@@ -495,27 +515,29 @@ __device__ __forceinline__ void quartet_regs(const EriArgs& g, int qi) {
 #pragma unroll
         for (int d = 0; d < nd; ++d) {
           const int idx[4] = {A0 + a, b, c, d};
-          out[orig_offset(perm, idx, n4)] = gv[a][b][c][d];
+          const int e = ((a * nb + b) * nc + c) * nd + d;
+          if ((e & (g.lanes - 1)) == part) out[orig_offset(perm, idx, n4)] = gv[a][b][c][d];
         }
 }
 
 template <int La, int Lb, int Lc, int Ld, typename R, int CHA, int C>
-__device__ __forceinline__ void dispatch_chunk(const EriArgs& g, int qi, int chunk) {
+__device__ __forceinline__ void dispatch_chunk(const EriArgs& g, int qi, int part, int chunk) {
   constexpr int na = ncart(La);
   constexpr int A0 = C * CHA;
   constexpr int A1 = (A0 + CHA < na) ? A0 + CHA : na;
   if (chunk == C) {
-    quartet_regs<La, Lb, Lc, Ld, R, A0, A1>(g, qi);
+    quartet_regs<La, Lb, Lc, Ld, R, A0, A1>(g, qi, part);
   } else if constexpr (A1 < na) {
-    dispatch_chunk<La, Lb, Lc, Ld, R, CHA, C + 1>(g, qi, chunk);
+    dispatch_chunk<La, Lb, Lc, Ld, R, CHA, C + 1>(g, qi, part, chunk);
   }
 }
 
 template <int La, int Lb, int Lc, int Ld, typename R, int CHA>
 __global__ __launch_bounds__(128) void eri_kernel_regs(EriArgs g) {
   const int chunk = blockIdx.y;
-  for (int qi = blockIdx.x * blockDim.x + threadIdx.x; qi < g.nq; qi += gridDim.x * blockDim.x)
-    dispatch_chunk<La, Lb, Lc, Ld, R, CHA, 0>(g, qi, chunk);
+  const int part = threadIdx.x & (g.lanes - 1), step = blockDim.x / g.lanes;
+  for (int qi = blockIdx.x * step + threadIdx.x / g.lanes; qi < g.nq; qi += gridDim.x * step)
+    dispatch_chunk<La, Lb, Lc, Ld, R, CHA, 0>(g, qi, part, chunk);
 }
 
 // --------------------------------------------------------------------------
