@@ -1088,7 +1088,9 @@ std::vector<JkChunk> cut_runs(const lai_basis* b, const ClassList& cl, int cmax,
 }
 
 int class_shape(const ClassInfo& info, const ClassTune& t) {
-  return (t.alt && info.alt != kShapeNone) ? info.alt : info.shape;
+  return (t.alt == 2 && info.alt2 != kShapeNone)  ? info.alt2
+         : (t.alt && info.alt != kShapeNone) ? info.alt
+                                             : info.shape;
 }
 
 // Whether a mixed build runs class c's FP32 quartets through the float
@@ -1854,12 +1856,13 @@ extern "C" int lai_dev_set_tuning(lai_basis* b, const lai_class_tune* table, int
     if (e.cls < 0 || e.cls >= kNumClasses)
       return fail(LAI_ERR_INVALID_ARGUMENT, "lai_dev_set_tuning: class " + std::to_string(e.cls) + " out of range");
     const ClassInfo& info = Ls.info[e.cls];
-    if (e.strategy != info.shape && (info.alt == kShapeNone || e.strategy != info.alt))
+    if (e.strategy != info.shape && (info.alt == kShapeNone || e.strategy != info.alt) &&
+        (info.alt2 == kShapeNone || e.strategy != info.alt2))
       return fail(LAI_ERR_UNSUPPORTED, "lai_dev_set_tuning: strategy " + std::to_string(e.strategy) +
                                            " is not compiled for class " + std::to_string(e.cls));
     if (e.chunk < 0 || e.chunk > (1 << 20) || e.blocks_per_cu < 0 || e.blocks_per_cu > 4096)
       return fail(LAI_ERR_INVALID_ARGUMENT, "lai_dev_set_tuning: chunk or blocks_per_cu out of range");
-    next[e.cls].alt = e.strategy == info.shape ? 0 : 1;
+    next[e.cls].alt = e.strategy == info.shape ? 0 : e.strategy == info.alt ? 1 : 2;
     next[e.cls].chunk = e.chunk;
     next[e.cls].bpc = e.blocks_per_cu;
     touched[e.cls] = true;
@@ -1960,8 +1963,9 @@ extern "C" int lai_dev_autotune(lai_basis* b, const double* d_D, int flags, int 
     if ((rc = eval(best, dflt_ms)) != LAI_OK) break;
     best_ms = dflt_ms;
     tried.emplace_back(info.shape, default_cap(b, c, info.shape, info.nt));
-    for (int alt = 0; alt <= (info.alt != kShapeNone ? 1 : 0) && rc == LAI_OK; ++alt) {
-      const int shape = alt ? info.alt : info.shape;
+    const int n_alt = info.alt2 != kShapeNone ? 2 : info.alt != kShapeNone ? 1 : 0;
+    for (int alt = 0; alt <= n_alt && rc == LAI_OK; ++alt) {
+      const int shape = alt == 2 ? info.alt2 : alt ? info.alt : info.shape;
       std::vector<int> caps;
       // lane-per-quartet classes: up to whole ket runs per chunk (fewer
       // exchange-row flushes, fewer workgroups)

@@ -86,7 +86,7 @@ void launch_class(const EriArgs& a0, hipStream_t s, const LaunchTune& t) {
   if (a.mode == 1) {  // raw ERIs, one launch over the quartet list
     if (MIXED || a.nq <= 0) return;
     const int max_blocks = t.n_cu * 16;  // grid-stride over the quartet list
-    if constexpr (P::regs) {
+    if constexpr (P::regs1) {
       int blocks = int(((long long)a.nq * a.lanes + 127) / 128);
       if (blocks > max_blocks) blocks = max_blocks;
       dim3 grid(blocks, P::NCH);
@@ -100,7 +100,7 @@ void launch_class(const EriArgs& a0, hipStream_t s, const LaunchTune& t) {
   // J/K digestion over the bra-anchored chunks
   if (a.nchunks <= 0) return;
   const size_t nbf = size_t(a.nbf);
-  const int shape = (t.alt && P::alt >= 0) ? P::alt : P::shape;
+  const int shape = (t.alt == 2 && P::alt2 >= 0) ? P::alt2 : (t.alt && P::alt >= 0) ? P::alt : P::shape;
   auto grid_cap = [&](int dflt) {
     const long long cap = (long long)t.n_cu * (t.blocks_per_cu > 0 ? t.blocks_per_cu : dflt);
     return int(a.nchunks < cap ? a.nchunks : cap);
@@ -175,7 +175,7 @@ void launch_class(const EriArgs& a0, hipStream_t s, const LaunchTune& t) {
                          dim3(64 * P::NW), 0, s, a);
     }
   } else {
-    if constexpr (!P::regs) {
+    if constexpr (!P::regs1) {
       a.klds = 0;
       hipLaunchKernelGGL((jk_kernel_lds<La, Lb, Lc, Ld, MIXED, P::NT>), dim3(grid_cap(kBlocksPerCuLds)),
                          dim3(P::NT), 0, s, a);
@@ -201,6 +201,7 @@ void fill(ClassLauncher* f64, ClassLauncher* f32, ClassInfo* info) {
     info[ID].waves = P::waves ? P::NW : 0;
     info[ID].shape = P::shape;
     info[ID].alt = P::alt;
+    info[ID].alt2 = P::alt2;
   }
   if constexpr (ID + 1 < kNumClasses) fill<ID + 1>(f64, f32, info);
 }

@@ -2021,8 +2021,22 @@ struct ClassPolicy {
   // of a 512-lane workgroup)
   static constexpr int CHA0 = rest >= 27 ? 1 : (27 / rest < na ? 27 / rest : na);
   static constexpr int NCH0 = (na + CHA0 - 1) / CHA0;
-  static constexpr bool regs = rest <= 27 && NCH0 <= 6;
-  static constexpr int CHA1 = regs && NCH0 > 1 ? (54 / rest < na ? 54 / rest : na) : CHA0;
+  static constexpr bool regs1 = rest <= 27 && NCH0 <= 6;
+  // classes whose bra goes into more than six slices of 27 but at most five of
+  // 60: (fp|pp), (fs|dp), (fp|ds), (fd|ps), (fp|fs).  A wavefront per quartet
+  // spends its time waiting for the tables that 12 or 15 of its lanes build
+  // and reads three LDS values for two products; ms so and in slices, four
+  // molecules / one molecule in cc-pVTZ: (fp|ds) 3.02 1.32 / 0.67 0.39,
+  // (fd|ps) 2.25 1.42 / 0.90 0.47, (fs|dp) 2.20 1.59 / 0.69 0.45, (fp|pp) 1.91
+  // 1.24 / 1.02 0.52, (fp|fs) 1.50 1.09 / 0.64 0.49.  Not (ff|ps), 1.01 0.89 /
+  // 0.40 0.51 (longer chains, fewer quartets), nor the d bras of this size,
+  // (dp|dp) 1.85 1.19 / 0.52 0.56, which lose on small molecules.
+  static constexpr bool regs2 = !regs1 && La == 3 && Lb < 3 && rest <= 30;
+  static constexpr bool regs = regs1 || regs2;
+  static constexpr int CHA1 = regs && NCH0 > 1 ? (60 / rest < na && rest > 27 ? 60 / rest
+                                                  : 54 / rest < na            ? 54 / rest
+                                                                              : na)
+                                               : CHA0;
   static constexpr int NCH = (na + CHA1 - 1) / CHA1;
   // the bra components spread evenly over the slices (a group of slice
   // wavefronts finishes with its largest slice)
@@ -2043,6 +2057,8 @@ struct ClassPolicy {
   // wavefront classes a workgroup per quartet
   static constexpr int alt =
       (regs && NCH >= 2 && LdsTasks<La, Lb, Lc, Ld>::NTASK <= 6 * 64) ? 1 : (waves ? 2 : -1);
+  // a third one, that tables saved for a wavefront class may name
+  static constexpr int alt2 = regs2 ? 2 : -1;
 };
 
 }  // namespace lai

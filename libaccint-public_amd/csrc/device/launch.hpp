@@ -37,6 +37,7 @@ struct ClassInfo {
   int waves;   // LDS shape with one quartet per wavefront: wavefronts per workgroup, else 0
   int shape;   // primary shape (kShape*)
   int alt;     // alternative shape compiled for the autotuner, kShapeNone if none
+  int alt2;    // a second alternative, kShapeNone if none
 };
 
 #define LAI_NPARTS_FIXED 8
