@@ -612,8 +612,11 @@ def main():
         Jd = dJ.cpu().numpy()
         Jx, _ = engine.build_jk(D, opts)  # FP64 four-centre J
         ej_df, ej = 0.5 * float(np.sum(D * Jd)), 0.5 * float(np.sum(D * Jx))
-        b_bytes = float(n) * naux * n * 8.0
-        gemm_flops = 2.0 * n * naux * n * n
+        # the Coulomb pass reads the pairs b >= a of B; the exchange runs over the
+        # r columns of the factor of D (D is of rank n_occ), found on the device
+        b_bytes = 0.5 * n * (n + 1) * naux * 8.0
+        rank = int(np.linalg.matrix_rank(D))
+        gemm_flops = 2.0 * n * naux * n * rank
         # share of the exchange product's 64 x 80 tiles of K computed with a
         # symmetric D (tiles entirely below the diagonal are skipped)
         tm, tn = (128 if n >= 1024 else 64), 80
@@ -623,10 +626,10 @@ def main():
             "workload": "16-water cc-pVDZ (400 bf) / cc-pVDZ-RI (%d fitting functions), FP64 J+K from HBM-resident B"
                         % naux,
             "init_seconds": init_s, "jk_ms": df_ms,
-            # J and K together: gamma_P = sum_a (B_P D)_aa from the diagonal of X
-            "kernels_ms": {"gamma_from_X_diagonal": km[0], "coulomb_pass": km[1], "gemm_X_eq_BD": km[2],
-                           "gemm_K_eq_XBt_slices": km[3], "slice_sum": km[4]},
-            "density_symmetric": True,
+            # one after another on one stream; X = B L includes the factorisation D = L L^T
+            "kernels_ms": {"gamma_pass": km[0], "coulomb_pass": km[1], "factor_and_gemm_X_eq_BL": km[2],
+                           "gemm_K_eq_XXt_slices": km[3], "slice_sum": km[4]},
+            "density_symmetric": True, "density_rank": rank,
             "roofline": {"gemm_X_tflops": gemm_flops / km[2] / 1e9,
                          "gemm_K_tflops_algorithmic": gemm_flops / km[3] / 1e9,
                          "gemm_K_tflops_executed": k_share * gemm_flops / km[3] / 1e9,
@@ -634,7 +637,8 @@ def main():
                          "gemm_peak_tflops": FP64_PEAK_TFLOPS,
                          "coulomb_pass_GBs": b_bytes / km[1] / 1e6,
                          "hbm_peak_GBs": 8000.0,
-                         "units": "gemm: 2 n^2 n_aux n flops each; Coulomb pass: one read of B (n^2 n_aux doubles)"},
+                         "units": "gemm: 2 n^2 n_aux r flops each (r: rank of D), X with the factorisation's time; Coulomb "
+                                  "pass: one read of the pairs b >= a of B"},
             "E_J_df_minus_exact": ej_df - ej}}
         log("DF J+K (16 waters, cc-pVDZ-RI): %.3f ms, init %.2f s; X %.1f TF/s, K %.1f TF/s executed" %
             (df_ms, init_s, gemm_flops / km[2] / 1e9, k_share * gemm_flops / km[3] / 1e9))
