@@ -1112,8 +1112,29 @@ int default_cap(const lai_basis* b, int c, int shape, int nt) {
   return default_chunk(shape, n, b->ctx->n_cu, nt);
 }
 
+void drop_graph(lai_basis* b) {
+  if (b->graph_exec) {
+    (void)hipGraphExecDestroy(b->graph_exec);
+    b->graph_exec = nullptr;
+  }
+  if (b->graph) {
+    (void)hipGraphDestroy(b->graph);
+    b->graph = nullptr;
+  }
+}
+
+// No list to run until one is whole again: chunks name pairs by their positions
+// in the list, so chunks, pair records, bounds and Coulomb offsets have to be
+// of one list, and a captured graph holds their addresses.
+void invalidate_worklist(lai_basis* b) {
+  b->have_worklist = false;
+  b->pitems_valid = false;
+  drop_graph(b);
+}
+
 // Chunks of class c under its launch choice (and, when that is not the
-// default, the default chunks for the gradient kernels) on the device.
+// default, the default chunks for the gradient kernels) on the device; none of
+// them after a failure.
 int upload_chunks(lai_basis* b, int c) {
   const auto& Ls = launchers();
   ClassList& C = b->cls[c];
@@ -1122,11 +1143,10 @@ int upload_chunks(lai_basis* b, int c) {
   const int cmax = t.chunk > 0 ? t.chunk : default_cap(b, c, shape, nt);
   const std::vector<JkChunk> ch = cut_runs(b, C, cmax, shape == kShapeRegs ? C.chain : 0);
   hipError_t e;
+  C.nchunks = C.ngchunks = 0;
+  C.gchunks.release();
   if ((e = C.chunks.assign(ch.data(), ch.size())) != hipSuccess)
     return fail(LAI_ERR_MEMORY, std::string("chunk upload: ") + hipGetErrorString(e));
-  C.nchunks = int64_t(ch.size());
-  C.gchunks.release();
-  C.ngchunks = 0;
   if (!t.is_default()) {
     const int dshape = Ls.info[c].shape;
     const std::vector<JkChunk> g =
@@ -1135,6 +1155,7 @@ int upload_chunks(lai_basis* b, int c) {
       return fail(LAI_ERR_MEMORY, std::string("chunk upload: ") + hipGetErrorString(e));
     C.ngchunks = int64_t(g.size());
   }
+  C.nchunks = int64_t(ch.size());
   return LAI_OK;
 }
 }  // namespace
@@ -1147,6 +1168,7 @@ extern "C" int lai_dev_build_worklist(lai_basis* b, double thr, const double* sh
     return fail(LAI_ERR_INVALID_STATE, "lai_dev_build_worklist: Schwarz bounds not computed");
   if (screen && density_screen && !shell_dmax)
     return fail(LAI_ERR_INVALID_ARGUMENT, "lai_dev_build_worklist: density screening needs shell_dmax");
+  invalidate_worklist(b);  // until every part of the new one is in place
   const int npairs = b->mol_pair.back();
   std::vector<double> Qp(npairs, 1.0);
   if (b->have_Q)
@@ -1374,15 +1396,6 @@ extern "C" int lai_dev_build_worklist(lai_basis* b, double thr, const double* sh
   b->n_fp32 = total32;
   b->checksum = sum;
   b->have_worklist = true;
-  b->pitems_valid = false;
-  if (b->graph_exec) {
-    (void)hipGraphExecDestroy(b->graph_exec);
-    b->graph_exec = nullptr;
-  }
-  if (b->graph) {
-    (void)hipGraphDestroy(b->graph);
-    b->graph = nullptr;
-  }
   if (n_out) *n_out = total;
   if (n32_out) *n32_out = total32;
   if (checksum) *checksum = sum;
@@ -1796,17 +1809,6 @@ extern "C" int lai_dev_jk_grad(lai_basis* b, const double* d_D, double xscale, d
 // autotuner and dispatch table
 // ---------------------------------------------------------------------------
 namespace {
-void drop_graph(lai_basis* b) {
-  if (b->graph_exec) {
-    (void)hipGraphExecDestroy(b->graph_exec);
-    b->graph_exec = nullptr;
-  }
-  if (b->graph) {
-    (void)hipGraphDestroy(b->graph);
-    b->graph = nullptr;
-  }
-}
-
 lai_class_tune tune_entry(const lai_basis* b, int c) {
   lai_class_tune e{};
   e.cls = c;
@@ -1872,7 +1874,10 @@ extern "C" int lai_dev_set_tuning(lai_basis* b, const lai_class_tune* table, int
     b->tune[c] = next[c];
     if (b->have_worklist) {
       const int rc = upload_chunks(b, c);
-      if (rc != LAI_OK) return rc;
+      if (rc != LAI_OK) {  // a class without its chunks
+        invalidate_worklist(b);
+        return rc;
+      }
     }
   }
   drop_graph(b);
@@ -2021,7 +2026,7 @@ extern "C" int lai_dev_autotune(lai_basis* b, const double* d_D, int flags, int 
   }
   if (rc != LAI_OK && failed_class >= 0) {  // leave the failing class as it was
     b->tune[failed_class] = failed_saved;
-    (void)upload_chunks(b, failed_class);
+    if (upload_chunks(b, failed_class) != LAI_OK) invalidate_worklist(b);
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);

@@ -86,7 +86,9 @@ std::vector<Real> BatchEngine::shell_dmax(const Real* D) const {
 WorklistInfo BatchEngine::prepare_worklist(const JKOptions& o, const Real* D_host) {
     lai_basis* h = device_handle();
     const bool need_d = (o.density_weighted && o.schwarz_threshold > 0.0) || o.mixed_precision;
-    const bool same_opts = wl_valid_ && wl_opts_.schwarz_threshold == o.schwarz_threshold &&
+    // (a rebuild or a tuning that failed leaves the handle without a list)
+    const bool have = wl_valid_ && lai_dev_worklist_stats(h, nullptr, nullptr, nullptr, nullptr) == LAI_OK;
+    const bool same_opts = have && wl_opts_.schwarz_threshold == o.schwarz_threshold &&
                            wl_opts_.density_weighted == o.density_weighted &&
                            wl_opts_.mixed_precision == o.mixed_precision && wl_opts_.fp32_threshold == o.fp32_threshold;
     if (same_opts && (!need_d || !D_host)) return wl_info_;

@@ -342,7 +342,9 @@ std::vector<Real> Engine::shell_dmax(const Real* D) const {
 WorklistInfo Engine::prepare_worklist(const JKOptions& o, const Real* D_host) {
     lai_basis* b = device_basis();
     const bool need_d = (o.density_weighted && o.schwarz_threshold > 0.0) || o.mixed_precision;
-    const bool same_opts = wl_valid_ && wl_opts_.schwarz_threshold == o.schwarz_threshold &&
+    // (a rebuild or a tuning that failed leaves the handle without a list)
+    const bool have = wl_valid_ && lai_dev_worklist_stats(b, nullptr, nullptr, nullptr, nullptr) == LAI_OK;
+    const bool same_opts = have && wl_opts_.schwarz_threshold == o.schwarz_threshold &&
                            wl_opts_.density_weighted == o.density_weighted &&
                            wl_opts_.mixed_precision == o.mixed_precision && wl_opts_.fp32_threshold == o.fp32_threshold;
     // no density given: a worklist built for the same options is reused as is
@@ -505,6 +507,8 @@ std::vector<Real> Engine::compute_jk_gradient(const Real* D, Real exchange_scale
     const Size n = basis_->n_basis_functions();
     // the gradient uses every canonical quartet that the current options keep
     if (!wl_valid_) prepare_worklist(JKOptions{}, D);
+    else if (lai_dev_worklist_stats(device_basis(), nullptr, nullptr, nullptr, nullptr) != LAI_OK)
+        prepare_worklist(wl_opts_, D);
     device::DeviceArray dD(n * n), dG(3 * static_cast<Size>(std::max(n_atoms, 1)));
     dD.upload(D, n * n);
     dG.zero();
