@@ -363,10 +363,19 @@ int lai_dev_df_dims(const lai_df* df, int* n_orb, int* n_aux);
  * diagonal and copies the lower triangle of K from the upper one.  A D that is
  * also positive semidefinite of rank at most n_orb/2, as the density of
  * occupied orbitals is, is factored on the device and the exchange runs over
- * the factor's columns (D is reproduced to 7e-15 of its largest diagonal
- * element, else the general products run) */
+ * the factor's columns (L L^T differs from D by at most 8.9e-16 of its norm,
+ * else the general products run) */
 #define LAI_DF_SYMMETRIC 4
 int lai_dev_df_jk(lai_df* df, const double* d_D, double* d_J, double* d_K, int flags, void* stream);
+/* Which of the two the last such build took: accepted 1 (the factor's columns,
+ * rank of them), 0 (the general products), -1 if this handle factors no
+ * density.  Waits for the device.  No reference counterpart (measurement). */
+int lai_dev_df_factor_info(const lai_df* df, int* accepted, int* rank);
+/* That factorisation alone: the n x n symmetric d_D (2 to 2048 rows) into d_L,
+ * (n/2) x n, row k column k of L; residual is the norm of D - L L^T over that
+ * of D (Frobenius), as far as it was computed.  Synchronous.  No reference
+ * counterpart (measurement). */
+int lai_dev_df_factor(const double* d_D, int n, double* d_L, int* accepted, int* rank, double* residual);
 /* as lai_dev_df_jk, synchronous, with each kernel timed by HIP events on
  * stream: ms[0] the fitted density gamma (a pass over B for J alone and for a
  * D that is factored; with J and K together otherwise the diagonal of X:

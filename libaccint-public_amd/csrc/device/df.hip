@@ -16,9 +16,14 @@
 // index n_aux n, split into slices that are summed by a last kernel).
 // A symmetric D that is positive semidefinite of low rank, as the density of
 // occupied orbitals is, is factored first (df_factor, D = L L^T with r
-// columns, checked against D): then X = B L has r columns instead of n and
-// K[a][c] = sum_(P,i) X[a][P][i] X[c][P][i], r/n of the work (16 waters / cc-pVDZ, n 400, r 80:
-// 7.5 -> 2.1 ms; X = B L 0.6, K 0.55 and df_factor 0.62 ms are what is left).
+// columns, corrected and checked against D): then X = B L has r columns instead
+// of n and K[a][c] = sum_(P,i) X[a][P][i] X[c][P][i], r/n of the work (16 waters
+// / cc-pVDZ, n 400, r 80: 7.6 -> 2.3 ms; X = B L 0.86, K 0.58, df_factor 0.35
+// and its correction 0.3 to 0.4 ms are what is left).  Relative error of K (long
+// double, B as it is), general products and factored, 225 / 300 / 400
+// functions, in 1e-16: localised orbitals 5.9 8.2 10.2 and 5.6 7.5 9.0,
+// delocalised 5.8 7.2 9.3 and 5.8 7.3 8.2, graded 6.9 7.9 10.4 and 6.2 6.1
+// 10.5; without the correction 5.8 4.8 10.0, 9.2 11.0 12.3 and 18.7 29.8 33.6.
 // The device decides (Factor::ok); the launches of the other form return at
 // once.
 #include "lai_device.h"
@@ -65,24 +70,36 @@ constexpr int ncart_of(int L) { return (L + 1) * (L + 2) / 2; }
 typedef double v4d __attribute__((ext_vector_type(4)));
 constexpr int KT = 16;  // summation step
 
-// What df_factor and df_check found out about a density.
+// What the factorisation of a density found out (factor_density).
 struct Factor {
   int ok;    // 1: D = L L^T to rounding, rank columns
   int rank;
   double dmax;  // largest diagonal element of D
-  int low;      // 1 once ok is final and 1: the general product under way may end
+  double e2, d2;  // ||D - L L^T||^2 and ||D||^2 (Frobenius) over dmax^2
+  int low;      // 1 once pivoting has ended well: the general product under way may end
 };
-// Rounding bound of the factorisation, relative to dmax: columns are taken
-// while a diagonal element of D - L L^T exceeds half of it, and every element
-// of D - L L^T has to lie within it.  (r terms of size at most dmax are
-// subtracted from each element: their rounding is about sqrt(r) 1e-16 dmax.)
-constexpr double kFactorTol = 32 * 2.220446049250313e-16;
+constexpr double kEps = 2.220446049250313e-16;
+// df_factor takes columns while a diagonal element of D - L L^T exceeds half of
+// this, relative to dmax, and refuses a D of which one falls below minus this:
+// what is left of a D of rank r after r pivots is D's own rounding, amplified by
+// the pivots, which grows with n (random columns, n/5 of them, eps of dmax: 10
+// at 225, 15 at 400, 22 at 800).
+__host__ __device__ constexpr double factor_tol(int n) { return 32 * kEps * (n > 300 ? n / 300.0 : 1.0); }
+// Bound of the corrected factor: ||D - L L^T|| <= kResidTol ||D||.  The
+// exchange averages over D - L L^T: at 225 to 400 functions the relative error
+// of K from it is a quarter of this or less, at most one eps, where the rounding
+// of the general products gives K 2.5 to 4.5 eps.
+constexpr double kResidTol = 4 * kEps;
+
+// which sizes of a product are the rank (GemmArgs::low)
+enum : int { kRankM = 1, kRankN = 2, kRankK = 4, kRankLda = 8, kRankLdb = 16, kRankLdc = 32, kRankSlices = 64 };
 
 struct GemmArgs {
   const Factor* fac;  // null: run; else run only when fac->ok == want
-  int want;           // (-1: beside the factorisation, workgroups begin until fac->low)
-  // with fac and want = 1, sizes from the rank r: 1: N = ldc = r (X = B L); 2:
-  // K = lda = ldb = naux r in kslices slices (K = X X^T)
+  int want;           // (-1: beside the factorisation, workgroups begin until fac->low;
+                      // -2: what -1 began for a D that is refused after fac->low)
+  // with fac and want = 1, the sizes that are the rank r (kRank*);
+  // kRankSlices: K = lda = ldb = naux r in kslices slices (K = X X^T)
   int low, naux, kslices;
   const double* A;
   const double* B;
@@ -104,18 +121,21 @@ struct GemmArgs {
 template <int BM, int BN>
 __global__ __launch_bounds__(256) void dgemm_mfma(GemmArgs g) {
   if (g.fac) {  // uniform over the grid
-    if (g.want < 0) {  // one answer for the workgroup: low may be set meanwhile
+    if (g.want == -1) {  // one answer for the workgroup: low may be set meanwhile
       __shared__ int low;
       if (threadIdx.x == 0) low = __hip_atomic_load(&g.fac->low, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __syncthreads();
       if (low) return;
-    } else if (g.fac->ok != g.want)
+    } else if (g.want == -2 ? (g.fac->ok || !g.fac->low) : g.fac->ok != g.want)
       return;
     const int r = g.fac->rank;
-    if (g.low == 1) {
-      g.N = r;
-      g.ldc = r;
-    } else if (g.low == 2) {
+    if (g.low & kRankM) g.M = r;
+    if (g.low & kRankN) g.N = r;
+    if (g.low & kRankK) g.K = r;
+    if (g.low & kRankLda) g.lda = r;
+    if (g.low & kRankLdb) g.ldb = r;
+    if (g.low & kRankLdc) g.ldc = r;
+    if (g.low & kRankSlices) {
       g.K = g.naux * r;
       g.lda = g.ldb = g.K;
       g.kchunk = ((g.K + g.kslices - 1) / g.kslices + KT - 1) / KT * KT;
@@ -147,7 +167,7 @@ __global__ __launch_bounds__(256) void dgemm_mfma(GemmArgs g) {
     }
   }
   const int m0 = mi * TM, n0 = ni * TN;
-  if (n0 >= g.N) return;  // column tiles beyond the rank
+  if (m0 >= g.M || n0 >= g.N) return;  // tiles beyond the rank
   if (g.skip_lower && m0 > n0 + TN - 1) return;  // uniform over the workgroup, before any barrier
   const double* A = g.A;
   const double* B = g.B;
@@ -375,9 +395,9 @@ __global__ __launch_bounds__(256) void df_coulomb(const double* __restrict__ B, 
 }
 
 // ---------------------------------------------------------------------------
-// D = L L^T by pivoted Cholesky in one workgroup: Lc[k][i] holds column k.
-// Columns are taken while the largest diagonal element of D - L L^T exceeds
-// kFactorTol/2 times the largest of D, at most rmax; any order of pivots gives
+// D = L L^T by pivoted Cholesky in one workgroup: Lc[k][i] holds column k,
+// Lh[k][i] the column over its pivot element dk[k].  Columns are taken while the largest diagonal element of D - L L^T exceeds
+// factor_tol/2 times the largest of D, at most rmax; any order of pivots gives
 // a semidefinite D of rank r in r columns.  They are taken in panels: up to
 // kPanel rows whose diagonal element is at least half of the largest are the
 // candidates, their columns of D - L L^T are formed in registers (a lane per
@@ -386,21 +406,21 @@ __global__ __launch_bounds__(256) void df_coulomb(const double* __restrict__ B, 
 // below a quarter.  (Random D of rank 81 in 200: residual 11 eps; with a tenth
 // and a hundredth instead 125 eps in as many panels, since small pivots amplify
 // the rounding of the earlier ones.)  A step is bound by latency (two barriers and
-// a few LDS reads): 0.62 ms for 80 columns of 400; each column formed by itself
-// took 0.86 ms.
+// a few LDS reads): 0.35 ms for 80 columns of 400.
 // RP rows per lane: n at most RP kFactorNT.
 // ---------------------------------------------------------------------------
 // From kFactorMinN functions on: J and K in ms without and with the factor, and
 // for a D that is refused (indefinite or of full rank), water / cc-pVDZ:
-//   100: 0.144 0.151   150: 0.343 0.353   200: 0.863 0.637 refused 0.98
-//   250: 1.82  0.99 refused 1.90   300: 3.07 1.48 refused 3.27
-//   400: 7.53  2.14 refused 7.74   600: 53.8 16.0
+//   225: 1.13 0.93 refused 1.28   250: 1.82 1.10 refused 1.95
+//   300: 3.08 1.64 refused 3.32   400: 7.6  2.34 refused 8.0
+//   600: 42.9 17.0 refused 43.9
 // (the step from 400 to 600 is B, 2.2 GB, outgrowing the cache).  Up to
 // kFactorMaxN rows stay in registers.
 constexpr int kFactorMaxN = 2048, kFactorMinN = 224, kFactorNT = 1024, kPanel = 16, kPanelK = 32;
 template <int RP>
 __global__ __launch_bounds__(kFactorNT) void df_factor(const double* __restrict__ D, int n, int rmax,
-                                                       double* __restrict__ Lc, Factor* __restrict__ fac) {
+                                                       double* __restrict__ Lc, double* __restrict__ Lh,
+                                                       double* __restrict__ dk, Factor* __restrict__ fac) {
   __shared__ double prow[kPanelK][kPanel];  // L[candidate][k] of a block of earlier columns
   __shared__ double pd[kPanel];             // diagonal elements of the candidates
   __shared__ double prw[kPanel];            // the pivot row of the panel
@@ -416,9 +436,10 @@ __global__ __launch_bounds__(kFactorNT) void df_factor(const double* __restrict_
     open[q] = i < n;
     diag[q] = open[q] ? D[(long long)i * n + i] : 0.0;
   }
+  const double eps = factor_tol(n);
   double dmax = -1.0;
   int k = 0;
-  bool low = true;
+  bool low = true, full = false;
   for (;;) {
     // largest diagonal element
     double m = -1.0;
@@ -433,19 +454,19 @@ __global__ __launch_bounds__(kFactorNT) void df_factor(const double* __restrict_
     for (int w = 0; w < kFactorNT / 64; ++w) m = fmax(m, wv[w]);
     if (dmax < 0.0) dmax = m;
     // (also ends where dmax is not a positive number)
-    if (!(m > 0.5 * kFactorTol * dmax) || !(dmax > 0.0)) break;
+    if (!(m > 0.5 * eps * dmax) || !(dmax > 0.0)) break;
     // a negative diagonal element: indefinite (a difference of densities ends
     // here, at the first panel or soon after)
     bool neg = false;
 #pragma unroll
-    for (int q = 0; q < RP; ++q) neg |= open[q] && diag[q] < -kFactorTol * dmax;
+    for (int q = 0; q < RP; ++q) neg |= open[q] && diag[q] < -eps * dmax;
     if (__syncthreads_or(neg)) {
       low = false;
       break;
     }
     // candidates, in row order: each of them may become a pivot, so every panel
     // takes at least one column and the loop ends after at most rmax panels
-    const double tol = 0.5 * kFactorTol * dmax;
+    const double tol = 0.5 * eps * dmax;
     const int k_panel = k;
     int nc = 0;
     for (int q = 0; q < RP; ++q) {
@@ -510,8 +531,9 @@ __global__ __launch_bounds__(kFactorNT) void df_factor(const double* __restrict_
         }
       }
       if (!(v > floor_v)) break;  // uniform: every lane read the same values
-      if (k == rmax) {
-        low = false;
+      if (k == rmax) {  // (rounding left of a D of rank rmax: the residual decides)
+        low = v <= 4.0 * eps * dmax;
+        full = true;
         break;
       }
       const int at = cand[best];
@@ -539,42 +561,85 @@ __global__ __launch_bounds__(kFactorNT) void df_factor(const double* __restrict_
         } else if (!open[q]) {
           x = 0.0;
         }
-        if (i < n) Lc[(long long)k * n + i] = x;
+        if (i < n) {
+          Lc[(long long)k * n + i] = x;
+          Lh[(long long)k * n + i] = x * inv;
+        }
         diag[q] -= x * x;
 #pragma unroll
         for (int p = 0; p < kPanel; ++p) c[q][p] = fma(-x, rp[p], c[q][p]);
       }
       if (tid < kPanel) pd[tid] -= prw[tid] * prw[tid] / v;
+      if (tid == 0) dk[k] = v * inv;
       left &= ~(1u << best);
       ++k;
       __syncthreads();  // pd is updated, prw is read
     }
     __syncthreads();  // every lane has read pd before the next panel
-    if (!low || k == k_panel) break;  // (no column: a diagonal element that is not finite)
+    if (full || k == k_panel) break;  // (no column: a diagonal element that is not finite)
   }
   if (tid == 0) {
     fac->ok = low && dmax > 0.0 && dmax < HUGE_VAL ? 1 : 0;
     fac->rank = k;
     fac->dmax = dmax;
+    fac->e2 = 0.0;
+    fac->d2 = 0.0;
+    // (the general product ends here, not after the correction, whose small
+    // kernels would wait for its workgroups: 400 functions 2.59 -> 2.34 ms)
+    __hip_atomic_store(&fac->low, fac->ok, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
-// Clears fac->ok where an element of D - L L^T exceeds kFactorTol dmax (an
-// indefinite D, or one that df_factor did not bring to rounding).  64 x 64
-// elements per workgroup, 4 x 4 per lane, columns of L through LDS.
-__global__ __launch_bounds__(256) void df_check(const double* __restrict__ D, const double* __restrict__ Lc, int n,
-                                                Factor* fac) {
-  // (ok may be cleared meanwhile: then nothing is lost)
-  if (!__hip_atomic_load(&fac->ok, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) || blockIdx.x < blockIdx.y) return;
+// ---------------------------------------------------------------------------
+// Correction of the factor.  What pivoting leaves of D is small on the pivot
+// rows and holds D's own rounding, amplified, everywhere else: 4 to 20 eps of
+// ||D|| at 400 functions, 40 at 800, whatever precision the pivoting runs in,
+// and K inherits it (relative error of K, 400 functions, graded orbital sizes:
+// 3.4e-15, the general products 1.0e-15).  The nearest L L^T of the same rank
+// takes E = D - L L^T to first order to (1 - P) E (1 - P), P the projection on
+// the columns of L:
+//   L += E Z - L (Z^T E Z) / 2,  Z = L (L^T L)^-1,
+// with E summed in two doubles (df_resid).  Computed with the columns scaled
+// to pivots of one (Lh), whose L^T L has a condition of 10 to 1e3; two digits
+// of the correction are enough.  One step brings ||E|| to 0.8-2 eps of ||D||
+// up to 400 functions; where the pivots took columns of D's rounding as well
+// the second order counts and a second step is needed (800 functions: 4 and
+// 8 eps after one, 1.7 and 2.7 after two).
+// ---------------------------------------------------------------------------
+// hi + lo -= a b, the product and the sum exact
+__device__ __forceinline__ void sub_product(double& hi, double& lo, double a, double b) {
+#pragma clang fp contract(off)
+  const double p = a * b, e = __builtin_fma(a, b, -p);
+  const double t = hi - p, v = t - hi;
+  const double err = (hi - (t - v)) - (p + v);
+  hi = t;
+  lo += err - e;
+}
+
+// E = D - L L^T (D's upper triangle, both of E), or with LAST its norm and D's
+// into fac.  32 x 32 elements per workgroup, 2 x 2 per lane, columns of L
+// through LDS; 15 operations a term, 5 us of 400 functions and 80 columns.
+template <bool LAST>
+__global__ __launch_bounds__(256) void df_resid(const double* __restrict__ D, const double* __restrict__ Lc, int n,
+                                                double* __restrict__ E, Factor* fac) {
+  if (!fac->ok || blockIdx.x < blockIdx.y) return;
   constexpr int KB = 16;
-  __shared__ double La[KB][64], Lb[KB][64];
+  __shared__ double La[KB][32], Lb[KB][32];
   const int tid = threadIdx.x, ti = tid / 16, tj = tid % 16;
-  const int i0 = blockIdx.y * 64, j0 = blockIdx.x * 64, r = fac->rank;
-  const double bound = kFactorTol * fac->dmax;
-  double acc[4][4] = {};
+  const int i0 = blockIdx.y * 32, j0 = blockIdx.x * 32, r = fac->rank;
+  double hi[2][2], lo[2][2], d[2][2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int y = 0; y < 2; ++y) {
+      const int i = i0 + ti + 16 * x, j = j0 + tj + 16 * y;
+      d[x][y] = i < n && j < n ? D[(long long)min(i, j) * n + max(i, j)] : 0.0;
+      hi[x][y] = d[x][y];
+      lo[x][y] = 0.0;
+    }
   for (int k0 = 0; k0 < r; k0 += KB) {
-    for (int e = tid; e < KB * 64; e += 256) {
-      const int k = e / 64, i = e - k * 64;
+    for (int e = tid; e < KB * 32; e += 256) {
+      const int k = e / 32, i = e - k * 32;
       La[k][i] = k0 + k < r && i0 + i < n ? Lc[(long long)(k0 + k) * n + i0 + i] : 0.0;
       Lb[k][i] = k0 + k < r && j0 + i < n ? Lc[(long long)(k0 + k) * n + j0 + i] : 0.0;
     }
@@ -582,24 +647,141 @@ __global__ __launch_bounds__(256) void df_check(const double* __restrict__ D, co
 #pragma unroll
     for (int k = 0; k < KB; ++k)
 #pragma unroll
-      for (int x = 0; x < 4; ++x)
+      for (int x = 0; x < 2; ++x)
 #pragma unroll
-        for (int y = 0; y < 4; ++y) acc[x][y] = fma(La[k][ti + 16 * x], Lb[k][tj + 16 * y], acc[x][y]);
+        for (int y = 0; y < 2; ++y) sub_product(hi[x][y], lo[x][y], La[k][ti + 16 * x], Lb[k][tj + 16 * y]);
     __syncthreads();
   }
-  bool bad = false;
+  double e2 = 0.0, d2 = 0.0;
+  const double inv = 1.0 / fac->dmax;
 #pragma unroll
-  for (int x = 0; x < 4; ++x)
+  for (int x = 0; x < 2; ++x)
 #pragma unroll
-    for (int y = 0; y < 4; ++y) {
+    for (int y = 0; y < 2; ++y) {
       const int i = i0 + ti + 16 * x, j = j0 + tj + 16 * y;
-      if (i < n && j < n && !(fabs(D[(long long)i * n + j] - acc[x][y]) <= bound)) bad = true;
+      if (i >= n || j >= n) continue;
+      const double v = hi[x][y] + lo[x][y];
+      if constexpr (LAST) {  // (tiles on the diagonal hold both triangles)
+        const double w = i0 == j0 ? 1.0 : 2.0, ev = v * inv, dv = d[x][y] * inv;
+        e2 += w * ev * ev;
+        d2 += w * dv * dv;
+      } else {
+        E[(long long)i * n + j] = v;
+        E[(long long)j * n + i] = v;
+      }
     }
-  if (bad) atomicAnd(&fac->ok, 0);
+  if constexpr (LAST) {
+    e2 = wave_sum(e2);
+    d2 = wave_sum(d2);
+    if ((tid & 63) == 0) {
+      __hip_atomic_fetch_add(&fac->e2, e2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_fetch_add(&fac->d2, d2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
 }
 
-__global__ void df_set_low(Factor* fac, int decided) {
-  __hip_atomic_store(&fac->low, decided ? fac->ok : 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+// G = G^-1 in place (r x r, symmetric positive definite: Gauss-Jordan without
+// pivoting) in one workgroup.  Up to 128 columns a lane holds 4 x 4 elements
+// and a step costs one barrier; beyond, the matrix stays in the cache, two
+// barriers and a pass over it a step.
+constexpr int kInvReg = 128;
+__global__ __launch_bounds__(1024) void df_invert(double* G, const Factor* __restrict__ fac) {
+  if (!fac->ok) return;
+  const int r = fac->rank, tid = threadIdx.x, ty = tid >> 5, tx = tid & 31;
+  if (r <= kInvReg) {
+    __shared__ double col[2][kInvReg], row[2][kInvReg];
+    double A[4][4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const int i = ty + 32 * a, j = tx + 32 * b;
+        A[a][b] = i < r && j < r ? G[i * r + j] : 0.0;
+      }
+    for (int k = 0; k < r; ++k) {
+      const int u = k & 1;
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        if (tx + 32 * m == k)
+#pragma unroll
+          for (int a = 0; a < 4; ++a) col[u][ty + 32 * a] = A[a][m];
+        if (ty + 32 * m == k)
+#pragma unroll
+          for (int b = 0; b < 4; ++b) row[u][tx + 32 * b] = A[m][b];
+      }
+      __syncthreads();  // (the other buffer was read before this)
+      const double p = 1.0 / row[u][k];
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        const int i = ty + 32 * a;
+        const double c = col[u][i];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+          const int j = tx + 32 * b;
+          const double x = row[u][j] * p;
+          A[a][b] = i == k ? (j == k ? p : x) : j == k ? -c * p : fma(-c, x, A[a][b]);
+        }
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const int i = ty + 32 * a, j = tx + 32 * b;
+        if (i < r && j < r) G[i * r + j] = A[a][b];
+      }
+  } else {
+    __shared__ double col[kFactorMaxN / 2], row[kFactorMaxN / 2];
+    for (int k = 0; k < r; ++k) {
+      if (tid < r) {
+        col[tid] = G[(long long)tid * r + k];
+        row[tid] = G[(long long)k * r + tid];
+      }
+      __syncthreads();
+      const double p = 1.0 / row[k];
+      for (int i = ty; i < r; i += 32) {
+        const double c = col[i];
+        double* Gi = G + (long long)i * r;
+        for (int j = tx; j < r; j += 32) {
+          const double x = row[j] * p;
+          Gi[j] = i == k ? (j == k ? p : x) : j == k ? -c * p : fma(-c, x, Gi[j]);
+        }
+      }
+      __syncthreads();
+    }
+  }
+}
+
+// L += (F - Lh H / 2) / dk by columns: 64 rows i by 16 columns k per workgroup.
+__global__ __launch_bounds__(256) void df_update(const double* __restrict__ Lh, const double* __restrict__ F,
+                                                 const double* __restrict__ H, const double* __restrict__ dk, int n,
+                                                 double* __restrict__ Lc, const Factor* __restrict__ fac) {
+  if (!fac->ok) return;
+  const int r = fac->rank, i = blockIdx.x * 64 + (threadIdx.x & 63);
+  const int k0 = blockIdx.y * 16 + 4 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (i >= n || k0 >= r) return;
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int l = 0; l < r; ++l) {
+    const double v = Lh[(long long)l * n + i];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) s[q] = fma(H[(long long)min(k0 + q, r - 1) * r + l], v, s[q]);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int k = k0 + q;
+    if (k >= r) break;
+    const long long at = (long long)k * n + i;
+    Lc[at] += (F[at] - 0.5 * s[q]) / dk[k];
+  }
+}
+
+// Before a factorisation: the general product may begin.
+__global__ void df_open(Factor* fac) {
+  __hip_atomic_store(&fac->low, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// After it: the decision.  (An e2 that is not finite refuses.)
+__global__ void df_decide(Factor* fac) {
+  if (!(fac->e2 < HUGE_VAL && fac->e2 <= kResidTol * kResidTol * fac->d2)) fac->ok = 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -679,6 +861,78 @@ int gemm(const GemmArgs& g0, int gz, hipStream_t st) {
   return LAI_OK;
 }
 
+// Memory of a factorisation: factor_doubles(n) doubles at one address.
+struct FactorBufs {
+  double *Lc, *Lh, *Z, *F;  // [rmax][n]: L, its scaled columns, Z and E Z
+  double* E;                // [n][n]
+  double *G, *H;            // [rmax][rmax]
+  double* dk;               // [rmax]
+  int rmax;
+  FactorBufs(double* p, int n) : rmax(n / 2) {
+    const size_t rn = size_t(rmax) * n, rr = size_t(rmax) * rmax;
+    Lc = p;
+    Lh = Lc + rn;
+    Z = Lh + rn;
+    F = Z + rn;
+    E = F + rn;
+    G = E + size_t(n) * n;
+    H = G + rr;
+    dk = H + rr;
+  }
+};
+size_t factor_doubles(int n) {
+  const size_t r = size_t(n / 2);
+  return 4 * r * n + size_t(n) * n + 2 * r * r + r;
+}
+
+// Factors D into f.Lc and decides (fac->ok), all on st.
+int factor_density(const double* D, int n, const FactorBufs& f, Factor* fac, hipStream_t st) {
+  if (n <= kFactorNT)
+    hipLaunchKernelGGL(df_factor<1>, dim3(1), dim3(kFactorNT), 0, st, D, n, f.rmax, f.Lc, f.Lh, f.dk, fac);
+  else
+    hipLaunchKernelGGL(df_factor<2>, dim3(1), dim3(kFactorNT), 0, st, D, n, f.rmax, f.Lc, f.Lh, f.dk, fac);
+  DF_HIP(hipGetLastError());
+  const unsigned t = unsigned((n + 31) / 32);
+  // C = A B or A B^T with the given sizes of the rank
+  auto mul = [&](const double* A, const double* B, double* C, int M, int N, int K, int bt, int low) -> int {
+    GemmArgs g{};
+    g.fac = fac;
+    g.want = 1;
+    g.low = low;
+    g.A = A;
+    g.B = B;
+    g.C = C;
+    g.M = M;
+    g.N = N;
+    g.K = K;
+    g.lda = g.ldb = g.ldc = n;
+    g.bt = bt;
+    return gemm(g, 1, st);
+  };
+  const int r = f.rmax;
+  for (int step = 0; step < (n <= 512 ? 1 : 2); ++step) {
+    int rc;
+    hipLaunchKernelGGL(df_resid<false>, dim3(t, t), dim3(256), 0, st, D, f.Lc, n, f.E, fac);
+    DF_HIP(hipGetLastError());
+    if (step == 0) {  // G = (Lh^T Lh)^-1, Z (the projection hardly changes)
+      if ((rc = mul(f.Lh, f.Lh, f.G, r, r, n, 1, kRankM | kRankN | kRankLdc))) return rc;
+      hipLaunchKernelGGL(df_invert, dim3(1), dim3(1024), 0, st, f.G, fac);
+      DF_HIP(hipGetLastError());
+      if ((rc = mul(f.G, f.Lh, f.Z, r, n, r, 0, kRankM | kRankK | kRankLda))) return rc;
+    }
+    if ((rc = mul(f.Z, f.E, f.F, r, n, n, 0, kRankM))) return rc;
+    if ((rc = mul(f.Z, f.F, f.H, r, r, n, 1, kRankM | kRankN | kRankLdc))) return rc;
+    hipLaunchKernelGGL(df_update, dim3((n + 63) / 64, (r + 15) / 16), dim3(256), 0, st, f.Lh, f.F, f.H, f.dk, n, f.Lc,
+                       fac);
+    DF_HIP(hipGetLastError());
+  }
+  hipLaunchKernelGGL(df_resid<true>, dim3(t, t), dim3(256), 0, st, D, f.Lc, n, nullptr, fac);
+  DF_HIP(hipGetLastError());
+  hipLaunchKernelGGL(df_decide, dim3(1), dim3(1), 0, st, fac);
+  DF_HIP(hipGetLastError());
+  return LAI_OK;
+}
+
 // Lower Cholesky factor of the row-major SPD matrix A in place (upper part
 // zeroed): the row-oriented algorithm of math::cholesky_decompose
 // (include/libaccint/math/cholesky.hpp), which fails when a pivot is <= 0.
@@ -734,9 +988,8 @@ struct lai_df {
   double* gamma = nullptr;  // [naux]
   hipEvent_t ev[6] = {};
   bool have_ev = false;
-  double* Lc = nullptr;     // [rmax][n]: factor of the density, null where it is not tried
+  double* fbuf = nullptr;   // memory of the density's factor (FactorBufs), null where it is not tried
   Factor* fac = nullptr;
-  int rmax = 0;
   // the Coulomb passes run beside the exchange GEMMs on this stream
   hipStream_t side = nullptr;
   hipEvent_t fork = nullptr, join = nullptr;
@@ -750,7 +1003,7 @@ void df_release(lai_df* d) {
   if (d->part) (void)hipFree(d->part);
   if (d->gpart) (void)hipFree(d->gpart);
   if (d->gamma) (void)hipFree(d->gamma);
-  if (d->Lc) (void)hipFree(d->Lc);
+  if (d->fbuf) (void)hipFree(d->fbuf);
   if (d->fac) (void)hipFree(d->fac);
   if (d->side) (void)hipStreamDestroy(d->side);
   if (d->fork) (void)hipEventDestroy(d->fork);
@@ -998,12 +1251,12 @@ extern "C" int lai_dev_df_create(lai_basis* b, int n_orb_shells, int n_aux_shell
   if (n >= kFactorMinN && n <= kFactorMaxN) {
     Dev<double> dl;
     Dev<Factor> df;
-    if ((e = dl.alloc(size_t(n / 2) * n)) != hipSuccess || (e = df.alloc(1)) != hipSuccess) {
+    if ((e = dl.alloc(factor_doubles(n))) != hipSuccess || (e = df.alloc(1)) != hipSuccess ||
+        (e = hipMemset(df.p, 0, sizeof(Factor))) != hipSuccess) {
       df_release(d);
       return set_error(LAI_ERR_MEMORY, std::string("lai_dev_df_create: ") + hipGetErrorString(e));
     }
-    d->rmax = n / 2;
-    d->Lc = dl.take();
+    d->fbuf = dl.take();
     d->fac = df.take();
   }
   if ((e = hipStreamCreateWithFlags(&d->side, hipStreamNonBlocking)) != hipSuccess ||
@@ -1040,7 +1293,8 @@ int df_run(lai_df* d, const double* D, double* J, double* K, int flags, hipStrea
     for (int i = 0; i < 5; ++i) ms[i] = 0.0;
   const bool both = (flags & LAI_DF_J) && (flags & LAI_DF_K);
   const int sym = (flags & LAI_DF_SYMMETRIC) ? 1 : 0;
-  const bool factor = (flags & LAI_DF_K) && sym && d->Lc;  // the exchange from a factor of D, if there is one
+  const bool factor = (flags & LAI_DF_K) && sym && d->fbuf;  // the exchange from a factor of D, if there is one
+  const FactorBufs fb(d->fbuf, n);
   auto coulomb = [&](hipStream_t s) -> int {
     hipLaunchKernelGGL(df_coulomb, dim3((n + 63) / 64, n), dim3(256), 0, s, d->B, d->gamma, n, naux, J);
     DF_HIP(hipGetLastError());
@@ -1054,31 +1308,20 @@ int df_run(lai_df* d, const double* D, double* J, double* K, int flags, hipStrea
     DF_HIP(hipGetLastError());
     return LAI_OK;
   };
-  auto factor_density = [&]() -> int {
-    if (n <= kFactorNT)
-      hipLaunchKernelGGL(df_factor<1>, dim3(1), dim3(kFactorNT), 0, st, D, n, d->rmax, d->Lc, d->fac);
-    else
-      hipLaunchKernelGGL(df_factor<2>, dim3(1), dim3(kFactorNT), 0, st, D, n, d->rmax, d->Lc, d->fac);
-    DF_HIP(hipGetLastError());
-    const unsigned t = unsigned((n + 63) / 64);
-    hipLaunchKernelGGL(df_check, dim3(t, t), dim3(256), 0, st, D, d->Lc, n, d->fac);
-    DF_HIP(hipGetLastError());
-    return LAI_OK;
-  };
   auto x_low = [&]() -> int {  // X = B L
     GemmArgs g{};
     g.fac = d->fac;
     g.want = 1;
-    g.low = 1;
+    g.low = kRankN | kRankLdc;
     g.A = d->B;
-    g.B = d->Lc;  // given transposed: rows i, columns b
+    g.B = fb.Lc;  // given transposed: rows i, columns b
     g.bt = 1;
     g.C = d->X;
     g.lda = n;
     g.ldb = n;
     g.M = n * naux;
-    g.N = d->rmax;
-    g.ldc = d->rmax;
+    g.N = fb.rmax;
+    g.ldc = fb.rmax;
     g.K = n;
     g.xcd = 1;
     return gemm(g, 1, st);
@@ -1107,7 +1350,7 @@ int df_run(lai_df* d, const double* D, double* J, double* K, int flags, hipStrea
       GemmArgs h{};
       h.fac = d->fac;
       h.want = 1;
-      h.low = 2;
+      h.low = kRankSlices;
       h.naux = naux;
       h.kslices = nsym;
       h.A = d->X;
@@ -1173,20 +1416,18 @@ int df_run(lai_df* d, const double* D, double* J, double* K, int flags, hipStrea
     // until D is known to be of low rank.  A density that is refused so costs
     // the pass over B; with X = B D after the factorisation a full rank took
     // 1.23 ms instead of 0.86 at 200 functions, 8.2 instead of 7.5 at 400.
-    hipLaunchKernelGGL(df_set_low, dim3(1), dim3(1), 0, st, d->fac, 0);
+    hipLaunchKernelGGL(df_open, dim3(1), dim3(1), 0, st, d->fac);
     DF_HIP(hipGetLastError());
     DF_HIP(hipEventRecord(d->fork, st));
     DF_HIP(hipStreamWaitEvent(d->side, d->fork, 0));
     auto beside = [&]() -> int {
       int r;
-      if ((r = factor_density())) return r;
-      hipLaunchKernelGGL(df_set_low, dim3(1), dim3(1), 0, st, d->fac, 1);
-      DF_HIP(hipGetLastError());
+      if ((r = factor_density(D, n, fb, d->fac, st))) return r;
       if (both && ((r = gamma_pass(d->side)) || (r = coulomb(d->side)))) return r;
       return x_gemm(d->side, -1);
     };
     rc = beside();
-    if ((rc = join_side(rc)) || (rc = x_low())) return rc;
+    if ((rc = join_side(rc)) || (rc = x_gemm(st, -2)) || (rc = x_low())) return rc;
     return k_product();
   }
   if (both) {
@@ -1197,7 +1438,7 @@ int df_run(lai_df* d, const double* D, double* J, double* K, int flags, hipStrea
     const bool overlap = !ms && d->side;
     const hipStream_t sj = overlap ? d->side : st;
     if ((rc = mark(0))) return rc;
-    if (factor && ((rc = factor_density()) || (rc = x_low()))) return rc;
+    if (factor && ((rc = factor_density(D, n, fb, d->fac, st)) || (rc = x_low()))) return rc;
     if ((rc = x_gemm(st, 0))) return rc;
     if ((rc = mark(1))) return rc;
     if ((rc = take(0, 1, 2))) return rc;
@@ -1236,7 +1477,7 @@ int df_run(lai_df* d, const double* D, double* J, double* K, int flags, hipStrea
   }
   if (flags & LAI_DF_K) {
     if ((rc = mark(0))) return rc;
-    if (factor && ((rc = factor_density()) || (rc = x_low()))) return rc;
+    if (factor && ((rc = factor_density(D, n, fb, d->fac, st)) || (rc = x_low()))) return rc;
     if ((rc = x_gemm(st, 0))) return rc;
     if ((rc = mark(1))) return rc;
     if ((rc = take(0, 1, 2))) return rc;
@@ -1245,6 +1486,41 @@ int df_run(lai_df* d, const double* D, double* J, double* K, int flags, hipStrea
   return LAI_OK;
 }
 }  // namespace
+
+extern "C" int lai_dev_df_factor_info(const lai_df* df, int* accepted, int* rank) {
+  if (!df || !accepted || !rank)
+    return set_error(LAI_ERR_INVALID_ARGUMENT, "lai_dev_df_factor_info: invalid arguments");
+  Factor f{};
+  f.ok = -1;
+  if (df->fac) {
+    DF_HIP(hipDeviceSynchronize());
+    DF_HIP(hipMemcpy(&f, df->fac, sizeof(f), hipMemcpyDeviceToHost));
+  }
+  *accepted = f.ok;
+  *rank = f.rank;
+  return LAI_OK;
+}
+
+extern "C" int lai_dev_df_factor(const double* d_D, int n, double* d_L, int* accepted, int* rank, double* residual) {
+  if (!d_D || !d_L || !accepted || !rank || !residual || n < 2 || n > kFactorMaxN)
+    return set_error(LAI_ERR_INVALID_ARGUMENT, "lai_dev_df_factor: invalid arguments");
+  Dev<double> buf;
+  Dev<Factor> fac;
+  hipError_t e;
+  if ((e = buf.alloc(factor_doubles(n))) != hipSuccess || (e = fac.alloc(1)) != hipSuccess)
+    return set_error(LAI_ERR_MEMORY, std::string("lai_dev_df_factor: ") + hipGetErrorString(e));
+  const FactorBufs f(buf.p, n);
+  const int rc = factor_density(d_D, n, f, fac.p, nullptr);
+  DF_HIP(hipDeviceSynchronize());
+  if (rc != LAI_OK) return rc;
+  Factor h{};
+  DF_HIP(hipMemcpy(&h, fac.p, sizeof(h), hipMemcpyDeviceToHost));
+  DF_HIP(hipMemcpy(d_L, f.Lc, sizeof(double) * size_t(f.rmax) * n, hipMemcpyDeviceToDevice));
+  *accepted = h.ok;
+  *rank = h.rank;
+  *residual = std::sqrt(h.e2 / h.d2);
+  return LAI_OK;
+}
 
 extern "C" int lai_dev_df_jk(lai_df* df, const double* d_D, double* d_J, double* d_K, int flags, void* stream) {
   if (!df || !d_D || (flags & ~(LAI_DF_J | LAI_DF_K | LAI_DF_SYMMETRIC)) || ((flags & LAI_DF_J) && !d_J) ||

@@ -86,6 +86,8 @@ _SIGNATURES = {
     "lai_dev_df_free": ([_vp], ctypes.c_int),
     "lai_dev_df_dims": ([_vp, _ip, _ip], ctypes.c_int),
     "lai_dev_df_jk": ([_vp, _vp, _vp, _vp, ctypes.c_int, _vp], ctypes.c_int),
+    "lai_dev_df_factor_info": ([_vp, _ip, _ip], ctypes.c_int),
+    "lai_dev_df_factor": ([_vp, ctypes.c_int, _vp, _ip, _ip, _dp], ctypes.c_int),
     "lai_dev_df_jk_profile": ([_vp, _vp, _vp, _vp, ctypes.c_int, _vp, _dp], ctypes.c_int),
     "lai_dev_rys": ([ctypes.c_int, ctypes.c_int, _vp, _vp, _vp, _vp], ctypes.c_int),
     "lai_dev_boys": ([ctypes.c_int, ctypes.c_int, _vp, _vp, _vp], ctypes.c_int),
