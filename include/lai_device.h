@@ -377,10 +377,9 @@ int lai_dev_df_factor_info(const lai_df* df, int* accepted, int* rank);
  * counterpart (measurement). */
 int lai_dev_df_factor(const double* d_D, int n, double* d_L, int* accepted, int* rank, double* residual);
 /* as lai_dev_df_jk, synchronous, with each kernel timed by HIP events on
- * stream: ms[0] the fitted density gamma (a pass over B for J alone and for a
- * D that is factored; with J and K together otherwise the diagonal of X:
- * gamma_P = sum_a (B_P D)_aa), ms[1] the J pass, ms[2] the X = B D GEMM (or the
- * factorisation of D and X = B L),
+ * stream: ms[0] the fitted density gamma (a pass over B for J alone; with J
+ * and K together from X: gamma_P = sum_a (B_P D)_aa), ms[1] the J pass, ms[2]
+ * the X = B D GEMM (or the factorisation of D and X = B L),
  * ms[3] the K = X B^T GEMM (split over the summation index), ms[4] the sum of
  * its slices (entries of kernels not run are 0).  No reference counterpart
  * (measurement). */

@@ -18,12 +18,13 @@
 // occupied orbitals is, is factored first (df_factor, D = L L^T with r
 // columns, corrected and checked against D): then X = B L has r columns instead
 // of n and K[a][c] = sum_(P,i) X[a][P][i] X[c][P][i], r/n of the work (16 waters
-// / cc-pVDZ, n 400, r 80: 7.6 -> 2.3 ms; X = B L 0.86, K 0.58, df_factor 0.35
-// and its correction 0.3 to 0.4 ms are what is left).  Relative error of K (long
-// double, B as it is), general products and factored, 225 / 300 / 400
-// functions, in 1e-16: localised orbitals 5.9 8.2 10.2 and 5.6 7.5 9.0,
-// delocalised 5.8 7.2 9.3 and 5.8 7.3 8.2, graded 6.9 7.9 10.4 and 6.2 6.1
-// 10.5; without the correction 5.8 4.8 10.0, 9.2 11.0 12.3 and 18.7 29.8 33.6.
+// / cc-pVDZ, n 400, r 80: 7.6 -> 2.24 ms; X = B L 0.84, K beside the Coulomb
+// passes 0.75, df_factor 0.34 and its correction 0.2 ms are what is left).
+// Relative error of K (40 rows against long double, B as it is) by the general
+// products and factored, 225 / 300 / 400 functions, in 1e-16: localised orbitals
+// 6.1 8.0 11.0 and 5.6 7.5 9.0, delocalised 6.2 7.6 11.7 and 5.8 7.3 8.0, graded
+// 7.5 8.0 14.6 and 6.2 6.1 10.5; without the correction (6 rows) 5.8 4.8 10.0,
+// 9.2 11.0 12.3 and 18.7 29.8 33.6.
 // The device decides (Factor::ok); the launches of the other form return at
 // once.
 #include "lai_device.h"
@@ -76,7 +77,8 @@ struct Factor {
   int rank;
   double dmax;  // largest diagonal element of D
   double e2, d2;  // ||D - L L^T||^2 and ||D||^2 (Frobenius) over dmax^2
-  int low;      // 1 once pivoting has ended well: the general product under way may end
+  int low;      // 0 until pivoting has ended, then 1 (the general product under way
+                // may end) or -1 (D has no factor of at most n/2 columns)
 };
 constexpr double kEps = 2.220446049250313e-16;
 // df_factor takes columns while a diagonal element of D - L L^T exceeds half of
@@ -91,16 +93,19 @@ __host__ __device__ constexpr double factor_tol(int n) { return 32 * kEps * (n >
 // of the general products gives K 2.5 to 4.5 eps.
 constexpr double kResidTol = 4 * kEps;
 
-// which sizes of a product are the rank (GemmArgs::low)
+// which sizes of a product are the rank (GemmArgs::low, SmallArgs::low)
 enum : int { kRankM = 1, kRankN = 2, kRankK = 4, kRankLda = 8, kRankLdb = 16, kRankLdc = 32, kRankSlices = 64 };
 
 struct GemmArgs {
   const Factor* fac;  // null: run; else run only when fac->ok == want
-  int want;           // (-1: beside the factorisation, workgroups begin until fac->low;
-                      // -2: what -1 began for a D that is refused after fac->low)
+  int want;           // (-1: beside the factorisation, workgroups begin until fac->low)
   // with fac and want = 1, the sizes that are the rank r (kRank*);
   // kRankSlices: K = lda = ldb = naux r in kslices slices (K = X X^T)
   int low, naux, kslices;
+  // with want = 1 and not null: the right factor (row-major, bt = 0) and sizes
+  // as given where the D was refused after fac->low, so that want = -1 left
+  // the product undone
+  const double* Blate;
   const double* A;
   const double* B;
   double* C;
@@ -116,24 +121,30 @@ struct GemmArgs {
   // tile m on XCD m % 8 (the row tile of A is read once).  mt, nt: tiles
   // along M and N; nz: slices.
   int xcd, mt, nt, nz;
+  // 1 (NCOLS): one workgroup takes every column tile of its row tile, one after another
+  // (the number of columns is the rank, which the host does not know: a
+  // workgroup that finds nothing to do still takes its 55 KB of LDS, some 70 ns
+  // on each XCD; X = B L of 300 functions and rank 60 0.52 -> 0.38 ms)
+  int ncols;
 };
 
-template <int BM, int BN>
-__global__ __launch_bounds__(256) void dgemm_mfma(GemmArgs g) {
+template <int BM, int BN, bool NCOLS = false>
+__global__ __launch_bounds__(256, 2) void dgemm_mfma(GemmArgs g) {
   if (g.fac) {  // uniform over the grid
+    const int r = g.fac->rank;
     if (g.want == -1) {  // one answer for the workgroup: low may be set meanwhile
       __shared__ int low;
       if (threadIdx.x == 0) low = __hip_atomic_load(&g.fac->low, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __syncthreads();
-      if (low) return;
-    } else if (g.want == -2 ? (g.fac->ok || !g.fac->low) : g.fac->ok != g.want)
+      if (low > 0) return;
+    } else if (g.Blate && !g.fac->ok) {
+      if (g.fac->low < 0) return;
+      g.B = g.Blate;
+      g.bt = 0;
+      g.low = 0;
+    } else if (g.fac->ok != g.want)
       return;
-    const int r = g.fac->rank;
-    if (g.low & kRankM) g.M = r;
     if (g.low & kRankN) g.N = r;
-    if (g.low & kRankK) g.K = r;
-    if (g.low & kRankLda) g.lda = r;
-    if (g.low & kRankLdb) g.ldb = r;
     if (g.low & kRankLdc) g.ldc = r;
     if (g.low & kRankSlices) {
       g.K = g.naux * r;
@@ -166,8 +177,9 @@ __global__ __launch_bounds__(256) void dgemm_mfma(GemmArgs g) {
       z = 0;
     }
   }
-  const int m0 = mi * TM, n0 = ni * TN;
-  if (m0 >= g.M || n0 >= g.N) return;  // tiles beyond the rank
+  const int m0 = mi * TM;
+  int n0 = ni * TN;
+  if (!NCOLS && n0 >= g.N) return;
   if (g.skip_lower && m0 > n0 + TN - 1) return;  // uniform over the workgroup, before any barrier
   const double* A = g.A;
   const double* B = g.B;
@@ -182,10 +194,6 @@ __global__ __launch_bounds__(256) void dgemm_mfma(GemmArgs g) {
   }
   const int wm = wave * 16 * BM;
   v4d acc[BM][BN];
-#pragma unroll
-  for (int i = 0; i < BM; ++i)
-#pragma unroll
-    for (int j = 0; j < BN; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
   double ra[NA], rb[NB];
   auto load = [&](int k0) {
 #pragma unroll
@@ -227,6 +235,11 @@ __global__ __launch_bounds__(256) void dgemm_mfma(GemmArgs g) {
       }
     }
   };
+  do {
+#pragma unroll
+  for (int i = 0; i < BM; ++i)
+#pragma unroll
+    for (int j = 0; j < BN; ++j) acc[i][j] = v4d{0.0, 0.0, 0.0, 0.0};
   if (kb < ke) {
     load(kb);
     store(0);
@@ -262,6 +275,8 @@ __global__ __launch_bounds__(256) void dgemm_mfma(GemmArgs g) {
         const int col = n0 + 16 * j + (lane & 15);
         if (row < g.M && col < g.N) C[(long long)row * g.ldc + col] = acc[i][j][r];
       }
+  n0 += TN;
+  } while (NCOLS && n0 < g.N);
 }
 
 // K[r][c] = K[c][r] for r > c (n x n, row-major)
@@ -365,6 +380,40 @@ __global__ __launch_bounds__(1024) void df_gamma_diag(const double* __restrict__
   }
 }
 
+// The same where the device decided which X there is: part[a][P] = sum_i
+// X[a][P][i] L[a][i] of X = B L (r columns; a fifth of the bytes of a pass over
+// half of B; Lt holds rows of L, rmax apart), or X[a][P][a] of X = B D;
+// df_gamma_sum sums over a.  A wavefront takes 32 rows, 16 lanes each.  0.37 ms
+// beside the K product of 400 functions and rank 80 (with a cache line of L per
+// lane 0.45 to 0.61; in the epilogue of X = B L it costs that product 0.13 ms).
+__global__ __launch_bounds__(256) void df_gamma_x(const double* __restrict__ X, const double* __restrict__ Lt, int rmax,
+                                                  int n, int naux, const Factor* __restrict__ fac,
+                                                  double* __restrict__ part) {
+  const int a = blockIdx.x, lane = threadIdx.x & 63, l16 = lane & 15;
+  const int Pw = blockIdx.y * 128 + (threadIdx.x >> 6) * 32;
+  const long long row0 = (long long)a * naux;
+  if (!fac->ok) {
+    if (lane < 32 && Pw + lane < naux) part[row0 + Pw + lane] = X[(row0 + Pw + lane) * n + a];
+    return;
+  }
+  const int rank = fac->rank, P0 = Pw + (lane >> 4);
+  double s[8];
+#pragma unroll
+  for (int t = 0; t < 8; ++t) s[t] = 0.0;
+  for (int i = l16; i < rank; i += 16) {
+    const double l = Lt[(long long)a * rmax + i];
+#pragma unroll
+    for (int t = 0; t < 8; ++t)
+      if (P0 + 4 * t < naux) s[t] = fma(X[(row0 + P0 + 4 * t) * rank + i], l, s[t]);
+  }
+#pragma unroll
+  for (int t = 0; t < 8; ++t) {
+#pragma unroll
+    for (int o = 8; o >= 1; o >>= 1) s[t] += __shfl_xor(s[t], o, 64);
+    if (l16 == 0 && P0 + 4 * t < naux) part[row0 + P0 + 4 * t] = s[t];
+  }
+}
+
 // J[a][b] = sum_P B[a][P][b] gamma[P] for b >= a, and J[b][a] (each B_P is
 // symmetric: half of B is read, 0.45 -> 0.25 ms for 400 x 1536 x 400):
 // workgroup (64 columns b, a), the four wavefronts take every fourth P (lanes
@@ -409,13 +458,14 @@ __global__ __launch_bounds__(256) void df_coulomb(const double* __restrict__ B, 
 // a few LDS reads): 0.35 ms for 80 columns of 400.
 // RP rows per lane: n at most RP kFactorNT.
 // ---------------------------------------------------------------------------
-// From kFactorMinN functions on: J and K in ms without and with the factor, and
-// for a D that is refused (indefinite or of full rank), water / cc-pVDZ:
-//   225: 1.13 0.93 refused 1.28   250: 1.82 1.10 refused 1.95
-//   300: 3.08 1.64 refused 3.32   400: 7.6  2.34 refused 8.0
-//   600: 42.9 17.0 refused 43.9
-// (the step from 400 to 600 is B, 2.2 GB, outgrowing the cache).  Up to
-// kFactorMaxN rows stay in registers.
+// From kFactorMinN functions on: J and K in ms by the general products alone,
+// with a factor (a fifth of the functions), and where D is refused as indefinite
+// and for its rank, water / cc-pVDZ:
+//   225: 1.13 0.80 1.19 1.22   250: 1.82 0.92 1.86 1.89   300: 3.07 1.30 3.09 3.12
+//   400: 7.63 2.24 7.76 7.85   600: 43.1 11.4 43.2 43.6
+// (the step from 400 to 600 is B, 2.2 GB, outgrowing the cache; what a refused D
+// loses are 30 us of launches that do nothing, and under 300 functions the pivoting
+// beside a short X = B D).  Up to kFactorMaxN rows stay in registers.
 constexpr int kFactorMaxN = 2048, kFactorMinN = 224, kFactorNT = 1024, kPanel = 16, kPanelK = 32;
 template <int RP>
 __global__ __launch_bounds__(kFactorNT) void df_factor(const double* __restrict__ D, int n, int rmax,
@@ -586,7 +636,7 @@ __global__ __launch_bounds__(kFactorNT) void df_factor(const double* __restrict_
     fac->d2 = 0.0;
     // (the general product ends here, not after the correction, whose small
     // kernels would wait for its workgroups: 400 functions 2.59 -> 2.34 ms)
-    __hip_atomic_store(&fac->low, fac->ok, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&fac->low, fac->ok ? 1 : -1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
@@ -700,28 +750,31 @@ __global__ __launch_bounds__(1024) void df_invert(double* G, const Factor* __res
       }
     for (int k = 0; k < r; ++k) {
       const int u = k & 1;
+      // row k and column k, the pivot less one in the column: with row k over
+      // the pivot q, and 1 + 1/q at k, A - col row is then the step for every
+      // element, row and column k among them
 #pragma unroll
       for (int m = 0; m < 4; ++m) {
         if (tx + 32 * m == k)
 #pragma unroll
-          for (int a = 0; a < 4; ++a) col[u][ty + 32 * a] = A[a][m];
+          for (int a = 0; a < 4; ++a) col[u][ty + 32 * a] = ty + 32 * a == k ? A[a][m] - 1.0 : A[a][m];
         if (ty + 32 * m == k)
 #pragma unroll
           for (int b = 0; b < 4; ++b) row[u][tx + 32 * b] = A[m][b];
       }
       __syncthreads();  // (the other buffer was read before this)
-      const double p = 1.0 / row[u][k];
+      const double q = row[u][k];
+      double p = __builtin_amdgcn_rcp(q);
+      p = fma(p, fma(-q, p, 1.0), p);
+      double c[4], x[4];
 #pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        const int i = ty + 32 * a;
-        const double c = col[u][i];
+      for (int a = 0; a < 4; ++a) c[a] = col[u][ty + 32 * a];
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const int j = tx + 32 * b;
-          const double x = row[u][j] * p;
-          A[a][b] = i == k ? (j == k ? p : x) : j == k ? -c * p : fma(-c, x, A[a][b]);
-        }
-      }
+      for (int b = 0; b < 4; ++b) x[b] = tx + 32 * b == k ? 1.0 + p : row[u][tx + 32 * b] * p;
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < 4; ++b) A[a][b] = fma(-c[a], x[b], A[a][b]);
     }
 #pragma unroll
     for (int a = 0; a < 4; ++a)
@@ -752,26 +805,67 @@ __global__ __launch_bounds__(1024) void df_invert(double* G, const Factor* __res
   }
 }
 
-// L += (F - Lh H / 2) / dk by columns: 64 rows i by 16 columns k per workgroup.
-__global__ __launch_bounds__(256) void df_update(const double* __restrict__ Lh, const double* __restrict__ F,
-                                                 const double* __restrict__ H, const double* __restrict__ dk, int n,
-                                                 double* __restrict__ Lc, const Factor* __restrict__ fac) {
-  if (!fac->ok) return;
-  const int r = fac->rank, i = blockIdx.x * 64 + (threadIdx.x & 63);
-  const int k0 = blockIdx.y * 16 + 4 * __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (i >= n || k0 >= r) return;
-  double s[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int l = 0; l < r; ++l) {
-    const double v = Lh[(long long)l * n + i];
+// The products of the correction: C = A B (BT: A B^T) of at most some hundred
+// rows, rows and columns from the rank where low says so.  A workgroup computes
+// 16 x 16 elements, its four wavefronts a quarter of the summation each, with
+// the operands straight from the cache (dgemm_mfma has 7 tiles for 80 x 400
+// and takes 40 us for a summation over 400, this 10).  UPDATE: instead of C,
+// L += (F - C / 2) / dk by rows.
+struct SmallArgs {
+  const Factor* fac;
+  int low;
+  const double *A, *B;
+  double* C;
+  int M, N, K;
+  int lda, ldb, ldc;
+  const double *F, *dk;  // UPDATE: F laid out as C
+  double* Lt;            // and L by columns too, column j at Lt + j ldt
+  int ldt;
+};
+template <bool BT, bool UPDATE>
+__global__ __launch_bounds__(256) void df_small(SmallArgs g) {
+  if (!g.fac->ok) return;
+  const int r = g.fac->rank;
+  if (g.low & kRankM) g.M = r;
+  if (g.low & kRankN) g.N = r;
+  if (g.low & kRankK) g.K = r;
+  if (g.low & kRankLda) g.lda = r;
+  if (g.low & kRankLdc) g.ldc = r;
+  const int m0 = blockIdx.y * 16, n0 = blockIdx.x * 16;
+  if (m0 >= g.M || n0 >= g.N) return;
+  __shared__ double part[4][16][17];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, l16 = lane & 15, q = lane >> 4;
+  // lane (l16, q) holds elements k0 + 4 q .. + 3 of its row of A and column of B
+  // (any order of the summation index will do, if it is the same in both)
+  const bool am = m0 + l16 < g.M, bn = n0 + l16 < g.N;
+  const double* A = g.A + (long long)(m0 + l16) * g.lda;
+  const double* B = BT ? g.B + (long long)(n0 + l16) * g.ldb : g.B + n0 + l16;
+  v4d acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 2
+  for (int k0 = 16 * wave; k0 < g.K; k0 += 64) {
+    double a[4], b[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) s[q] = fma(H[(long long)min(k0 + q, r - 1) * r + l], v, s[q]);
+    for (int t = 0; t < 4; ++t) {
+      const int k = k0 + 4 * q + t;
+      a[t] = am && k < g.K ? A[k] : 0.0;
+      b[t] = bn && k < g.K ? (BT ? B[k] : B[(long long)k * g.ldb]) : 0.0;
+    }
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t], b[t], acc, 0, 0, 0);
   }
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int k = k0 + q;
-    if (k >= r) break;
-    const long long at = (long long)k * n + i;
-    Lc[at] += (F[at] - 0.5 * s[q]) / dk[k];
+  for (int t = 0; t < 4; ++t) part[wave][q + 4 * t][l16] = acc[t];
+  __syncthreads();
+  const int i = threadIdx.x >> 4, j = threadIdx.x & 15;
+  if (m0 + i >= g.M || n0 + j >= g.N) return;
+  const double v = (part[0][i][j] + part[1][i][j]) + (part[2][i][j] + part[3][i][j]);
+  const long long at = (long long)(m0 + i) * g.ldc + n0 + j;
+  if constexpr (UPDATE) {
+    const double x = g.C[at] + (g.F[at] - 0.5 * v) / g.dk[m0 + i];
+    g.C[at] = x;
+    g.Lt[(long long)(n0 + j) * g.ldt + m0 + i] = x;
+  } else {
+    g.C[at] = v;
   }
 }
 
@@ -836,9 +930,10 @@ struct Dev {
 int gemm(const GemmArgs& g0, int gz, hipStream_t st) {
   GemmArgs g = g0;
   if (g.M <= 0 || g.N <= 0 || gz <= 0) return LAI_OK;
-  const bool tall = g.M >= 1024;
+  const bool tall = g.M >= 1024 || g.ncols;
   const int TM = tall ? 128 : 64, TN = 80;
   dim3 grid((g.M + TM - 1) / TM, (g.N + TN - 1) / TN, gz);
+  if (g.ncols) grid.y = 1;
   if (g.xcd) {
     if (!g.split && gz != 1)
       return set_error(LAI_ERR_INVALID_ARGUMENT, "density fitting: XCD order needs one batch or a split product");
@@ -853,7 +948,9 @@ int gemm(const GemmArgs& g0, int gz, hipStream_t st) {
   }
   if (grid.y > 65535u || grid.z > 65535u)
     return set_error(LAI_ERR_INVALID_ARGUMENT, "density fitting: GEMM grid beyond the launch limits");
-  if (tall)
+  if (g.ncols)
+    hipLaunchKernelGGL((dgemm_mfma<2, 5, true>), grid, dim3(256), 0, st, g);
+  else if (tall)
     hipLaunchKernelGGL((dgemm_mfma<2, 5>), grid, dim3(256), 0, st, g);
   else
     hipLaunchKernelGGL((dgemm_mfma<1, 5>), grid, dim3(256), 0, st, g);
@@ -864,7 +961,8 @@ int gemm(const GemmArgs& g0, int gz, hipStream_t st) {
 // Memory of a factorisation: factor_doubles(n) doubles at one address.
 struct FactorBufs {
   double *Lc, *Lh, *Z, *F;  // [rmax][n]: L, its scaled columns, Z and E Z
-  double* E;                // [n][n]
+  double* E;                // [n][n]: D - L L^T, and once L is corrected
+  double* Lt;               // [n][rmax] in its place: the rows of L
   double *G, *H;            // [rmax][rmax]
   double* dk;               // [rmax]
   int rmax;
@@ -874,7 +972,7 @@ struct FactorBufs {
     Lh = Lc + rn;
     Z = Lh + rn;
     F = Z + rn;
-    E = F + rn;
+    E = Lt = F + rn;
     G = E + size_t(n) * n;
     H = G + rr;
     dk = H + rr;
@@ -893,11 +991,11 @@ int factor_density(const double* D, int n, const FactorBufs& f, Factor* fac, hip
     hipLaunchKernelGGL(df_factor<2>, dim3(1), dim3(kFactorNT), 0, st, D, n, f.rmax, f.Lc, f.Lh, f.dk, fac);
   DF_HIP(hipGetLastError());
   const unsigned t = unsigned((n + 31) / 32);
-  // C = A B or A B^T with the given sizes of the rank
-  auto mul = [&](const double* A, const double* B, double* C, int M, int N, int K, int bt, int low) -> int {
-    GemmArgs g{};
+  const int r = f.rmax;
+  // C = A B or A B^T, M rows and N columns of which the rank is as low says
+  auto args = [&](const double* A, const double* B, double* C, int M, int N, int K, int low) {
+    SmallArgs g{};
     g.fac = fac;
-    g.want = 1;
     g.low = low;
     g.A = A;
     g.B = B;
@@ -906,24 +1004,30 @@ int factor_density(const double* D, int n, const FactorBufs& f, Factor* fac, hip
     g.N = N;
     g.K = K;
     g.lda = g.ldb = g.ldc = n;
-    g.bt = bt;
-    return gemm(g, 1, st);
+    return g;
   };
-  const int r = f.rmax;
+  auto grid = [](const SmallArgs& g) { return dim3((g.N + 15) / 16, (g.M + 15) / 16); };
+  const SmallArgs gram = args(f.Lh, f.Lh, f.G, r, r, n, kRankM | kRankN | kRankLdc);
+  const SmallArgs z = args(f.G, f.Lh, f.Z, r, n, r, kRankM | kRankK | kRankLda);
+  const SmallArgs ez = args(f.Z, f.E, f.F, r, n, n, kRankM);
+  const SmallArgs h = args(f.Z, f.F, f.H, r, r, n, kRankM | kRankN | kRankLdc);
+  SmallArgs up = args(f.H, f.Lh, f.Lc, r, n, r, kRankM | kRankK | kRankLda);
+  up.F = f.F;
+  up.dk = f.dk;
+  up.Lt = f.Lt;
+  up.ldt = r;
   for (int step = 0; step < (n <= 512 ? 1 : 2); ++step) {
-    int rc;
     hipLaunchKernelGGL(df_resid<false>, dim3(t, t), dim3(256), 0, st, D, f.Lc, n, f.E, fac);
     DF_HIP(hipGetLastError());
     if (step == 0) {  // G = (Lh^T Lh)^-1, Z (the projection hardly changes)
-      if ((rc = mul(f.Lh, f.Lh, f.G, r, r, n, 1, kRankM | kRankN | kRankLdc))) return rc;
+      hipLaunchKernelGGL((df_small<true, false>), grid(gram), dim3(256), 0, st, gram);
       hipLaunchKernelGGL(df_invert, dim3(1), dim3(1024), 0, st, f.G, fac);
+      hipLaunchKernelGGL((df_small<false, false>), grid(z), dim3(256), 0, st, z);
       DF_HIP(hipGetLastError());
-      if ((rc = mul(f.G, f.Lh, f.Z, r, n, r, 0, kRankM | kRankK | kRankLda))) return rc;
     }
-    if ((rc = mul(f.Z, f.E, f.F, r, n, n, 0, kRankM))) return rc;
-    if ((rc = mul(f.Z, f.F, f.H, r, r, n, 1, kRankM | kRankN | kRankLdc))) return rc;
-    hipLaunchKernelGGL(df_update, dim3((n + 63) / 64, (r + 15) / 16), dim3(256), 0, st, f.Lh, f.F, f.H, f.dk, n, f.Lc,
-                       fac);
+    hipLaunchKernelGGL((df_small<false, false>), grid(ez), dim3(256), 0, st, ez);
+    hipLaunchKernelGGL((df_small<true, false>), grid(h), dim3(256), 0, st, h);
+    hipLaunchKernelGGL((df_small<false, true>), grid(up), dim3(256), 0, st, up);
     DF_HIP(hipGetLastError());
   }
   hipLaunchKernelGGL(df_resid<true>, dim3(t, t), dim3(256), 0, st, D, f.Lc, n, nullptr, fac);
@@ -990,7 +1094,7 @@ struct lai_df {
   bool have_ev = false;
   double* fbuf = nullptr;   // memory of the density's factor (FactorBufs), null where it is not tried
   Factor* fac = nullptr;
-  // the Coulomb passes run beside the exchange GEMMs on this stream
+  // X = B D beside the factorisation, the Coulomb pass beside the K product
   hipStream_t side = nullptr;
   hipEvent_t fork = nullptr, join = nullptr;
 };
@@ -1300,15 +1404,29 @@ int df_run(lai_df* d, const double* D, double* J, double* K, int flags, hipStrea
     DF_HIP(hipGetLastError());
     return LAI_OK;
   };
-  auto gamma_pass = [&](hipStream_t s) -> int {
-    hipLaunchKernelGGL(df_gamma_part, dim3(n, (naux + kGammaRows - 1) / kGammaRows), dim3(256), 0, s, d->B, D, n, naux,
-                       sym, d->gpart);
-    DF_HIP(hipGetLastError());
+  auto gamma_sum = [&](hipStream_t s) -> int {
     hipLaunchKernelGGL(df_gamma_sum, dim3((naux + 63) / 64), dim3(1024), 0, s, d->gpart, n, naux, d->gamma);
     DF_HIP(hipGetLastError());
     return LAI_OK;
   };
-  auto x_low = [&]() -> int {  // X = B L
+  auto gamma_pass = [&](hipStream_t s) -> int {
+    hipLaunchKernelGGL(df_gamma_part, dim3(n, (naux + kGammaRows - 1) / kGammaRows), dim3(256), 0, s, d->B, D, n, naux,
+                       sym, d->gpart);
+    DF_HIP(hipGetLastError());
+    return gamma_sum(s);
+  };
+  auto gamma_of_x = [&](hipStream_t s) -> int {  // the fitted density from X, whichever it is
+    if (!factor) {
+      hipLaunchKernelGGL(df_gamma_diag, dim3((naux + 63) / 64), dim3(1024), 0, s, d->X, n, naux, d->gamma);
+      DF_HIP(hipGetLastError());
+      return LAI_OK;
+    }
+    hipLaunchKernelGGL(df_gamma_x, dim3(n, (naux + 127) / 128), dim3(256), 0, s, d->X, fb.Lt, fb.rmax, n, naux, d->fac,
+                       d->gpart);
+    DF_HIP(hipGetLastError());
+    return gamma_sum(s);
+  };
+  auto x_low = [&](const double* late = nullptr) -> int {  // X = B L (or B late: GemmArgs::Blate)
     GemmArgs g{};
     g.fac = d->fac;
     g.want = 1;
@@ -1320,8 +1438,10 @@ int df_run(lai_df* d, const double* D, double* J, double* K, int flags, hipStrea
     g.lda = n;
     g.ldb = n;
     g.M = n * naux;
-    g.N = fb.rmax;
-    g.ldc = fb.rmax;
+    g.Blate = late;
+    g.ncols = 1;
+    g.N = n;
+    g.ldc = n;
     g.K = n;
     g.xcd = 1;
     return gemm(g, 1, st);
@@ -1409,55 +1529,49 @@ int df_run(lai_df* d, const double* D, double* J, double* K, int flags, hipStrea
     }
     return rc;
   };
-  int rc;
-  if (factor && !ms && d->side) {
-    // beside the factorisation, which is one workgroup: the Coulomb passes (the
-    // fitted density from a pass over B), then X = B D, whose workgroups begin
-    // until D is known to be of low rank.  A density that is refused so costs
-    // the pass over B; with X = B D after the factorisation a full rank took
-    // 1.23 ms instead of 0.86 at 200 functions, 8.2 instead of 7.5 at 400.
-    hipLaunchKernelGGL(df_open, dim3(1), dim3(1), 0, st, d->fac);
-    DF_HIP(hipGetLastError());
+  auto fork_side = [&]() -> int {
     DF_HIP(hipEventRecord(d->fork, st));
     DF_HIP(hipStreamWaitEvent(d->side, d->fork, 0));
-    auto beside = [&]() -> int {
-      int r;
-      if ((r = factor_density(D, n, fb, d->fac, st))) return r;
-      if (both && ((r = gamma_pass(d->side)) || (r = coulomb(d->side)))) return r;
-      return x_gemm(d->side, -1);
-    };
-    rc = beside();
-    if ((rc = join_side(rc)) || (rc = x_gemm(st, -2)) || (rc = x_low())) return rc;
-    return k_product();
-  }
+    return LAI_OK;
+  };
+  const bool overlap = !ms && d->side;  // not profiled
+  // X: B D, or from a factor of D
+  auto x_product = [&]() -> int {
+    int r;
+    if (!factor) return x_gemm(st, 0);
+    if (!overlap) {
+      if ((r = factor_density(D, n, fb, d->fac, st)) || (r = x_low())) return r;
+      return x_gemm(st, 0);
+    }
+    // beside the factorisation, which is one workgroup, X = B D, whose
+    // workgroups begin until pivoting has ended well: a density that is refused
+    // loses little
+    hipLaunchKernelGGL(df_open, dim3(1), dim3(1), 0, st, d->fac);
+    DF_HIP(hipGetLastError());
+    if ((r = fork_side())) return r;
+    if ((r = factor_density(D, n, fb, d->fac, st)) == LAI_OK) r = x_gemm(d->side, -1);
+    r = join_side(r);
+    return r ? r : x_low(D);
+  };
+  int rc;
   if (both) {
-    // X = B D first: J's fitted density is the diagonal of X, so B is read
-    // twice per build (X, Coulomb pass) plus once more with X by the K product.
-    // Not profiled: the Coulomb pass (HBM-bound) runs on the side stream
-    // beside the K product (matrix cores), joined back into st.
-    const bool overlap = !ms && d->side;
+    // X first: J's fitted density comes from it, so B is read twice per build
+    // (X, Coulomb pass) plus, where there is no factor, once more with X by the
+    // K product.  The Coulomb pass (HBM-bound) runs on the side stream beside
+    // the K product (matrix cores), joined back into st.
     const hipStream_t sj = overlap ? d->side : st;
     if ((rc = mark(0))) return rc;
-    if (factor && ((rc = factor_density(D, n, fb, d->fac, st)) || (rc = x_low()))) return rc;
-    if ((rc = x_gemm(st, 0))) return rc;
+    if ((rc = x_product())) return rc;
     if ((rc = mark(1))) return rc;
     if ((rc = take(0, 1, 2))) return rc;
-    if (overlap) {
-      DF_HIP(hipEventRecord(d->fork, st));
-      DF_HIP(hipStreamWaitEvent(d->side, d->fork, 0));
-    }
+    if (overlap && (rc = fork_side())) return rc;
     // from here on st is joined to the side stream on every return path, so
     // that a failed launch never leaves work writing J or gamma unordered
     // with the caller's stream
     auto side_part = [&]() -> int {
       int r;
       if ((r = mark(0))) return r;
-      if (factor) {  // X may hold B L: the fitted density from a pass over B
-        if ((r = gamma_pass(sj))) return r;
-      } else {
-        hipLaunchKernelGGL(df_gamma_diag, dim3((naux + 63) / 64), dim3(1024), 0, sj, d->X, n, naux, d->gamma);
-        DF_HIP(hipGetLastError());
-      }
+      if ((r = gamma_of_x(sj))) return r;
       if ((r = mark(1))) return r;
       if ((r = coulomb(sj))) return r;
       if ((r = mark(2))) return r;
@@ -1477,8 +1591,7 @@ int df_run(lai_df* d, const double* D, double* J, double* K, int flags, hipStrea
   }
   if (flags & LAI_DF_K) {
     if ((rc = mark(0))) return rc;
-    if (factor && ((rc = factor_density(D, n, fb, d->fac, st)) || (rc = x_low()))) return rc;
-    if ((rc = x_gemm(st, 0))) return rc;
+    if ((rc = x_product())) return rc;
     if ((rc = mark(1))) return rc;
     if ((rc = take(0, 1, 2))) return rc;
     if ((rc = k_product())) return rc;
