@@ -1059,30 +1059,32 @@ std::vector<JkChunk> cut_runs(const lai_basis* b, const ClassList& cl, int cmax,
       for (int k0 = 0; k0 < len; k0 += per) C.push_back(JkChunk{r.bra, r.seg, k0, std::min(len, k0 + per)});
       continue;
     }
-    // entries before position k of the run
+    // entries before each segment, and before position m of segment s
     const JkSegs& sg = b->segs_h[r.seg];
-    auto before = [&](int k) {
-      double x = 0.0;
-      for (int s = 0; s < sg.n && sg.cum[s] < k; ++s) {
-        const int m = std::min(k, sg.cum[s + 1]) - sg.cum[s];
-        x += m + double(b->lcum[sg.start[s] + m] - b->lcum[sg.start[s]]) / sp.per;
-      }
-      return x;
+    double base[kMaxSegs + 1] = {};
+    auto before = [&](int s, int m) {
+      const long long* l = &b->lcum[sg.start[s]];
+      return base[s] + (m + double(l[m] - l[0]) / sp.per);
     };
-    const double tot = before(len);
+    for (int s = 0; s < sg.n; ++s) base[s + 1] = before(s, sg.cum[s + 1] - sg.cum[s]);
+    const double tot = base[sg.n];
     const int pieces = std::min(len, int(tot / cmax) + 1);
     int k0 = 0;
-    for (int q = 1; q <= pieces && k0 < len; ++q) {
-      int lo = k0 + 1, hi = len;  // first k with before(k) >= q/pieces of all
+    for (int q = 1, s = 0; q < pieces && k0 + 1 < len; ++q) {
+      // first position with q/pieces of all entries before it
+      const double want = tot * q / pieces;
+      while (s + 1 < sg.n && base[s + 1] < want) ++s;
+      int lo = std::max(k0 + 1 - sg.cum[s], 0), hi = std::max(sg.cum[s + 1] - sg.cum[s], lo);
       while (lo < hi) {
         const int mid = (lo + hi) / 2;
-        if (before(mid) >= tot * q / pieces) hi = mid;
+        if (before(s, mid) >= want) hi = mid;
         else lo = mid + 1;
       }
-      if (q == pieces) lo = len;
-      C.push_back(JkChunk{r.bra, r.seg, k0, lo});
-      k0 = lo;
+      const int k = std::min(sg.cum[s] + lo, len);
+      C.push_back(JkChunk{r.bra, r.seg, k0, k});
+      k0 = k;
     }
+    if (k0 < len) C.push_back(JkChunk{r.bra, r.seg, k0, len});
   }
   return C;
 }

@@ -4,6 +4,7 @@
 // class kernels (each launch looks at what it was given).
 //   worklist_driver alloc  every allocation of a rebuild and of a tuning fails
 //                          in turn; nothing may run on parts of two lists
+//   worklist_driver cut    the chunks of divided kets against their definition
 #include "../../libaccint-public_amd/csrc/device/api.hip"
 
 #include <cstdio>
@@ -257,12 +258,79 @@ static int alloc_test(lai_ctx* ctx) {
   return g_bad;
 }
 
+// The chunks of a run by their definition: entry by entry, a chunk ends at the
+// first position that has its share of all entries before it.
+static std::vector<JkChunk> cut_plainly(const lai_basis* b, const JkChunk& r, int kmax, int cmax, int chain) {
+  const JkSegs& sg = b->segs_h[r.seg];
+  const KetSplit sp = ket_split(chain, kmax, int(b->lcum[r.bra + 1] - b->lcum[r.bra]));
+  std::vector<double> before(1, 0.0);
+  double done = 0.0;
+  for (int s = 0; s < sg.n; ++s) {
+    const long long* l = &b->lcum[sg.start[s]];
+    const int len = sg.cum[s + 1] - sg.cum[s];
+    for (int m = 1; m <= len; ++m) before.push_back(done + (m + double(l[m] - l[0]) / sp.per));
+    done = before.back();
+  }
+  std::vector<JkChunk> C;
+  const int pieces = std::min(r.k1, int(done / cmax) + 1);
+  int k0 = 0;
+  for (int q = 1; q <= pieces && k0 < r.k1; ++q) {
+    int k = k0 + 1;
+    while (k < r.k1 && (q == pieces || before[k] < done * q / pieces)) ++k;
+    C.push_back(JkChunk{r.bra, r.seg, k0, k});
+    k0 = k;
+  }
+  return C;
+}
+
+static int cut_test(lai_ctx* ctx) {
+  long divided = 0, several = 0;
+  for (int atoms : {1, 2, 5}) {
+    lai_basis* b = make_basis(ctx, atoms, atoms);
+    if (build(b, 1e-12) != LAI_OK) complain("a build without failures failed");
+    for (int c = 0; c < kNumClasses; ++c) {
+      const ClassList& C = b->cls[c];
+      for (int chain : {C.chain, 1, 16, 100})
+        for (int cmax : {1, 3, 64, 256, 2048}) {
+          const std::vector<JkChunk> got = cut_runs(b, C, cmax, chain);
+          size_t at = 0;
+          for (const JkChunk& r : C.runs) {
+            const KetSplit sp = ket_split(chain, C.kmax, int(b->lcum[r.bra + 1] - b->lcum[r.bra]));
+            int k = 0;
+            const size_t first = at;
+            for (; at < got.size() && k < r.k1; ++at) {
+              const JkChunk& x = got[at];
+              if (x.bra != r.bra || x.seg != r.seg || x.k0 != k || x.k1 <= x.k0 || x.k1 > r.k1)
+                complain("the chunks of a run are not its parts in order");
+              k = x.k1;
+            }
+            if (k != r.k1) complain("a run is not covered");
+            if (sp.per >= C.kmax) continue;
+            ++divided;
+            const std::vector<JkChunk> want = cut_plainly(b, r, C.kmax, cmax, chain);
+            several += want.size() > 1;
+            bool same = want.size() == at - first;
+            for (size_t i = 0; same && i < want.size(); ++i)
+              same = want[i].k0 == got[first + i].k0 && want[i].k1 == got[first + i].k1;
+            if (!same) complain("a divided run is cut elsewhere");
+            if (g_bad) return std::printf("%d atoms, class %d, chain %d, cap %d\n", atoms, c, chain, cmax), 1;
+          }
+          if (at != got.size()) complain("chunks beyond the runs");
+        }
+    }
+    lai_dev_basis_free(b);
+  }
+  std::printf("%ld divided runs, %ld of several chunks\n", divided, several);
+  return g_bad || several == 0;
+}
+
 int main(int argc, char** argv) {
   lai_ctx* ctx = nullptr;
   if (lai_dev_init(0, &ctx) != LAI_OK) return std::printf("init: %s\n", lai_dev_last_error()), 2;
   const std::string what = argc > 1 ? argv[1] : "alloc";
   int rc = 2;
   if (what == "alloc") rc = alloc_test(ctx);
+  if (what == "cut") rc = cut_test(ctx);
   if (rc == 0) std::printf("worklist driver ok\n");
   return rc;
 }

@@ -37,3 +37,9 @@ def test_failed_rebuild_leaves_no_list(driver):
     whose calls are refused, not one that runs chunks of one list on the pair
     records of another (or a captured graph on freed ones)."""
     run(driver, "alloc")
+
+
+def test_chunks_of_divided_kets(driver):
+    """The chunks of every run, by class, chain and cap, against their definition
+    evaluated entry by entry."""
+    assert "divided runs" in run(driver, "cut")
