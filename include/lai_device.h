@@ -269,7 +269,9 @@ int lai_dev_jk_graph_launch(lai_basis* b, void* stream);
  * quartet, register tables), LAI_STRATEGY_WAVEFRONT (a wavefront per quartet)
  * or LAI_STRATEGY_BLOCK (a workgroup per quartet, LDS tables) -- the quartets
  * per chunk (a chunk is one bra pair with a run of its kets, taken by one
- * workgroup; 0 = the strategy's default rule) and the grid cap in workgroups
+ * workgroup; 0 = the strategy's default rule; for LAI_STRATEGY_THREAD the
+ * lanes of a chunk: where a class has so few quartets that their kets'
+ * primitive pairs are divided over lanes, each part counts) and the grid cap in workgroups
  * per CU (0 = the strategy's default).  Mirrors
  * OptimalDispatchTable / TwoElectronEntry::gpu_strategy
  * (include/libaccint/kernels/optimal_dispatch_table.hpp:29-33,64-67,83-149),
@@ -286,8 +288,12 @@ typedef struct lai_class_tune {
   double ms_default; /* lai_dev_autotune: milliseconds per launch of the default, else 0 */
 } lai_class_tune;
 
-/* The strategy compiled as a class's default and its alternative (-1: none). */
+/* The strategy compiled as a class's default and its first alternative (-1:
+ * none). */
 int lai_dev_class_strategies(int cls, int* strategy, int* alternative);
+/* Every strategy compiled for a class, which are those that lai_dev_set_tuning
+ * takes: bit LAI_STRATEGY_x of mask.  (Five f classes have all three.) */
+int lai_dev_class_strategy_mask(int cls, int* mask);
 /* Times candidate launches of every class of the current worklist on d_D --
  * each compiled strategy with several chunk caps, then grid caps for the best
  * -- reps launches each after one warm-up, and keeps per class the fastest

@@ -1837,6 +1837,16 @@ extern "C" int lai_dev_class_strategies(int cls, int* strategy, int* alternative
   return LAI_OK;
 }
 
+extern "C" int lai_dev_class_strategy_mask(int cls, int* mask) {
+  if (cls < 0 || cls >= kNumClasses || !mask)
+    return fail(LAI_ERR_INVALID_ARGUMENT, "lai_dev_class_strategy_mask: invalid arguments");
+  const ClassInfo& info = launchers().info[cls];
+  *mask = 0;
+  for (int s : {info.shape, info.alt, info.alt2})
+    if (s != kShapeNone) *mask |= 1 << s;
+  return LAI_OK;
+}
+
 extern "C" int lai_dev_get_tuning(const lai_basis* b, lai_class_tune* table, int cap, int* n_out) {
   if (!b || cap < 0 || (cap > 0 && !table)) return fail(LAI_ERR_INVALID_ARGUMENT, "lai_dev_get_tuning: invalid arguments");
   const int n = std::min(cap, kNumClasses);

@@ -75,6 +75,7 @@ _SIGNATURES = {
     "lai_dev_jk_graph_launch": ([_vp, _vp], ctypes.c_int),
     "lai_dev_set_mixed_prim_cut": ([_vp, ctypes.c_double], ctypes.c_int),
     "lai_dev_class_strategies": ([ctypes.c_int, _ip, _ip], ctypes.c_int),
+    "lai_dev_class_strategy_mask": ([ctypes.c_int, _ip], ctypes.c_int),
     "lai_dev_autotune": ([_vp, _vp, ctypes.c_int, ctypes.c_int, _tp, ctypes.c_int, _ip, _vp], ctypes.c_int),
     "lai_dev_get_tuning": ([_vp, _tp, ctypes.c_int, _ip], ctypes.c_int),
     "lai_dev_set_tuning": ([_vp, _tp, ctypes.c_int], ctypes.c_int),

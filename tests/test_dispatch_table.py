@@ -125,3 +125,23 @@ def test_class_index_helpers_agree_with_decode():
     assert lai.quartet_class_index([4, 0, 0, 0]) == -1  # beyond f
     with pytest.raises(ValueError):
         lai.quartet_class_am(55)
+
+
+def strategy_mask(c):
+    m = ctypes.c_int()
+    assert _cabi.lib().lai_dev_class_strategy_mask(c, ctypes.byref(m)) == 0
+    return m.value
+
+
+def test_strategy_mask_names_every_compiled_strategy():
+    """The mask holds the default and the alternative of every class, and the
+    third strategy of the five f classes that run in slices ((fp|pp), (fs|dp),
+    (fp|ds), (fd|ps), (fp|fs))."""
+    three = {(3, 1, 1, 1), (3, 0, 2, 1), (3, 1, 2, 0), (3, 2, 1, 0), (3, 1, 3, 0)}
+    for c in range(55):
+        s, a = strategies(c)
+        two = (1 << s) | (1 << a if a >= 0 else 0)
+        assert strategy_mask(c) == (7 if class_am(c) in three else two), class_am(c)
+    m = ctypes.c_int()
+    assert _cabi.lib().lai_dev_class_strategy_mask(55, ctypes.byref(m)) == -1
+    assert _cabi.lib().lai_dev_class_strategy_mask(0, None) == -1

@@ -215,3 +215,29 @@ def test_persistent_launch_equals_per_class_launches():
         be.launch_jk_graph(s.cuda_stream)
         s.synchronize()
         assert rel(tJ.cpu().numpy(), Jb0) < 1e-12 and rel(tK.cpu().numpy(), Kb0) < 1e-12, rep
+
+
+@pytest.mark.parametrize("strategy", [0, 1, 2])
+def test_each_strategy_of_the_mask_matches_default(strategy):
+    """Every class that has the strategy on it, the third one of a class among
+    them; a class without it refuses it."""
+    print("dispatch mask", strategy, flush=True)
+    b = lai.basis_set("cc-pvtz", systems.water_cluster(2, 8.0, seed=5))
+    n = b.n_basis_functions()
+    D = systems.density(n, 10, 17, 1.0 / np.sqrt(n))
+    e = lai.Engine(b)
+    opts = lai.JKOptions(schwarz_threshold=1e-12)
+    J0, K0 = e.build_jk(D, opts)
+    S = lai.GpuExecutionStrategy
+    ents, m = [], ctypes.c_int()
+    for c in range(55):
+        _cabi.check(_cabi.lib().lai_dev_class_strategy_mask(c, ctypes.byref(m)))
+        if m.value >> strategy & 1:
+            ents.append(lai.DispatchEntry(c, S(strategy), 0, 0))
+        else:
+            with pytest.raises(Exception):
+                e.set_dispatch_table(lai.DispatchTable([lai.DispatchEntry(c, S(strategy), 0, 0)]))
+    assert len(ents) >= 20
+    e.set_dispatch_table(lai.DispatchTable(ents))
+    J1, K1 = e.build_jk(D, opts)
+    assert rel(J1, J0) < 1e-12 and rel(K1, K0) < 1e-12
