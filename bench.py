@@ -568,8 +568,9 @@ def main():
                     "flops_raised_tables": F1, "tflops_raised_tables": F1 / gs / 1e12,
                     "frac_raised_tables": F1 / gs / 1e12 / FP64_PEAK_TFLOPS, "peak": FP64_PEAK_TFLOPS,
                     "units": "executed primitive pairs; derivative classes: per centre (3 of 4) F_prim of the "
-                             "class with that l raised and with it lowered, + 9 N_cart per root; raised tables: "
-                             "30 + n_r (50 + 3 F_dir(La+1, Lb+1, Lc+1, Ld) + 12 N_cart)"}}
+                             "class with that l raised and with it lowered, + 9 N_cart per root; raised tables (one "
+                             "bra and one ket centre raised, as the kernels build them; closed forms for (ss|ss) and "
+                             "(ps|ss)): 30 + n_r (50 + 3 F_dir(La+1, Lb, Lc+1, Ld) + 12 N_cart)"}}
         log("gradient (32-water def2-SVP): %.3f s, %.2f TFLOP/s (derivative classes) / %.2f (raised tables)" %
             (gs, F0 / gs / 1e12, F1 / gs / 1e12))
 
@@ -613,9 +614,11 @@ def main():
         Jx, _ = engine.build_jk(D, opts)  # FP64 four-centre J
         ej_df, ej = 0.5 * float(np.sum(D * Jd)), 0.5 * float(np.sum(D * Jx))
         # the Coulomb pass reads the pairs b >= a of B; the exchange runs over the
-        # r columns of the factor of D (D is of rank n_occ), found on the device
+        # columns of the factor of D that the device found, or over all of D
         b_bytes = 0.5 * n * (n + 1) * naux * 8.0
-        rank = int(np.linalg.matrix_rank(D))
+        factored, rank = ctypes.c_int(), ctypes.c_int()
+        _cabi.check(L.lai_dev_df_factor_info(hdf, ctypes.byref(factored), ctypes.byref(rank)))
+        rank = rank.value if factored.value == 1 else n
         gemm_flops = 2.0 * n * naux * n * rank
         # share of the exchange product's 64 x 80 tiles of K computed with a
         # symmetric D (tiles entirely below the diagonal are skipped)
@@ -627,9 +630,9 @@ def main():
                         % naux,
             "init_seconds": init_s, "jk_ms": df_ms,
             # one after another on one stream; X = B L includes the factorisation D = L L^T
-            "kernels_ms": {"gamma_pass": km[0], "coulomb_pass": km[1], "factor_and_gemm_X_eq_BL": km[2],
+            "kernels_ms": {"gamma_from_X": km[0], "coulomb_pass": km[1], "factor_and_gemm_X_eq_BL": km[2],
                            "gemm_K_eq_XXt_slices": km[3], "slice_sum": km[4]},
-            "density_symmetric": True, "density_rank": rank,
+            "density_symmetric": True, "density_factored": factored.value == 1, "density_rank": rank,
             "roofline": {"gemm_X_tflops": gemm_flops / km[2] / 1e9,
                          "gemm_K_tflops_algorithmic": gemm_flops / km[3] / 1e9,
                          "gemm_K_tflops_executed": k_share * gemm_flops / km[3] / 1e9,

@@ -227,10 +227,11 @@ int lai_dev_worklist_class_flops(const lai_basis* b, double* flops_fp64, double*
  * executed primitive pairs, the same selection as lai_dev_jk_grad).  model0:
  * per primitive quartet the derivative classes of three centres (each
  * centre's l raised and, when l > 0, lowered by one), F_prim each, plus
- * 9 N_cart contraction flops per root; model1: one table per (root, axis)
- * with the three centres raised together, 30 + n_r (50 + 3 F_dir(La+1, Lb+1,
- * Lc+1, Ld) + 12 N_cart).  Measurement aid; no reference counterpart (the
- * reference has no derivative integrals). */
+ * 9 N_cart contraction flops per root; model1: what lai_dev_jk_grad does, one
+ * table per (root, axis) with a bra and a ket centre raised, 30 + n_r (50 +
+ * 3 F_dir(La+1, Lb, Lc+1, Ld) + 12 N_cart) in the class's order, and 104 and
+ * 168 for the closed forms of (ss|ss) and (ps|ss).  Measurement aid; no
+ * reference counterpart (the reference has no derivative integrals). */
 int lai_dev_worklist_grad_flops(const lai_basis* b, double* model0, double* model1);
 
 /* ---- J/K build ---------------------------------------------------------------

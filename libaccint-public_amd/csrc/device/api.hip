@@ -144,14 +144,23 @@ double fprim(int La, int Lb, int Lc, int Ld) {
 // the derivatives on three centres (the fourth by translational invariance):
 // model 0 evaluates, per centre, the derivative classes with that centre's l
 // raised and (l > 0) lowered by one, F_prim each, plus 9 N_cart contraction
-// flops per root; model 1 builds one table per (root, axis) with the three
-// centres raised together (what the adjoint kernels do):
-// 30 + n_r (50 + 3 F_dir(La+1, Lb+1, Lc+1, Ld) + 12 N_cart), n_r of the raised
-// total angular momentum.
+// flops per root; model 1 is what the adjoint kernels do: one table per (root,
+// axis) with the first bra and the first ket centre of the class raised,
+// 30 + n_r (50 + 3 F_dir(La+1, Lb, Lc+1, Ld) + 12 N_cart), n_r of the raised
+// total angular momentum, and the operations of the closed forms for (ss|ss)
+// and (ps|ss), which build no tables.
 double fgrad(int model, int La, int Lb, int Lc, int Ld) {
   const double ncart4 = double(ncart(La) * ncart(Lb) * ncart(Lc) * ncart(Ld));
   const int nrg = (La + Lb + Lc + Ld + 1) / 2 + 1;
-  if (model == 1) return 30.0 + nrg * (50.0 + 3.0 * fdir(La + 1, Lb + 1, Lc + 1, Ld) + 12.0 * ncart4);
+  if (model == 1) {
+    if (La + Lb + Lc + Ld == 0) return 30.0 + 26.0 + 48.0;  // F_0 and F_1, three derivatives
+    if (La + Lb + Lc + Ld == 1) return 30.0 + 46.0 + 92.0;  // F_0 to F_2, likewise
+    // in the order of the class: larger l first in a pair, larger pair first
+    if (La < Lb) std::swap(La, Lb);
+    if (Lc < Ld) std::swap(Lc, Ld);
+    if (pair_class(La, Lb) < pair_class(Lc, Ld)) std::swap(La, Lc), std::swap(Lb, Ld);
+    return 30.0 + nrg * (50.0 + 3.0 * fdir(La + 1, Lb, Lc + 1, Ld) + 12.0 * ncart4);
+  }
   double f = nrg * 9.0 * ncart4;
   const int l[4] = {La, Lb, Lc, Ld};
   for (int x = 0; x < 3; ++x)

@@ -5,6 +5,7 @@
 //   worklist_driver alloc  every allocation of a rebuild and of a tuning fails
 //                          in turn; nothing may run on parts of two lists
 //   worklist_driver cut    the chunks of divided kets against their definition
+//   worklist_driver flops  the gradient's work model on classes counted by hand
 #include "../../libaccint-public_amd/csrc/device/api.hip"
 
 #include <cstdio>
@@ -324,6 +325,25 @@ static int cut_test(lai_ctx* ctx) {
   return g_bad || several == 0;
 }
 
+// (dp|ps): three roots; tables of x^3 on d, p, p^2 on the ket: 10 recursion
+// operations along the bra, 13 + 23 along the ket, 24 of transfer to b, so 70;
+// 54 components: 30 + 3 (50 + 3 70 + 12 54).  In every order of the quartet.
+static int flops_test() {
+  const int q[3][4] = {{2, 1, 1, 0}, {0, 0, 0, 0}, {1, 0, 0, 0}};
+  const double want[3] = {2754.0, 104.0, 168.0};
+  for (int t = 0; t < 3; ++t)
+    for (int o = 0; o < 8; ++o) {
+      int l[4] = {q[t][0], q[t][1], q[t][2], q[t][3]};
+      if (o & 1) std::swap(l[0], l[1]);
+      if (o & 2) std::swap(l[2], l[3]);
+      if (o & 4) std::swap(l[0], l[2]), std::swap(l[1], l[3]);
+      const double got = fgrad(1, l[0], l[1], l[2], l[3]);
+      if (got != want[t])
+        std::printf("(%d %d|%d %d): %g instead of %g\n", l[0], l[1], l[2], l[3], got, want[t]), g_bad = true;
+    }
+  return g_bad;
+}
+
 int main(int argc, char** argv) {
   lai_ctx* ctx = nullptr;
   if (lai_dev_init(0, &ctx) != LAI_OK) return std::printf("init: %s\n", lai_dev_last_error()), 2;
@@ -331,6 +351,7 @@ int main(int argc, char** argv) {
   int rc = 2;
   if (what == "alloc") rc = alloc_test(ctx);
   if (what == "cut") rc = cut_test(ctx);
+  if (what == "flops") rc = flops_test();
   if (rc == 0) std::printf("worklist driver ok\n");
   return rc;
 }

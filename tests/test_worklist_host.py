@@ -43,3 +43,10 @@ def test_chunks_of_divided_kets(driver):
     """The chunks of every run, by class, chain and cap, against their definition
     evaluated entry by entry."""
     assert "divided runs" in run(driver, "cut")
+
+
+def test_gradient_work_model(driver):
+    """The work that the model gives the gradient kernels: what they build (one
+    bra and one ket centre raised, closed forms for (ss|ss) and (ps|ss)),
+    whatever the order of the quartet's shells."""
+    run(driver, "flops")
