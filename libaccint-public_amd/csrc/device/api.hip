@@ -253,8 +253,8 @@ struct ClassList {
 };
 
 // Launch choice of one class (autotuner or caller table): alt selects the
-// class's alternative kernel shape, chunk caps the quartets per chunk (0: the
-// shape's default rule), bpc the workgroups per CU (0: the shape's default).
+// class's alternative kernel shape (1, or 2 for its second one), chunk caps the
+// entries per chunk (cut_runs; 0: the shape's default rule), bpc the workgroups per CU (0: the shape's default).
 struct ClassTune {
   int alt = 0;
   int chunk = 0;
@@ -1026,7 +1026,7 @@ extern "C" uint64_t lai_quartet_mix64(int i, int j, int k, int l) {
 
 namespace {
 // Chunk cap of the default rule for a class run in shape `shape` with n
-// quartets: lane-per-quartet kernels take up to 2048 quartets (a workgroup of
+// entries: lane-per-quartet kernels take up to 2048 entries (a workgroup of
 // nt to 512 lanes; the launch replicates the nt-lane unit), wavefront-per-
 // quartet kernels up to 64, workgroup-per-quartet kernels up to 32; small
 // classes get shorter chunks so that a launch still has a few workgroups per

@@ -1311,7 +1311,7 @@ __device__ __forceinline__ void jk_chunk_merged(const EriArgs& g, const JkChunk&
             jpart[(C * NCD + c * nd + d) * kJPad + lane] = fJ * t;
           }
         if constexpr (C == 0) jpos[lane] = kp;
-            // Kt[ac] += fK sum_bd g D[bd]
+        // Kt[ac] += fK sum_bd g D[bd]
 #pragma unroll
         for (int a = 0; a < NA; ++a)
 #pragma unroll

@@ -20,8 +20,10 @@
 // B = AB - A, and by translational invariance D = -AB - C.  (Raising b as well
 // instead of the AB derivative makes the tables (Lb+2)/(Lb+1) larger: 36
 // instead of 22 entries an axis for (dp|ps), 8 instead of 3 for (ss|ss).)
-// Shape: one workgroup per shell quartet, (root, axis) tables and the weights
-// W in LDS, each lane a strided subset of the Cartesian components.
+// Shapes (GradPolicy): a lane per shell quartet and bra slice with tables and
+// weights W in registers, for all classes but (dd|dp) and (dd|dd), which take a
+// workgroup per quartet, (root, axis) tables and W in LDS, each lane a strided
+// subset of the Cartesian components.
 #pragma once
 
 #include "eri_kernels.hpp"
@@ -49,9 +51,6 @@ struct GradArgs {
   int chain, kmax;  // division of the kets' primitives over lanes (ket_split)
 };
 
-// The register shape's tables hold no entry raised in both a and c (never
-// used, so the compiler drops them).
-//
 // Primitive quartets per step of the LDS-shape gradient kernel: 3 n_r lanes
 // build the (root, axis) tables of one primitive quartet, as many primitive
 // quartets at once as the lanes and 16 KB of tables allow (more would cost
@@ -295,7 +294,8 @@ struct GradPolicy {
 
 // --------------------------------------------------------------------------
 // Register shape: one lane per shell quartet (bra components A0 .. A1 - 1) of a
-// bra-anchored chunk, the 2D tables raised by one on A or C held in registers.
+// bra-anchored chunk, the 2D tables raised by one on A or C held in registers
+// (entries raised on both are never used, so the compiler drops them).
 // f: the A, AB and C derivatives.  The forces on the bra atoms are summed over
 // the lane's quartets and reduced over the wavefront; those on the ket atoms go
 // to the workgroup's LDS force array (or to HBM atomics without one).

@@ -16,7 +16,7 @@ enum : int { kShapeNone = -1, kShapeRegs = 0, kShapeWaves = 1, kShapeLds = 2 };
 // Launch parameters of one class: which of its compiled shapes runs and the
 // grid cap in workgroups per CU (0: the shape's default).
 struct LaunchTune {
-  int alt = 0;            // 0: the class's primary shape, 1: its alternative
+  int alt = 0;            // 0: the class's primary shape, 1: its alternative, 2: its second one
   int blocks_per_cu = 0;  // grid = min(chunks, n_cu * blocks_per_cu)
   int n_cu = 256;
 };

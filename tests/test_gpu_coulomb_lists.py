@@ -1,11 +1,12 @@
 """The Coulomb accumulators in list order (blocks of the shell pairs in the
 order of the worklist, added whole cache lines at a time) against the oracle,
 at the sizes where the list arithmetic can go wrong: one pair; ket runs just
-below, at and above the 2048 quartets that are sorted at a time; (ss| kets,
-which go through the sort's slots, beside kets of 3 to 10 Coulomb elements,
-which go through the wavefront tiles; runs shortened by the density screen;
-molecules of different sizes in one list.  Bar: 1e-10 relative, the J/K bar of
-test_gpu_parity.py (FP64 sums in another order)."""
+below, at and above the 2048 quartets that are sorted at a time (in one chunk
+where the chunk cap is raised, else in chunks of equal length); (ss| kets,
+whose elements are summed by run position, beside kets of 3 to 10 Coulomb
+elements, which go through the wavefront tiles; runs shortened by the density
+screen; molecules of different sizes in one list.  Bar: 1e-10 relative, the J/K
+bar of test_gpu_parity.py (FP64 sums in another order)."""
 import numpy as np
 import pytest
 
@@ -107,3 +108,22 @@ def test_divided_kets_match_oracle(n_atoms, n_prim):
         return 0.5 * np.sum(D * J) - 0.25 * np.sum(D * K)
     fd = (8.0 * (energy(1e-4) - energy(-1e-4)) - (energy(2e-4) - energy(-2e-4))) / 12e-4
     assert abs(g[0, 0] - fd) < 1e-6 * max(1.0, abs(energy(0.0)))
+
+
+@pytest.mark.parametrize("name", ["h63", "h64", "h91"])
+@pytest.mark.parametrize("chunk", [2047, 2048, 4096, 8192])
+def test_chunks_beyond_one_sort(name, chunk):
+    """(ss|ss) chunks of up to 2016, 2080 and 4186 kets (every length below them
+    as the bra goes through its list, 2048 among them): one pass of the sort,
+    two, and three, the Coulomb elements added and cleared between them."""
+    print("coulomb lists, chunk cap", name, chunk, flush=True)
+    basis_name, atoms = case(name)
+    basis = lai.basis_set(basis_name, atoms)
+    n = basis.n_basis_functions()
+    D = systems.density(n, max(1, n // 4), 7, 1.0 / np.sqrt(n))
+    e = lai.Engine(basis)
+    e.set_dispatch_table(lai.DispatchTable([lai.DispatchEntry(0, lai.GpuExecutionStrategy(0), chunk, 0)]))
+    Jo, Ko = oracle.Oracle(oracle.RawBasis(basis_name, atoms)).jk_canonical(D)
+    for weighted in (False, True):
+        J, K = e.build_jk(D, lai.JKOptions(schwarz_threshold=0.0 if not weighted else 1e-12, density_weighted=weighted))
+        assert rel(J, Jo) < TOL and rel(K, Ko) < TOL

@@ -1,8 +1,11 @@
 """The f classes that run a lane per quartet with the bra in four or five slices
-((fp|pp), (fs|dp), (fp|ds), (fd|ps), (fp|fs)) against the oracle, in each of
-their three strategies (a saved table may name any), with the default chunk cap,
-one quartet per chunk, and caps just off a wavefront and a sort run.  Bar: 1e-10
-relative, the J/K bar of test_gpu_parity.py."""
+((fp|pp), (fs|dp), (fp|ds), (fd|ps), (fp|fs)) in each of their three strategies
+(a saved table may name any): one water in cc-pVTZ against the oracle, with the
+default chunk cap and one quartet per chunk (10 to 70 kets a bra), and three
+waters (90 to 630 kets a bra) against the workgroup kernel, with caps just off a
+wavefront and just off the lanes of a group of slices.  Bar: 1e-10 relative, the
+J/K bar of test_gpu_parity.py, against the oracle; 1e-12 between strategies (FP64
+sums in another order)."""
 import ctypes
 
 import numpy as np
@@ -49,3 +52,22 @@ def test_strategies_match_oracle(strategy, chunk):
         J, K = e.build_jk(D, lai.JKOptions(schwarz_threshold=1e-12, mixed_precision=mixed, fp32_threshold=1e-12))
         assert np.max(np.abs(J - Jo)) < 1e-10 * np.max(np.abs(Jo))
         assert np.max(np.abs(K - Ko)) < 1e-10 * np.max(np.abs(Ko))
+
+
+@pytest.mark.parametrize("chunk", [0, 63, 65, 255, 257, 321])
+def test_strategies_match_on_long_runs(chunk):
+    print("f slices, long runs", chunk, flush=True)
+    basis = lai.basis_set("cc-pvtz", systems.water_cluster(3, 10.0, seed=5))
+    n = basis.n_basis_functions()
+    D = systems.density(n, 15, 11, 1.0 / np.sqrt(n))
+    e = lai.Engine(basis)
+    S = lai.GpuExecutionStrategy
+    opts = lai.JKOptions(schwarz_threshold=1e-12)
+    got = []
+    for strategy in (2, 0, 1):
+        cap = 0 if strategy == 2 else chunk
+        e.set_dispatch_table(lai.DispatchTable([lai.DispatchEntry(c, S(strategy), cap, 0) for c in CLASSES]))
+        got.append(e.build_jk(D, opts))
+    for J, K in got[1:]:
+        assert np.max(np.abs(J - got[0][0])) < 1e-12 * np.max(np.abs(got[0][0]))
+        assert np.max(np.abs(K - got[0][1])) < 1e-12 * np.max(np.abs(got[0][1]))
